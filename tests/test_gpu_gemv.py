@@ -170,3 +170,64 @@ def test_native_16bit_gemv(capi, a_type, trans, shape):
     for tier, rtol in [(C.TIER_DEFAULT, 3e-6), (C.TIER_FAST, 1e-12), (C.TIER_EXACT, 1e-12)]:
         got = H.gemv(a_type, tier, trans, 1.5, m, n, Ad, None, lda, x, -0.5, y0, C.F64, C.F64)
         check_close(got, ref, scale, rtol)
+
+
+# The edges of the kernels' ranges: fewer rows than a vector, the last vector
+# of a column moved back over its neighbour's rows, columns on odd addresses,
+# one column, fewer columns than column groups, both sides of the whole-column
+# limit (128 KB a column) and of the column-split rules.
+EDGE = [(1, 1, 1), (7, 3, 7), (8, 1, 8), (9, 40, 9), (129, 66, 131), (4097, 9, 4099), (65535, 5, 65535),
+        (65536, 3, 65536), (65537, 67, 65537), (32769, 33, 32777), (300, 300, 300)]
+
+
+@pytest.mark.parametrize("a_type", [C.F32, C.F64, C.F16, C.BF16, C.FP32_16, C.FP32_BF16])
+@pytest.mark.parametrize("shape", EDGE)
+def test_gemv_edges(capi, orc, a_type, shape):
+    """Every tier and direction against FP64 products of the stored values.
+    The matrix holds every word class of FP32_16 (subnormal and overflowing
+    half words, saturated words), one Inf in the last row (rows next to it
+    are read twice) and padding rows of NaN.  Bounds as in the tests above:
+    n eps |A||x| is 65537 * 6e-8 = 4e-3 at worst for FP32 sums in one chain
+    and 300 * 6e-8 = 2e-5 in the chains used here; FP64 7e-12 and 3e-14."""
+    m, n, lda = shape
+    rng = np.random.default_rng(m * 7 + n)
+    A = data(m, n, m + 3 * n, wide=True)
+    k = rng.integers(0, m * n, 3)
+    A.flat[k] = np.array([3e4, -2e-9, 1e-6], np.float32)  # large, saturated, subnormal half
+    inf_at = (m - 1, n - 1)
+    if a_type in FORMATS:
+        variant, decs = FORMATS[a_type]
+        A[inf_at] = np.inf  # FP32_16: a saturated overflow word
+        ehh, err_ = orc.pack(variant, A)
+        sh, sr = np.full((lda, n), 0x7FFF, np.uint16, order="F"), np.full((lda, n), 0x7FFF, np.uint16, order="F")
+        sh[:m], sr[:m] = ehh, err_
+        a, wr = H.dev(sh), H.dev(sr)
+        value = {t: orc.unpack(decs[t], ehh, err_).astype(np.float64) for t in decs}
+    else:
+        dt = {C.F32: np.float32, C.F64: np.float64, C.F16: np.float16}.get(a_type)
+        A[inf_at] = np.inf
+        if a_type == C.BF16:
+            st = bf16_bits_rne(A)
+            v = (st.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+            pad = np.uint16(0x7FFF)
+        else:
+            st = A.astype(dt)
+            v, pad = st.astype(np.float64), np.nan
+        store = np.full((lda, n), pad, st.dtype, order="F")
+        store[:m] = st
+        a, wr = H.dev(store), None
+        value = {t: v for t in (C.TIER_DEFAULT, C.TIER_FAST, C.TIER_EXACT)}
+    for trans in (0, 1):
+        rows, cols = (n, m) if trans else (m, n)
+        x = rng.standard_normal(cols)
+        y0 = rng.standard_normal(rows)
+        for tier, rtol in ((C.TIER_DEFAULT, 3e-5), (C.TIER_FAST, 1e-12), (C.TIER_EXACT, 1e-12)):
+            print("edge", a_type, shape, trans, tier, flush=True)
+            op = value[tier].T if trans else value[tier]
+            with np.errstate(invalid="ignore"):
+                ref = 1.5 * (op @ x) - 0.5 * y0
+                scale = 1.5 * (np.abs(op) @ np.abs(x)) + 0.5 * np.abs(y0)
+            got = H.gemv(a_type, tier, trans, 1.5, m, n, a, wr, lda, x, -0.5, y0, C.F64, C.F64)
+            fin = np.isfinite(ref)
+            assert np.array_equal(got[~fin], ref[~fin], equal_nan=True)
+            check_close(got[fin], ref[fin], scale[fin], rtol)

@@ -165,6 +165,55 @@ TOMOS_HD uint32_t fp32_16_half_bits(uint32_t h) {
     return sel(ctl, special, h & 0xFFFFu);
 }
 
+#if defined(__HIPCC__)
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// All ones in each 16-bit half whose bit 0 is set in b (b has no other bits).
+__device__ __forceinline__ uint32_t half_masks(uint32_t b) {
+    const u16x2 zero = {0, 0};
+    return __builtin_bit_cast(uint32_t, static_cast<u16x2>(zero - __builtin_bit_cast(u16x2, b)));
+}
+
+// fp32_16_half_bits of two words in one register, on packed 16-bit integer
+// operations: 12 for the pair against about 13 for each word, which left the
+// hi-only GEMV of this format bound by the VALU and not by HBM (GEMV^T
+// 1e6 x 1000: 692 us).  v_pk_lshrrev_b16 takes its shift modulo 16, so the
+// bits above it may stay.
+__device__ __forceinline__ uint32_t fp32_16_half_bits2(uint32_t h) {
+    uint32_t m, sub;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(m) : "v"(h >> 1), "s"(0x01FF01FFu), "v"(0x02000200u));
+    asm("v_pk_lshrrev_b16 %0, %1, %2" : "=v"(sub) : "v"(h >> 10), "v"(m));
+    const uint32_t dir = half_masks((h >> 14) & 0x00010001u);
+    const uint32_t ctl = half_masks(h & 0x00010001u);
+    const uint32_t mag = (dir & 0x7C007C00u) | (~dir & sub);
+    return ((ctl & mag) | (~ctl & h)) | (h & 0x80008000u);
+}
+
+// Bits that are non-zero when one of the two words is saturated (control
+// set, shift 14); fp32_16_decode_exact2 does not decode those.
+__device__ __forceinline__ uint32_t fp32_16_saturated2(uint32_t h) {
+    const uint32_t x = (h & 0x3C013C01u) ^ 0x38013801u;
+    return (x - 0x00010001u) & ~x & 0x80008000u;
+}
+
+// fp32_16_decode_exact of two word pairs that are not saturated, mostly on
+// both halves at once.  t holds field and mant_hi (mant_hi at bit 1), biased
+// by 16 exponent steps so that nothing borrows across the halves: an
+// underflow word's exponent is 112 - field (t - 2 field), an overflow word's
+// 127 + field (t + 15 steps), and undoing the rounding (mant_hi - round_flag)
+// borrows into the exponent by itself.
+__device__ __forceinline__ void fp32_16_decode_exact2(uint32_t h, uint32_t r, float& v0, float& v1) {
+    const uint32_t ctl = h & 0x00010001u;
+    const uint32_t dir = (h >> 14) & 0x00010001u;
+    const uint32_t f = h & half_masks(ctl & ~dir) & 0x7C007C00u;
+    const uint32_t t = (h & 0x7FFE7FFEu) + 0x40004000u - 2u * f + (half_masks(ctl & dir) & 0x3C003C00u) -
+                       2u * (r & 0x00010001u);
+    const uint32_t lo = (r >> 2) & 0x3FFF3FFFu;
+    v0 = u2f((((t & 0xFFFFu) << 13) + (lo & 0xFFFFu)) + (((h << 16) & 0x80000000u) | 0x30000000u));
+    v1 = u2f((((t >> 16) << 13) + (lo >> 16)) + ((h & 0x80000000u) | 0x30000000u));
+}
+#endif
+
 // fp32_16_half_only_fast (fp32_16_pack.hpp:586-595): every control=1 word
 // saturates (+-Inf overflow, +-0 underflow).
 TOMOS_HD uint32_t fp32_16_half_bits_fast(uint32_t h) {

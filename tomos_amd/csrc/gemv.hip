@@ -10,16 +10,17 @@
 //           its block's column range, 8 columns per batch so 8 independent
 //           16-B loads are in flight per lane.  x[j] is wave-uniform and is
 //           read through the scalar cache.  When m is too small to fill the
-//           chip, columns are split across blocks and a second pass sums the
-//           per-split partials in a fixed order.
+//           chip, the waves of a block split the columns and add their sums
+//           through LDS in a fixed order.
 // z = A^T y (TRANSPOSE): a block owns a chunk of rows and a group of CB
 //           columns; each lane keeps CB column accumulators in VGPRs and
 //           walks the chunk in 16-B row vectors (loads coalesced along the
 //           column), the wave reduces the CB accumulators with a transpose
 //           butterfly (CB-1 shuffles per lane instead of 6*CB), the four
 //           waves combine through LDS, and the per-chunk partials are summed
-//           in a fixed order by a second pass.  No atomics anywhere: results
-//           are bit-reproducible run to run.
+//           in a fixed order by a second pass.  Short columns are owned whole
+//           by a block, without partials.  No atomics anywhere: results are
+//           bit-reproducible run to run.
 #include <algorithm>
 
 #include "codec.hpp"
@@ -54,6 +55,20 @@ struct Raw {
     uint32_t r[4];
 };
 
+// 16-byte vectors are read at element alignment: gfx950 global loads take
+// any, so an lda that is no multiple of the vector (an unpadded odd m) costs
+// a cache line more per 1 KB wave load, where element-wise loads cost eight
+// times the load instructions (131071 x 501 FP32_16 EXACT, odd lda, with the
+// pair decode: N 76 -> 51 us, T 118 -> 74 us).
+template <bool NTL>
+__device__ __forceinline__ uint4 load_vec16(const void* p) {
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4), aligned(2)));
+    u32x4 v;
+    if constexpr (NTL) v = __builtin_nontemporal_load(static_cast<const u32x4*>(p));
+    else v = *static_cast<const u32x4*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 template <int FMT, int DEC, int VEC, bool NTL>
 __device__ __forceinline__ void load_raw(const void* __restrict__ a,
                                          const uint16_t* __restrict__ wr, int64_t idx,
@@ -61,10 +76,10 @@ __device__ __forceinline__ void load_raw(const void* __restrict__ a,
     if constexpr (is16<FMT>()) {
         const uint16_t* p = static_cast<const uint16_t*>(a) + idx;
         if constexpr (VEC == 8) {
-            const uint4 t = load_a16<NTL>(p);
+            const uint4 t = load_vec16<NTL>(p);
             R.h[0] = t.x; R.h[1] = t.y; R.h[2] = t.z; R.h[3] = t.w;
             if constexpr (DEC == DEC_EXACT) {
-                const uint4 q = load_a16<NTL>(wr + idx);
+                const uint4 q = load_vec16<NTL>(wr + idx);
                 R.r[0] = q.x; R.r[1] = q.y; R.r[2] = q.z; R.r[3] = q.w;
             }
         } else {
@@ -74,7 +89,7 @@ __device__ __forceinline__ void load_raw(const void* __restrict__ a,
     } else if constexpr (FMT == FMT_F32) {
         const float* p = static_cast<const float*>(a) + idx;
         if constexpr (VEC == 4) {
-            const uint4 t = load_a16<NTL>(p);
+            const uint4 t = load_vec16<NTL>(p);
             R.h[0] = t.x; R.h[1] = t.y; R.h[2] = t.z; R.h[3] = t.w;
         } else {
             R.h[0] = __float_as_uint(*p);
@@ -82,7 +97,7 @@ __device__ __forceinline__ void load_raw(const void* __restrict__ a,
     } else {
         const double* p = static_cast<const double*>(a) + idx;
         if constexpr (VEC == 2) {
-            const uint4 t = load_a16<NTL>(p);
+            const uint4 t = load_vec16<NTL>(p);
             R.h[0] = t.x; R.h[1] = t.y; R.h[2] = t.z; R.h[3] = t.w;
         } else {
             const uint2 t = *reinterpret_cast<const uint2*>(p);
@@ -108,16 +123,48 @@ __device__ __forceinline__ float decode16(uint32_t h, uint32_t r) {
     }
 }
 
-template <int FMT, int DEC, int VEC, class ACC>
+// Whether an FP32_16 vector holds a saturated word (the exact pair decode
+// leaves those out).
+template <int FMT, int DEC>
+__device__ __forceinline__ bool saturated(const Raw<FMT, DEC, 8>& R) {
+    return (codec::fp32_16_saturated2(R.h[0]) | codec::fp32_16_saturated2(R.h[1]) |
+            codec::fp32_16_saturated2(R.h[2]) | codec::fp32_16_saturated2(R.h[3])) != 0;
+}
+
+// RARE = false: an exact FP32_16 vector without saturated words.
+template <int FMT, int DEC, int VEC, class ACC, bool RARE = true>
 __device__ __forceinline__ void decode(const Raw<FMT, DEC, VEC>& R, ACC (&out)[VEC]) {
     if constexpr (is16<FMT>()) {
         if constexpr (VEC == 8) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
+                if constexpr (FMT == FMT_P16) {
+                    float v0, v1;
+                    if constexpr (DEC == DEC_HI) {
+                        const uint32_t hb = codec::fp32_16_half_bits2(R.h[k]);
+                        v0 = half_bits_to_float(hb & 0xFFFFu);
+                        v1 = half_bits_to_float(hb >> 16);
+                    } else {
+                        codec::fp32_16_decode_exact2(R.h[k], R.r[k], v0, v1);
+                    }
+                    out[2 * k] = static_cast<ACC>(v0);
+                    out[2 * k + 1] = static_cast<ACC>(v1);
+                    continue;
+                }
                 const uint32_t h = R.h[k];
                 const uint32_t r = (DEC == DEC_EXACT) ? R.r[k] : 0u;
                 out[2 * k] = static_cast<ACC>(decode16<FMT, DEC>(h & 0xFFFFu, r & 0xFFFFu));
                 out[2 * k + 1] = static_cast<ACC>(decode16<FMT, DEC>(h >> 16, r >> 16));
+            }
+            if constexpr (FMT == FMT_P16 && DEC == DEC_EXACT && RARE) {
+                if (saturated(R)) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const int b = 16 * (k & 1);
+                        out[k] = static_cast<ACC>(
+                            decode16<FMT, DEC>((R.h[k / 2] >> b) & 0xFFFFu, (R.r[k / 2] >> b) & 0xFFFFu));
+                    }
+                }
             }
         } else {
             out[0] = static_cast<ACC>(decode16<FMT, DEC>(R.h[0], (DEC == DEC_EXACT) ? R.r[0] : 0u));
@@ -138,10 +185,45 @@ __device__ __forceinline__ double read_coef(double host, const double* dev, doub
     return dev ? mul * (*dev) : host;
 }
 
-template <class ACC>
-__device__ __forceinline__ ACC load_x(const void* __restrict__ x, bool x64, int64_t j) {
-    return x64 ? static_cast<ACC>(static_cast<const double*>(x)[j])
-               : static_cast<ACC>(static_cast<const float*>(x)[j]);
+// x[j .. j+U), a wave's U columns; entries at j1 and beyond repeat x[j1-1].
+// One branch on the type for all of them, so that their scalar loads are in
+// flight together.
+template <int U, class ACC>
+__device__ __forceinline__ void load_x_cols(const void* __restrict__ x, bool x64, int64_t j, int64_t j1,
+                                            ACC (&xs)[U]) {
+    if (x64) {
+        double t[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) t[u] = static_cast<const double*>(x)[min(j + u, j1 - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) xs[u] = static_cast<ACC>(t[u]);
+    } else {
+        float t[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) t[u] = static_cast<const float*>(x)[min(j + u, j1 - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) xs[u] = static_cast<ACC>(t[u]);
+    }
+}
+
+// x of a lane's VEC rows starting at i (all in range); the first `lo` are 0.
+template <int VEC, class ACC>
+__device__ __forceinline__ void load_x_rows(const void* __restrict__ x, bool x64, int64_t i, int lo,
+                                            ACC (&xv)[VEC]) {
+    if (x64) {
+        typedef double vd __attribute__((ext_vector_type(VEC), aligned(8)));
+        const vd t = *reinterpret_cast<const vd*>(static_cast<const double*>(x) + i);
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) xv[v] = static_cast<ACC>(t[v]);
+    } else {
+        typedef float vf __attribute__((ext_vector_type(VEC), aligned(4)));
+        const vf t = *reinterpret_cast<const vf*>(static_cast<const float*>(x) + i);
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) xv[v] = static_cast<ACC>(t[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < VEC - 1; ++v)
+        if (v < lo) xv[v] = ACC(0);
 }
 
 // Stores alpha*acc + beta*y (y not read when beta == 0); returns the
@@ -167,65 +249,82 @@ __device__ __forceinline__ double store_y(void* __restrict__ y, bool y64, int64_
 // Block-wide FP64 sum, fixed order; every thread of the block must call it.
 __device__ __forceinline__ void block_sumsq_out(double v, double* out) {
     for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-    __shared__ double part[kThreads / 64];
+    __shared__ double part[16];
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
     __syncthreads();
-    if (threadIdx.x == 0) *out = (part[0] + part[1]) + (part[2] + part[3]);
+    if (threadIdx.x == 0) {
+        double s = part[0];
+        for (unsigned w = 1; w < blockDim.x / 64; ++w) s += part[w];
+        *out = s;
+    }
 }
 
 // ------------------------------------------------------------ NO_TRANSPOSE
+// acc += A[i0 .. i0+VEC, j0 .. j1) x[j0 .. j1): U columns' loads in flight.
 template <int FMT, int DEC, int VEC, class ACC, bool NTL>
-__global__ __launch_bounds__(kThreads) void gemv_n_kernel(
-    int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
-    int64_t lda, const void* __restrict__ x, bool x64, void* __restrict__ y, bool y64, Coef coef,
-    int64_t col_chunk, ACC* __restrict__ partial) {
-    if (coef.skip && *coef.skip) return;
-    const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * VEC;
-    const int64_t j0 = static_cast<int64_t>(blockIdx.y) * col_chunk;
-    const int64_t j1 = min(n, j0 + col_chunk);
-    ACC acc[VEC];
-#pragma unroll
-    for (int v = 0; v < VEC; ++v) acc[v] = ACC(0);
-    if (i0 < m) {
-        constexpr int U = 8;
-        int64_t j = j0;
-        for (; j + U <= j1; j += U) {
-            Raw<FMT, DEC, VEC> R[U];
+__device__ __forceinline__ void sweep_columns(const void* __restrict__ a, const uint16_t* __restrict__ wr,
+                                              int64_t lda, const void* __restrict__ x, bool x64, int64_t i0,
+                                              int64_t j0, int64_t j1, ACC (&acc)[VEC]) {
+    constexpr int U = DEC == DEC_EXACT ? 4 : 8;  // EXACT: two planes, and 8 would take 256 VGPRs
+    for (int64_t j = j0; j < j1; j += U) {
+        Raw<FMT, DEC, VEC> R[U];
+        ACC xs[U];
+        load_x_cols<U, ACC>(x, x64, j, j1, xs);
+        if (j + U <= j1) {
 #pragma unroll
             for (int u = 0; u < U; ++u) load_raw<FMT, DEC, VEC, NTL>(a, wr, i0 + (j + u) * lda, R[u]);
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 ACC av[VEC];
                 decode<FMT, DEC, VEC, ACC>(R[u], av);
-                const ACC xv = load_x<ACC>(x, x64, j + u);
 #pragma unroll
-                for (int v = 0; v < VEC; ++v) acc[v] = fma(av[v], xv, acc[v]);
+                for (int v = 0; v < VEC; ++v) acc[v] = fma(av[v], xs[u], acc[v]);
+            }
+        } else {  // the last columns, their loads in flight together as well
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (j + u < j1) load_raw<FMT, DEC, VEC, NTL>(a, wr, i0 + (j + u) * lda, R[u]);
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (j + u < j1) {
+                    ACC av[VEC];
+                    decode<FMT, DEC, VEC, ACC>(R[u], av);
+#pragma unroll
+                    for (int v = 0; v < VEC; ++v) acc[v] = fma(av[v], xs[u], acc[v]);
+                }
             }
         }
-        for (; j < j1; ++j) {
-            Raw<FMT, DEC, VEC> R;
-            load_raw<FMT, DEC, VEC, NTL>(a, wr, i0 + j * lda, R);
-            ACC av[VEC];
-            decode<FMT, DEC, VEC, ACC>(R, av);
-            const ACC xv = load_x<ACC>(x, x64, j);
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) acc[v] = fma(av[v], xv, acc[v]);
-        }
     }
-    if (partial) {
-        if (i0 >= m) return;
+}
+
+// First row of a lane's vector: i, or m - VEC where the vector would run
+// past the matrix (the lane then reads rows of its neighbour as well and
+// uses only its own).
+template <int VEC>
+__device__ __forceinline__ int64_t first_row(int64_t i, int64_t m) {
+    return min(i, m - VEC);
+}
+
+// A lane owns VEC rows and all columns.  Bound by HBM when the rows alone
+// fill the chip (plan_n).
+template <int FMT, int DEC, int VEC, class ACC, bool NTL>
+__global__ __launch_bounds__(kThreads) void gemv_n_kernel(
+    int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
+    int64_t lda, const void* __restrict__ x, bool x64, void* __restrict__ y, bool y64, Coef coef) {
+    if (coef.skip && *coef.skip) return;
+    const int64_t ir = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * VEC;
+    ACC acc[VEC];
 #pragma unroll
-        for (int v = 0; v < VEC; ++v)
-            if (i0 + v < m) partial[static_cast<int64_t>(blockIdx.y) * m + i0 + v] = acc[v];
-        return;
-    }
+    for (int v = 0; v < VEC; ++v) acc[v] = ACC(0);
+    const int64_t i0 = first_row<VEC>(ir, m);
+    if (ir < m) sweep_columns<FMT, DEC, VEC, ACC, NTL>(a, wr, lda, x, x64, i0, 0, n, acc);
     const double al = read_coef(coef.alpha, coef.dalpha, coef.alpha_mul);
     const double be = read_coef(coef.beta, coef.dbeta, coef.beta_mul);
     double sq = 0.0;
-    if (i0 < m) {
+    if (ir < m) {
 #pragma unroll
         for (int v = 0; v < VEC; ++v)
-            if (i0 + v < m) {
+            if (i0 + v >= ir) {
                 const double r = store_y(y, y64, i0 + v, al, static_cast<double>(acc[v]), be);
                 sq += r * r;
             }
@@ -233,29 +332,55 @@ __global__ __launch_bounds__(kThreads) void gemv_n_kernel(
     if (coef.sumsq) block_sumsq_out(sq, coef.sumsq + blockIdx.x);
 }
 
-template <class ACC>
-__global__ __launch_bounds__(kThreads) void gemv_n_finish(int64_t m, int splits,
-                                                          const ACC* __restrict__ partial,
-                                                          void* __restrict__ y, bool y64,
-                                                          Coef coef) {
+// The rows alone do not fill the chip: a block takes RL x VEC rows and its
+// column groups (64 / RL in each wave) split the columns; their sums meet in
+// lane shuffles and LDS and are added in group order, in FP64 across waves.
+// No partials in memory (m x splits accumulators written and read back by a
+// second launch): 20000 x 200 bf16 hi 5.2 + 4.1 -> 5.5 us in one launch,
+// 1e6 x 1000 FP32_16 hi 389 + 5 -> 347 us (5.8 TB/s).  RL = 16, 256-byte runs of a column, where even 64-lane
+// rows times 16 waves are few.  VEC * sizeof(ACC) * waves is at most 512
+// bytes per row lane (32 KB of LDS).
+constexpr int kSplitLds = 512;
+template <int FMT, int DEC, int VEC, class ACC, int RL, bool NTL>
+__global__ __launch_bounds__(kSplitLds / VEC / sizeof(ACC) >= 16 ? 1024 : 64 * (kSplitLds / VEC / sizeof(ACC)))
+void gemv_n_split_kernel(int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
+                         int64_t lda, const void* __restrict__ x, bool x64, void* __restrict__ y, bool y64,
+                         Coef coef, int64_t col_chunk) {
     if (coef.skip && *coef.skip) return;
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    constexpr int kStride = RL + 1;  // v-major slots, odd stride: reads of consecutive rows spread over the banks
+    __shared__ ACC red[kSplitLds / sizeof(ACC) * kStride];
+    const int lane = threadIdx.x & 63, rl = lane % RL;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int waves = blockDim.x >> 6;
+    const int64_t b0 = static_cast<int64_t>(blockIdx.x) * RL * VEC;
+    const int64_t ir = b0 + rl * VEC;
+    ACC acc[VEC];
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) acc[v] = ACC(0);
+    const int64_t i0 = first_row<VEC>(ir, m);
+    if (ir < m) {
+        const int64_t j0 = RL == 64 ? wave * col_chunk : (wave * (64 / RL) + lane / RL) * col_chunk;
+        sweep_columns<FMT, DEC, VEC, ACC, NTL>(a, wr, lda, x, x64, i0, j0, min(n, j0 + col_chunk), acc);
+    }
+#pragma unroll
+    for (int o = RL; o < 64; o *= 2)
+#pragma unroll
+        for (int v = 0; v < VEC; ++v) acc[v] += __shfl_xor(acc[v], o);
+    if (ir < m && lane < RL) {
+        const int sh = static_cast<int>(ir - i0);
+#pragma unroll
+        for (int v = 0; v < VEC; ++v)
+            if (v >= sh) red[(wave * VEC + v - sh) * kStride + rl] = acc[v];
+    }
+    __syncthreads();
+    const double al = read_coef(coef.alpha, coef.dalpha, coef.alpha_mul);
+    const double be = read_coef(coef.beta, coef.dbeta, coef.beta_mul);
     double sq = 0.0;
-    if (i < m) {
-        // four chains: the partial sums' loads overlap
-        double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-        int c = 0;
-        for (; c + 3 < splits; c += 4) {
-            s0 += static_cast<double>(partial[static_cast<int64_t>(c) * m + i]);
-            s1 += static_cast<double>(partial[static_cast<int64_t>(c + 1) * m + i]);
-            s2 += static_cast<double>(partial[static_cast<int64_t>(c + 2) * m + i]);
-            s3 += static_cast<double>(partial[static_cast<int64_t>(c + 3) * m + i]);
-        }
-        for (; c < splits; ++c) s0 += static_cast<double>(partial[static_cast<int64_t>(c) * m + i]);
-        const double s = (s0 + s1) + (s2 + s3);
-        const double r = store_y(y, y64, i, read_coef(coef.alpha, coef.dalpha, coef.alpha_mul), s,
-                                 read_coef(coef.beta, coef.dbeta, coef.beta_mul));
-        sq = r * r;
+    for (int r = threadIdx.x; r < RL * VEC && b0 + r < m; r += blockDim.x) {
+        double s = 0.0;
+        for (int w = 0; w < waves; ++w) s += static_cast<double>(red[(w * VEC + r % VEC) * kStride + r / VEC]);
+        const double t = store_y(y, y64, b0 + r, al, s, be);
+        sq += t * t;
     }
     if (coef.sumsq) block_sumsq_out(sq, coef.sumsq + blockIdx.x);
 }
@@ -284,6 +409,60 @@ struct WaveTR<1, OFF, T> {
     }
 };
 
+// Replaces the first `lo` rows of a vector by words that decode to zero
+// (their x is zero too, but they may hold Inf).  On the raw words, so that
+// the decode stays next to its FMA (one v_fma_mix for a half).
+template <int FMT, int DEC, int VEC>
+__device__ __forceinline__ void clear_rows(Raw<FMT, DEC, VEC>& R, int lo) {
+    if (VEC == 1) return;
+    constexpr uint32_t zero = FMT == FMT_P16 ? 0x3801u : 0u;  // FP32_16: the saturated underflow word
+#pragma unroll
+    for (int v = 0; v < VEC - 1; ++v)
+        if (v < lo) {
+            if constexpr (is16<FMT>()) {
+                const uint32_t keep = 0xFFFF0000u >> (16 * (v & 1));
+                R.h[v / 2] = (R.h[v / 2] & keep) | (zero << (16 * (v & 1)));
+                if constexpr (DEC == DEC_EXACT) R.r[v / 2] &= keep;
+            } else if constexpr (FMT == FMT_F32) {
+                R.h[v] = 0;
+            } else {
+                R.h[2 * v] = R.h[2 * v + 1] = 0;
+            }
+        }
+}
+
+template <int FMT, int DEC, int VEC, class ACC>
+__device__ __forceinline__ ACC dot_rows(Raw<FMT, DEC, VEC>& R, const ACC (&xv)[VEC], int lo, bool edge, ACC s) {
+    if (edge) clear_rows<FMT, DEC, VEC>(R, lo);  // wave-uniform: skipped but at the last rows
+    if constexpr (FMT == FMT_P16 && DEC == DEC_EXACT && VEC == 8) {
+        if (__builtin_expect(__any(saturated(R)), 0)) {
+            // element by element in a rolled loop that shifts the vector down:
+            // unrolled here, a block of columns overflows the instruction cache
+            Raw<FMT, DEC, VEC> q = R;
+            ACC xs[VEC];
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) xs[v] = xv[v];
+#pragma clang loop unroll(disable)
+            for (int e = 0; e < VEC; ++e) {
+                s = fma(static_cast<ACC>(decode16<FMT, DEC>(q.h[0] & 0xFFFFu, q.r[0] & 0xFFFFu)), xs[0], s);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    q.h[k] = (q.h[k] >> 16) | (k < 3 ? q.h[(k + 1) & 3] << 16 : 0u);
+                    q.r[k] = (q.r[k] >> 16) | (k < 3 ? q.r[(k + 1) & 3] << 16 : 0u);
+                }
+#pragma unroll
+                for (int v = 0; v < VEC - 1; ++v) xs[v] = xs[v + 1];
+            }
+            return s;
+        }
+    }
+    ACC av[VEC];
+    decode<FMT, DEC, VEC, ACC, false>(R, av);
+#pragma unroll
+    for (int v = 0; v < VEC; ++v) s = fma(av[v], xv[v], s);
+    return s;
+}
+
 template <int FMT, int DEC, int VEC, class ACC, int CB, bool NTL>
 __global__ __launch_bounds__(kThreads) void gemv_t_kernel(
     int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
@@ -302,35 +481,33 @@ __global__ __launch_bounds__(kThreads) void gemv_t_kernel(
 #pragma unroll
     for (int c = 0; c < CB; ++c) acc[c] = ACC(0);
 
-    constexpr int UB = (sizeof(ACC) == 8 || DEC == DEC_EXACT) ? 8 : 16;
-    for (int64_t i = r0 + static_cast<int64_t>(threadIdx.x) * VEC; i < r1;
-         i += static_cast<int64_t>(kThreads) * VEC) {
-        const int nvalid = static_cast<int>(min<int64_t>(VEC, m - i));
+    constexpr int UB = DEC == DEC_EXACT ? 4 : 8;
+    for (int64_t ir = r0 + static_cast<int64_t>(threadIdx.x) * VEC; ir < r1;
+         ir += static_cast<int64_t>(kThreads) * VEC) {
+        const int64_t i = first_row<VEC>(ir, m);
+        const int lo = static_cast<int>(ir - i);
         ACC xv[VEC];
-#pragma unroll
-        for (int v = 0; v < VEC; ++v) xv[v] = (v < nvalid) ? load_x<ACC>(x, x64, i + v) : ACC(0);
+        load_x_rows<VEC, ACC>(x, x64, i, lo, xv);
+        const bool edge = __any(lo != 0);
         const int64_t base = i + c0 * lda;
+        // batches of UB columns, the next batch's loads in flight during this
+        // one's sums; past the last column the last one again, its sum unused
+        Raw<FMT, DEC, VEC> R[2][UB];
+#pragma unroll
+        for (int u = 0; u < UB; ++u)
+            load_raw<FMT, DEC, VEC, NTL>(a, wr, base + min(u, ncols - 1) * lda, R[0][u]);
 #pragma unroll
         for (int cb = 0; cb < CB; cb += UB) {
-            Raw<FMT, DEC, VEC> R[UB];
+            if (cb < ncols) {
+                if (cb + UB < ncols) {
 #pragma unroll
-            for (int u = 0; u < UB; ++u)
-                if (cb + u < ncols) load_raw<FMT, DEC, VEC, NTL>(a, wr, base + (cb + u) * lda, R[u]);
-#pragma unroll
-            for (int u = 0; u < UB; ++u) {
-                if (cb + u < ncols) {
-                    ACC av[VEC];
-                    decode<FMT, DEC, VEC, ACC>(R[u], av);
-                    if (nvalid < VEC) {
-#pragma unroll
-                        for (int v = 0; v < VEC; ++v)
-                            if (v >= nvalid) av[v] = ACC(0);
-                    }
-                    ACC s = acc[cb + u];
-#pragma unroll
-                    for (int v = 0; v < VEC; ++v) s = fma(av[v], xv[v], s);
-                    acc[cb + u] = s;
+                    for (int u = 0; u < UB; ++u)
+                        load_raw<FMT, DEC, VEC, NTL>(a, wr, base + min(cb + UB + u, ncols - 1) * lda,
+                                                     R[(cb / UB + 1) & 1][u]);
                 }
+#pragma unroll
+                for (int u = 0; u < UB; ++u)
+                    acc[cb + u] = dot_rows<FMT, DEC, VEC, ACC>(R[(cb / UB) & 1][u], xv, lo, edge, acc[cb + u]);
             }
         }
     }
@@ -349,25 +526,92 @@ __global__ __launch_bounds__(kThreads) void gemv_t_kernel(
     }
 }
 
+// Short columns: a block owns CG whole columns, so there are no chunk
+// partials and no second launch.  Each lane walks the rows in steps of the
+// block with the loads of four row steps in flight; a vector's VEC products
+// are summed in ACC, everything above that in FP64.  `partial` != nullptr:
+// the sums go there (one chunk) instead of y.  20000 x 200 bf16 hi:
+// 13.4 + 3.5 (chunks and their sum) -> 5.0 us; R^-T v, 300 x 300 FP64: 8.1 -> 4.0.
+constexpr int kColThreads = 512;
+template <int FMT, int DEC, int VEC, class ACC, int CG, bool NTL>
+__global__ __launch_bounds__(kColThreads) void gemv_t_cols_kernel(
+    int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr, int64_t lda,
+    const void* __restrict__ x, bool x64, ACC* __restrict__ partial, void* __restrict__ y, bool y64, Coef coef) {
+    if (coef.skip && *coef.skip) return;
+    constexpr int U = 4;
+    const int64_t c0 = static_cast<int64_t>(blockIdx.x) * CG;
+    const int ncols = static_cast<int>(min<int64_t>(CG, n - c0));
+    double acc[CG];
+#pragma unroll
+    for (int c = 0; c < CG; ++c) acc[c] = 0.0;
+    constexpr int64_t kStep = static_cast<int64_t>(kColThreads) * VEC;
+    for (int64_t ir = static_cast<int64_t>(threadIdx.x) * VEC; ir < m; ir += U * kStep) {
+        Raw<FMT, DEC, VEC> R[U][CG];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (ir + u * kStep < m) {
+                const int64_t base = first_row<VEC>(ir + u * kStep, m) + c0 * lda;
+#pragma unroll
+                for (int c = 0; c < CG; ++c)
+                    load_raw<FMT, DEC, VEC, NTL>(a, wr, base + min(c, ncols - 1) * lda, R[u][c]);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (ir + u * kStep < m) {
+                const int64_t i = first_row<VEC>(ir + u * kStep, m);
+                const int lo = static_cast<int>(ir + u * kStep - i);
+                ACC xv[VEC];
+                load_x_rows<VEC, ACC>(x, x64, i, lo, xv);
+                const bool edge = __any(lo != 0);
+#pragma unroll
+                for (int c = 0; c < CG; ++c)
+                    acc[c] += static_cast<double>(dot_rows<FMT, DEC, VEC, ACC>(R[u][c], xv, lo, edge, ACC(0)));
+            }
+    }
+    __shared__ double red[kColThreads / 64][CG];
+#pragma unroll
+    for (int c = 0; c < CG; ++c) {
+        for (int o = 32; o >= 1; o >>= 1) acc[c] += __shfl_xor(acc[c], o);
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][c] = acc[c];
+    }
+    __syncthreads();
+    if (static_cast<int>(threadIdx.x) < ncols) {
+        const int c = threadIdx.x;
+        double s = 0.0;
+        for (int w = 0; w < kColThreads / 64; ++w) s += red[w][c];
+        if (partial) partial[c0 + c] = static_cast<ACC>(s);
+        else
+            store_y(y, y64, c0 + c, read_coef(coef.alpha, coef.dalpha, coef.alpha_mul), s,
+                    read_coef(coef.beta, coef.dbeta, coef.beta_mul));
+    }
+}
+
+// Adds the chunk partials of 32 columns: 8 chunk slices per column (a slice
+// takes every eighth chunk, four loads in flight), added in slice order
+// (64 chunks x 501: 7.0 us with a thread per column, 5.1 with the slices).
+constexpr int kFinCols = 32, kFinSlices = kThreads / kFinCols;
 template <class ACC>
 __global__ __launch_bounds__(kThreads) void gemv_t_finish(int64_t n, int chunks,
                                                           const ACC* __restrict__ partial,
                                                           void* __restrict__ y, bool y64,
                                                           Coef coef) {
     if (coef.skip && *coef.skip) return;
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-    if (j >= n) return;
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-    int c = 0;
-    for (; c + 3 < chunks; c += 4) {
-        s0 += static_cast<double>(partial[static_cast<int64_t>(c) * n + j]);
-        s1 += static_cast<double>(partial[static_cast<int64_t>(c + 1) * n + j]);
-        s2 += static_cast<double>(partial[static_cast<int64_t>(c + 2) * n + j]);
-        s3 += static_cast<double>(partial[static_cast<int64_t>(c + 3) * n + j]);
-    }
-    for (; c < chunks; ++c) s0 += static_cast<double>(partial[static_cast<int64_t>(c) * n + j]);
-    const double s = (s0 + s1) + (s2 + s3);
-    store_y(y, y64, j, read_coef(coef.alpha, coef.dalpha, coef.alpha_mul), s,
+    const int col = threadIdx.x % kFinCols, slice = threadIdx.x / kFinCols;
+    const int64_t j = static_cast<int64_t>(blockIdx.x) * kFinCols + col;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    if (j < n)
+        for (int c = slice; c < chunks; c += 4 * kFinSlices)
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (c + q * kFinSlices < chunks)
+                    s[q] += static_cast<double>(partial[static_cast<int64_t>(c + q * kFinSlices) * n + j]);
+    __shared__ double red[kFinSlices][kFinCols];
+    red[slice][col] = (s[0] + s[1]) + (s[2] + s[3]);
+    __syncthreads();
+    if (slice != 0 || j >= n) return;
+    double t = 0.0;
+    for (int q = 0; q < kFinSlices; ++q) t += red[q][col];
+    store_y(y, y64, j, read_coef(coef.alpha, coef.dalpha, coef.alpha_mul), t,
             read_coef(coef.beta, coef.dbeta, coef.beta_mul));
 }
 
@@ -400,27 +644,33 @@ int vec_full_of(int fmt) { return fmt == FMT_F64 ? 2 : (fmt == FMT_F32 ? 4 : 8);
 int cb_of(const Kind& k) { return k.acc64 ? 32 : 64; }
 constexpr int64_t kTargetBlocks = 1024;
 
-struct PlanN {
-    int64_t bx;
-    int splits;
-    int64_t col_chunk;
-};
-PlanN plan_n(const Kind& k, int64_t m, int64_t n) {
-    PlanN p;
-    p.bx = ceil_div(m, kThreads * vec_full_of(k.fmt));
-    p.splits = 1;
-    p.col_chunk = std::max<int64_t>(n, 1);
-    if (p.bx < kTargetBlocks / 2 && n > 16) {
-        int64_t want = ceil_div(kTargetBlocks, p.bx);
-        // at most 32 column splits: the finishing pass adds them per row in
-        // sequence, and more blocks than that on a small matrix cost more
-        // there than they save in the pass over A
-        int64_t max_splits = std::min<int64_t>(ceil_div(n, 8), 32);
-        int64_t s = std::min(want, max_splits);
-        p.col_chunk = ceil_div(n, s);
-        p.splits = static_cast<int>(ceil_div(n, p.col_chunk));
-    }
-    return p;
+// NO_TRANSPOSE: `waves` = 1 gives every lane its own rows (gemv_n_kernel);
+// more split the columns over the waves of a block (gemv_n_split_kernel)
+// until about kTargetWaves waves share the work, two columns a wave at least.
+constexpr int64_t kTargetWaves = 4096;
+int n_waves(const Kind& k, int64_t m, int64_t n) {
+    const int64_t v = m >= vec_full_of(k.fmt) ? vec_full_of(k.fmt) : 1;
+    const int64_t row_waves = ceil_div(m, 64 * v);
+    const int64_t most = std::min<int64_t>(16, kSplitLds / (v * (k.acc64 ? 8 : 4)));
+    int64_t w = 1;
+    while (w < most && row_waves * w < kTargetWaves && n >= 4 * w) w *= 2;
+    return static_cast<int>(w);
+}
+
+// Row lanes of a split block: 16 while 64-lane blocks are under a quarter of
+// the wanted waves and every column group still has a column.
+int n_row_lanes(int64_t waves64, int64_t n, int waves) {
+    return waves64 < kTargetWaves / 4 && n >= 4 * waves ? 16 : 64;
+}
+
+// Scratch columns of the NO_TRANSPOSE size contract: callers size their
+// scratch by it, the kernels need none.
+int n_scratch_splits(const Kind& k, int64_t m, int64_t n) {
+    const int64_t bx = ceil_div(m, static_cast<int64_t>(kThreads) * vec_full_of(k.fmt));
+    if (bx >= kTargetBlocks / 2 || n <= 16) return 0;
+    const int64_t s = std::min(ceil_div(kTargetBlocks, bx), std::min<int64_t>(ceil_div(n, 8), 32));
+    const int64_t splits = ceil_div(n, ceil_div(n, s));
+    return splits > 1 ? static_cast<int>(splits) : 0;
 }
 
 struct PlanT {
@@ -441,6 +691,14 @@ PlanT plan_t(const Kind& k, int64_t m, int64_t n) {
     return p;
 }
 
+// TRANSPOSE: whole columns per block (gemv_t_cols_kernel) up to this many
+// bytes a column; longer ones are cut into row chunks.
+constexpr int64_t kColBytes = int64_t(128) << 10;
+bool t_cols(const Kind& k, int64_t m) {
+    const int64_t esz = k.fmt == FMT_F64 ? 8 : (k.fmt == FMT_F32 || k.dec == DEC_EXACT ? 4 : 2);
+    return m * esz <= kColBytes;
+}
+
 // The kind a GEMV runs with: F32 GEMV^T accumulates in FP64 in every tier
 // (the FP64-sum kernel streams A faster on gfx950 than the FP32-sum one,
 // and it is the more accurate; the reference's tiled FP32 GEMV accumulates
@@ -454,76 +712,107 @@ Kind kind_for(int a_type, int tier, int trans) {
 size_t scratch_for(const Kind& k, int trans, int64_t m, int64_t n) {
     const size_t acc = k.acc64 ? 8 : 4;
     if (trans == TOMOS_NO_TRANSPOSE) {
-        PlanN p = plan_n(k, m, n);
-        return p.splits > 1 ? static_cast<size_t>(p.splits) * static_cast<size_t>(m) * acc : 0;
+        return static_cast<size_t>(n_scratch_splits(k, m, n)) * static_cast<size_t>(m) * acc;
     }
     PlanT p = plan_t(k, m, n);
     return static_cast<size_t>(p.chunks) * static_cast<size_t>(n) * acc;
 }
 
-// Matrix bytes one GEMV pass reads.
+// Whether a pass over the matrix uses non-temporal loads: columns on 16-byte
+// boundaries only, since a vector that straddles two cache lines wants the
+// line kept for its neighbour (131071 x 501 EXACT, odd lda: N 115 us
+// non-temporal, 77 us cacheable).
 template <int FMT, int DEC>
-int64_t matrix_bytes(int64_t m, int64_t n) {
+bool streams(int64_t m, int64_t n, int64_t lda) {
     const int64_t esz = FMT == FMT_F64 ? 8 : (FMT == FMT_F32 ? 4 : (DEC == DEC_EXACT ? 4 : 2));
-    return m * n * esz;
+    return lda % vec_full<FMT>() == 0 && stream_loads(m * n * esz);
+}
+
+template <int FMT, int DEC, int VEC, class ACC, bool NTL>
+int launch_n(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x, bool x64,
+             void* y, bool y64, const Coef& coef, int waves, hipStream_t s) {
+    if (waves > 1) {
+        const int rl = n_row_lanes(ceil_div(m, 64 * VEC) * waves, n, waves);
+        const unsigned blocks = static_cast<unsigned>(ceil_div(m, rl * VEC));
+        const int64_t chunk = ceil_div(n, waves * (64 / rl));
+        if (rl == 16)
+            gemv_n_split_kernel<FMT, DEC, VEC, ACC, 16, NTL><<<blocks, 64 * waves, 0, s>>>(
+                m, n, a, wr, lda, x, x64, y, y64, coef, chunk);
+        else
+            gemv_n_split_kernel<FMT, DEC, VEC, ACC, 64, NTL><<<blocks, 64 * waves, 0, s>>>(
+                m, n, a, wr, lda, x, x64, y, y64, coef, chunk);
+        TOMOS_LAUNCH_CHECK("gemv_n_split_kernel");
+        return static_cast<int>(blocks);
+    }
+    const unsigned blocks = static_cast<unsigned>(ceil_div(m, static_cast<int64_t>(kThreads) * VEC));
+    gemv_n_kernel<FMT, DEC, VEC, ACC, NTL><<<blocks, kThreads, 0, s>>>(m, n, a, wr, lda, x, x64, y, y64, coef);
+    TOMOS_LAUNCH_CHECK("gemv_n_kernel");
+    return static_cast<int>(blocks);
 }
 
 template <int FMT, int DEC, class ACC>
 int run_n(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x,
-          bool x64, void* y, bool y64, const Coef& coef, void* scratch, bool vec,
-          const PlanN& p, hipStream_t s) {
+          bool x64, void* y, bool y64, const Coef& coef, int waves, hipStream_t s) {
     constexpr int VF = vec_full<FMT>();
-    ACC* part = p.splits > 1 ? static_cast<ACC*>(scratch) : nullptr;
-    const int width = vec ? VF : 1;
-    const dim3 grid(static_cast<unsigned>(ceil_div(m, static_cast<int64_t>(kThreads) * width)),
-                    static_cast<unsigned>(p.splits));
-    if (width == VF && stream_loads(matrix_bytes<FMT, DEC>(m, n)))
-        gemv_n_kernel<FMT, DEC, VF, ACC, true><<<grid, kThreads, 0, s>>>(m, n, a, wr, lda, x, x64, y, y64,
-                                                                         coef, p.col_chunk, part);
-    else if (width == VF)
-        gemv_n_kernel<FMT, DEC, VF, ACC, false><<<grid, kThreads, 0, s>>>(m, n, a, wr, lda, x, x64, y, y64,
-                                                                          coef, p.col_chunk, part);
-    else
-        gemv_n_kernel<FMT, DEC, 1, ACC, false><<<grid, kThreads, 0, s>>>(m, n, a, wr, lda, x, x64, y, y64,
-                                                                         coef, p.col_chunk, part);
-    TOMOS_LAUNCH_CHECK("gemv_n_kernel");
-    if (part) {
-        gemv_n_finish<ACC><<<dim3(static_cast<unsigned>(ceil_div(m, kThreads))), kThreads, 0, s>>>(
-            m, p.splits, part, y, y64, coef);
-        TOMOS_LAUNCH_CHECK("gemv_n_finish");
-        return static_cast<int>(ceil_div(m, kThreads));
-    }
-    return static_cast<int>(grid.x);
+    if (m < VF)
+        return launch_n<FMT, DEC, 1, ACC, false>(m, n, a, wr, lda, x, x64, y, y64, coef, waves, s);
+    if (streams<FMT, DEC>(m, n, lda))
+        return launch_n<FMT, DEC, VF, ACC, true>(m, n, a, wr, lda, x, x64, y, y64, coef, waves, s);
+    return launch_n<FMT, DEC, VF, ACC, false>(m, n, a, wr, lda, x, x64, y, y64, coef, waves, s);
 }
 
+template <int FMT, int DEC, int VEC, class ACC, bool NTL>
+void launch_t_cols(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x, bool x64,
+                   ACC* part, void* y, bool y64, const Coef& coef, hipStream_t s) {
+    // one column a block while that fills the chip about twice, then two, then four
+    if (n <= 512)
+        gemv_t_cols_kernel<FMT, DEC, VEC, ACC, 1, NTL><<<static_cast<unsigned>(n), kColThreads, 0, s>>>(
+            m, n, a, wr, lda, x, x64, part, y, y64, coef);
+    else if (n <= 1024)
+        gemv_t_cols_kernel<FMT, DEC, VEC, ACC, 2, NTL><<<static_cast<unsigned>(ceil_div(n, 2)), kColThreads, 0, s>>>(
+            m, n, a, wr, lda, x, x64, part, y, y64, coef);
+    else
+        gemv_t_cols_kernel<FMT, DEC, VEC, ACC, 4, NTL><<<static_cast<unsigned>(ceil_div(n, 4)), kColThreads, 0, s>>>(
+            m, n, a, wr, lda, x, x64, part, y, y64, coef);
+    TOMOS_LAUNCH_CHECK("gemv_t_cols_kernel");
+}
+
+// Returns the number of chunk partials written when `finish` is false.
 template <int FMT, int DEC, class ACC>
-void run_t(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x,
-           bool x64, void* y, bool y64, const Coef& coef, void* scratch, bool vec,
-           const PlanT& p, hipStream_t s, bool finish = true) {
+int run_t(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x,
+          bool x64, void* y, bool y64, const Coef& coef, void* scratch, bool cols,
+          const PlanT& p, hipStream_t s, bool finish = true) {
     constexpr int VF = vec_full<FMT>();
     constexpr int CB = sizeof(ACC) == 8 ? 32 : 64;
     ACC* part = static_cast<ACC*>(scratch);
+    if (cols && m > 0) {
+        require(n < (int64_t(1) << 31), "gemv: grid too large");
+        ACC* one = finish ? nullptr : part;
+        if (m < VF)
+            launch_t_cols<FMT, DEC, 1, ACC, false>(m, n, a, wr, lda, x, x64, one, y, y64, coef, s);
+        else
+            launch_t_cols<FMT, DEC, VF, ACC, false>(m, n, a, wr, lda, x, x64, one, y, y64, coef, s);
+        return 1;
+    }
     const int64_t blocks = static_cast<int64_t>(p.chunks) * p.ncg;
     require(blocks < (int64_t(1) << 31), "gemv: grid too large");
     if (m > 0) {
         const dim3 grid(static_cast<unsigned>(blocks));
         // the EXACT tier reads A with cacheable loads: its non-temporal form
         // needs 256 VGPRs (one wave per SIMD), the cacheable one ~140
-        if (vec && DEC != DEC_EXACT && stream_loads(matrix_bytes<FMT, DEC>(m, n)))
+        if (DEC != DEC_EXACT && streams<FMT, DEC>(m, n, lda))
             gemv_t_kernel<FMT, DEC, VF, ACC, CB, true><<<grid, kThreads, 0, s>>>(
                 m, n, a, wr, lda, x, x64, p.rows_per_chunk, p.ncg, part, coef.skip);
-        else if (vec)
+        else  // m > kColBytes / 8, so at least a vector
             gemv_t_kernel<FMT, DEC, VF, ACC, CB, false><<<grid, kThreads, 0, s>>>(
-                m, n, a, wr, lda, x, x64, p.rows_per_chunk, p.ncg, part, coef.skip);
-        else
-            gemv_t_kernel<FMT, DEC, 1, ACC, CB, false><<<grid, kThreads, 0, s>>>(
                 m, n, a, wr, lda, x, x64, p.rows_per_chunk, p.ncg, part, coef.skip);
         TOMOS_LAUNCH_CHECK("gemv_t_kernel");
     }
-    if (!finish) return;
-    gemv_t_finish<ACC><<<dim3(static_cast<unsigned>(ceil_div(n, kThreads))), kThreads, 0, s>>>(
+    if (!finish) return p.chunks;
+    gemv_t_finish<ACC><<<dim3(static_cast<unsigned>(ceil_div(n, kFinCols))), kThreads, 0, s>>>(
         n, m > 0 ? p.chunks : 0, part, y, y64, coef);
     TOMOS_LAUNCH_CHECK("gemv_t_finish");
+    return p.chunks;
 }
 
 }  // namespace
@@ -532,7 +821,12 @@ size_t gemv_scratch_bytes(int a_type, int tier, int trans, int64_t m, int64_t n)
     return scratch_for(kind_for(a_type, tier, trans), trans, m, n);
 }
 
-int64_t gemv_sumsq_blocks_max(int64_t m) { return ceil_div(std::max<int64_t>(m, 1), kThreads); }
+// 16 rows a block at least; split blocks of 16 row lanes only while there are
+// under kTargetWaves / 2 of them, otherwise at least 128 rows (m < VEC: one block).
+int64_t gemv_sumsq_blocks_max(int64_t m) {
+    m = std::max<int64_t>(m, 1);
+    return std::min(ceil_div(m, 16), std::max(ceil_div(m, 128), kTargetWaves / 2));
+}
 
 void gemv(int a_type, int tier, int trans, const Coef& coef, int64_t m, int64_t n, const void* a,
           const uint16_t* wr, int64_t lda, int x_type, const void* x, int y_type, void* y,
@@ -552,25 +846,22 @@ void gemv(int a_type, int tier, int trans, const Coef& coef, int64_t m, int64_t 
     if (inner > 0) require(a != nullptr && x != nullptr, "gemv: null A or x");
     if (k.dec == DEC_EXACT) require(wr != nullptr || inner == 0, "gemv: EXACT tier needs the wr plane");
     const size_t need = scratch_for(k, trans, m, n);
+    const bool cols = trans == TOMOS_TRANSPOSE && m > 0 && t_cols(k, m);
     if (need > 0) {
         if (scratch == nullptr) {
-            scratch = fallback_scratch(need);
+            if (trans == TOMOS_TRANSPOSE && !cols) scratch = fallback_scratch(need);
         } else {
             require(scratch_bytes >= need, "gemv: scratch too small (need " + std::to_string(need) +
                                                " bytes)");
         }
     }
     const bool x64 = x_type == TOMOS_F64, y64 = y_type == TOMOS_F64;
-    const int vf = vec_full_of(k.fmt);
-    const size_t vb = 16;
-    bool vec = (lda % vf == 0) && (reinterpret_cast<uintptr_t>(a) % vb == 0) &&
-               (k.dec != DEC_EXACT || reinterpret_cast<uintptr_t>(wr) % vb == 0);
 
     if (trans == TOMOS_NO_TRANSPOSE) {
         // n == 0 falls through with an empty column range: y = beta*y.
-        const PlanN p = plan_n(k, m, n);
-int nb = 0;
-#define RUN_N(F, D, A) nb = run_n<F, D, A>(m, n, a, wr, lda, x, x64, y, y64, coef, scratch, vec, p, s)
+        const int waves = n_waves(k, m, n);
+        int nb = 0;
+#define RUN_N(F, D, A) nb = run_n<F, D, A>(m, n, a, wr, lda, x, x64, y, y64, coef, waves, s)
         if (k.fmt == FMT_F32) { if (k.acc64) RUN_N(FMT_F32, DEC_NATIVE, double); else RUN_N(FMT_F32, DEC_NATIVE, float); }
         else if (k.fmt == FMT_F64) RUN_N(FMT_F64, DEC_NATIVE, double);
         else if (k.fmt == FMT_H16) { if (k.acc64) RUN_N(FMT_H16, DEC_HI, double); else RUN_N(FMT_H16, DEC_HI, float); }
@@ -587,7 +878,7 @@ int nb = 0;
         if (sumsq_blocks) *sumsq_blocks = nb;
     } else {
         const PlanT p = plan_t(k, m, n);
-#define RUN_T(F, D, A) run_t<F, D, A>(m, n, a, wr, lda, x, x64, y, y64, coef, scratch, vec, p, s)
+#define RUN_T(F, D, A) run_t<F, D, A>(m, n, a, wr, lda, x, x64, y, y64, coef, scratch, cols, p, s)
         if (k.fmt == FMT_F32) { if (k.acc64) RUN_T(FMT_F32, DEC_NATIVE, double); else RUN_T(FMT_F32, DEC_NATIVE, float); }
         else if (k.fmt == FMT_F64) RUN_T(FMT_F64, DEC_NATIVE, double);
         else if (k.fmt == FMT_H16) { if (k.acc64) RUN_T(FMT_H16, DEC_HI, double); else RUN_T(FMT_H16, DEC_HI, float); }
@@ -614,19 +905,19 @@ int gemv_t_partials(int a_type, int tier, int64_t m, int64_t n, const void* a, c
     require(scratch != nullptr && scratch_bytes >= need, "gemv_t_partials: scratch too small");
     const PlanT p = plan_t(k, m, n);
     const bool x64 = x_type == TOMOS_F64;
-    const int vf = vec_full_of(k.fmt);
-    const bool vec = (lda % vf == 0) && (reinterpret_cast<uintptr_t>(a) % 16 == 0) &&
-                     (k.dec != DEC_EXACT || reinterpret_cast<uintptr_t>(wr) % 16 == 0);
+    const bool cols = t_cols(k, m);
     Coef c;
     c.skip = skip;
-#define RUN_TP(F, D) run_t<F, D, double>(m, n, a, wr, lda, x, x64, nullptr, false, c, scratch, vec, p, s, false)
+    int chunks = 0;
+#define RUN_TP(F, D) \
+    chunks = run_t<F, D, double>(m, n, a, wr, lda, x, x64, nullptr, false, c, scratch, cols, p, s, false)
     if (k.fmt == FMT_F32) RUN_TP(FMT_F32, DEC_NATIVE);
     else if (k.fmt == FMT_F64) RUN_TP(FMT_F64, DEC_NATIVE);
     else if (k.fmt == FMT_H16) RUN_TP(FMT_H16, DEC_HI);
     else if (k.fmt == FMT_P16) { if (k.dec == DEC_EXACT) RUN_TP(FMT_P16, DEC_EXACT); else RUN_TP(FMT_P16, DEC_HI); }
     else { if (k.dec == DEC_EXACT) RUN_TP(FMT_PBF, DEC_EXACT); else RUN_TP(FMT_PBF, DEC_HI); }
 #undef RUN_TP
-    return p.chunks;
+    return chunks;
 }
 
 }  // namespace tomos_hip
