@@ -101,3 +101,27 @@ def test_decode_wh_all_words(capi, orc, dec, fn):
         assert np.all((got[nan] & 0x7F80) == 0x7F80) and np.all((got[nan] & 0x7F) != 0)
     else:
         assert np.array_equal(got, exp)
+
+
+@pytest.mark.parametrize("m,n", [(1, 1), (7, 3), (8, 2), (9, 5), (2047, 2), (2049, 3)])
+@pytest.mark.parametrize("pad", [0, 1, 8])
+def test_unpack_runs_and_remainders(capi, orc, m, n, pad):
+    """Every decoder on rows that end inside a run of 8, columns without
+    padding (one long column), at odd and at aligned leading dimensions; words
+    of every class, saturated ones among them; nothing is written past row m."""
+    rng = np.random.default_rng(m + pad)
+    A = (rng.standard_normal((m, n)) * 2.0 ** rng.integers(-34, 34, (m, n))).astype(np.float32)
+    ld = m + pad
+    for variant, decs in ((0, (0, 1, 2, 3)), (2, (7,)), (3, (4, 5)), (4, (6,))):
+        eh, er = orc.pack(variant, A)
+        sh, sr = np.full((ld, n), 0x7FFF, np.uint16, order="F"), np.full((ld, n), 0x7FFF, np.uint16, order="F")
+        sh[:m], sr[:m] = eh, er
+        wh, wr = H.dev(sh), H.dev(sr)
+        for dec in decs:
+            print("unpack", variant, dec, m, n, pad, flush=True)
+            out = H.dev(np.full((ld, n), -7.0, np.float32))
+            C.call("tomos_unpack", dec, m, n, wh.ptr, wr.ptr, ld, out.ptr, ld, None)
+            got = out.to_numpy(np.float32, (ld, n))
+            exp = orc.unpack(dec, eh, er)
+            assert np.array_equal(got[:m].view(np.uint32), np.ascontiguousarray(exp).astype(np.float32).view(np.uint32)), dec
+            assert np.all(got[m:] == -7.0)
