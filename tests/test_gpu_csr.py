@@ -291,3 +291,41 @@ def test_convert_roundtrip(capi):
     assert np.array_equal(got32, A.astype(np.float32))
     assert np.array_equal(d64.to_numpy(np.float64, (50, 7)), A.astype(np.float32).astype(np.float64))
     assert C.lib().tomos_convert(C.F16, C.F32, 1, 1, s.ptr, 1, d32.ptr, 1, None) == 1
+
+
+@pytest.mark.parametrize("vt", [C.F64, C.F32, C.BF16])
+@pytest.mark.parametrize("it", [C.INDEX_INT32, C.INDEX_INT64])
+@pytest.mark.parametrize("m,n,mean,long_row", [
+    (1, 1, 1, 0), (3, 2048, 5, 0), (5000, 256, 3, 0), (5000, 257, 3, 0), (3000, 1024, 40, 0), (3000, 1025, 40, 0),
+    (3000, 2049, 9, 0), (60000, 7, 1, 0), (900, 300, 20, 30000), (2, 64, 1, 20000)])
+def test_transpose_tiles(capi, vt, it, m, n, mean, long_row):
+    """The transpose is the stable one at the edges of its tiles: both sides
+    of the column limits, most rows empty, a row longer than a sorted chunk
+    (its columns repeat many times), fewer rows than a tile."""
+    rng = np.random.default_rng(m + n)
+    ln = rng.poisson(mean, m)
+    ln[rng.random(m) < 0.3] = 0
+    if long_row:
+        ln[m // 2] = long_row
+    ln[-1] = max(ln[-1], 1)
+    rp = np.concatenate([[0], np.cumsum(ln)])
+    nnz = int(rp[-1])
+    ci = rng.integers(0, n, nnz)
+    ci[rng.random(nnz) < 0.5] = 0  # one column far longer than the others
+    v = rng.standard_normal(nnz)
+    idt = np.int64 if it == C.INDEX_INT64 else np.int32
+    bits = {C.F64: lambda a: a, C.F32: lambda a: a.astype(np.float32),
+            C.BF16: lambda a: (a.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)}[vt](v)
+    rpd, cid, vd = H.dev(rp.astype(idt)), H.dev(ci.astype(idt)), H.dev(bits)
+    vt_, pt_, it_ = (C.DeviceBuffer(max(bits.nbytes, 8)), C.DeviceBuffer((n + 1) * idt().itemsize),
+                     C.DeviceBuffer(max(nnz * idt().itemsize, 8)))
+    need = C.lib().tomos_csr_transpose_scratch_size(vt, it, m, n, nnz)
+    sc = C.DeviceBuffer(need)
+    print("transpose", vt, it, m, n, nnz, flush=True)
+    C.call("tomos_csr_transpose", vt, it, m, n, nnz, vd.ptr, rpd.ptr, cid.ptr, vt_.ptr, pt_.ptr, it_.ptr, sc.ptr, need,
+           None)
+    order = np.argsort(ci, kind="stable")
+    rows = np.repeat(np.arange(m), ln)
+    assert np.array_equal(pt_.to_numpy(idt, (n + 1,)), np.concatenate([[0], np.cumsum(np.bincount(ci, minlength=n))]))
+    assert np.array_equal(it_.to_numpy(idt, (nnz,)), rows[order])
+    assert np.array_equal(vt_.to_numpy(bits.dtype, (nnz,)), bits[order])

@@ -3,17 +3,18 @@
 // src/kernels/cpu/matrix/matrix_cpu_kernels.cpp:92-131) and the CSR
 // transpose that lets LSQR form A^T u without atomics.
 //
-// A*x: L lanes of a wavefront share one row (L in {1, 4, 16, 64}, from the
-// mean row length), each lane sums a lane-strided part of the row in FP64
-// and the group folds its partial sums with a butterfly of lane shuffles.
+// A*x: L lanes of a wavefront share one row (L in {1, 4, 8, 16, 32, 64}, from
+// the mean row length), each lane sums four consecutive entries a round in
+// FP64 and the group folds its partial sums with a butterfly of lane shuffles.
 // The order of every sum depends only on (m, nnz), so results repeat bit
 // for bit.  Bound: HBM, nnz*(value + index bytes) + (m+1) index bytes + the
 // y traffic, with x gathered through the caches.
 //
 // A^T*x: the reference scatters into y (matrix_cpu_kernels.cpp:116-130);
-// here A^T is built once as a CSR matrix of its own (a stable radix sort of
-// the column indices keeps A's row order inside each row of A^T) and the
-// A*x kernel runs on it: no atomics, deterministic, coalesced.
+// here A^T is built once as a CSR matrix of its own (a stable counting sort by
+// column, a radix sort above 2048 columns, keeps A's row order inside each
+// row of A^T) and the A*x kernel runs on it: no atomics, deterministic,
+// coalesced.
 #include <type_traits>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -43,6 +44,42 @@ __device__ __forceinline__ int64_t clamp_ptr(I p, int64_t nnz) {
     const int64_t q = static_cast<int64_t>(p);
     return q < 0 ? 0 : (q > nnz ? nnz : q);
 }
+
+// Four consecutive entries k .. k+3 of a row that ends at k1, as one vector
+// load each of the indices and the values (element alignment), undecoded so
+// that a load can stay in flight; past the row's end the index is `none`,
+// which no product uses.
+template <int VT, class I>
+struct Entries {
+    using V = typename std::conditional<VT == TOMOS_F64, double,
+                                        typename std::conditional<VT == TOMOS_F32, float, uint16_t>::type>::type;
+    typedef I idx4 __attribute__((ext_vector_type(4), aligned(sizeof(I))));
+    typedef V val4 __attribute__((ext_vector_type(4), aligned(sizeof(V))));
+    idx4 i;
+    val4 w;
+
+    __device__ __forceinline__ void load(const void* vals, const I* ci, int64_t k, int64_t k1, I none) {
+        if (k + 4 <= k1) {
+            i = *reinterpret_cast<const idx4*>(ci + k);
+            w = *reinterpret_cast<const val4*>(static_cast<const V*>(vals) + k);
+        } else {
+            i = none;
+            w = V(0);
+#pragma unroll
+            for (int u = 0; u < 3; ++u)
+                if (k + u < k1) {
+                    i[u] = ci[k + u];
+                    w[u] = static_cast<const V*>(vals)[k + u];
+                }
+        }
+    }
+    __device__ __forceinline__ uint64_t col(int u) const { return static_cast<uint64_t>(static_cast<int64_t>(i[u])); }
+    __device__ __forceinline__ double val(int u) const {
+        if constexpr (VT == TOMOS_F16) return codec::half_bits_to_f32(w[u]);
+        else if constexpr (VT == TOMOS_BF16) return codec::u2f(static_cast<uint32_t>(w[u]) << 16);
+        else return w[u];
+    }
+};
 
 struct MvArgs {
     int64_t m, n, nnz;
@@ -88,24 +125,18 @@ __global__ __launch_bounds__(kCsrThreads) void csr_mv_kernel(MvArgs a) {
         const int64_t k0 = clamp_ptr(rp[row], a.nnz);
         int64_t k1 = clamp_ptr(rp[row + 1], a.nnz);
         k1 = k1 < k0 ? k0 : k1;
-        // four independent chains keep four entries' loads in flight per lane
+        // four chains; four consecutive entries a lane and round, one 16-byte
+        // load each of 32-bit indices and FP32 values (2e6 rows of 50: 225 us
+        // with entry-wise loads at stride L, 204 us so)
         double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0, acc3 = 0.0;
-        int64_t k = k0 + lane;
-        for (; k + 3 * L < k1; k += 4 * L) {
-            const uint64_t c0 = static_cast<uint64_t>(static_cast<int64_t>(ci[k]));
-            const uint64_t c1 = static_cast<uint64_t>(static_cast<int64_t>(ci[k + L]));
-            const uint64_t c2 = static_cast<uint64_t>(static_cast<int64_t>(ci[k + 2 * L]));
-            const uint64_t c3 = static_cast<uint64_t>(static_cast<int64_t>(ci[k + 3 * L]));
-            const double v0 = load_val<VT>(a.vals, k), v1 = load_val<VT>(a.vals, k + L);
-            const double v2 = load_val<VT>(a.vals, k + 2 * L), v3 = load_val<VT>(a.vals, k + 3 * L);
-            if (c0 < static_cast<uint64_t>(a.n)) acc0 = fma(v0, load_x(a, c0), acc0);
-            if (c1 < static_cast<uint64_t>(a.n)) acc1 = fma(v1, load_x(a, c1), acc1);
-            if (c2 < static_cast<uint64_t>(a.n)) acc2 = fma(v2, load_x(a, c2), acc2);
-            if (c3 < static_cast<uint64_t>(a.n)) acc3 = fma(v3, load_x(a, c3), acc3);
-        }
-        for (; k < k1; k += L) {
-            const uint64_t c0 = static_cast<uint64_t>(static_cast<int64_t>(ci[k]));
-            if (c0 < static_cast<uint64_t>(a.n)) acc0 = fma(load_val<VT>(a.vals, k), load_x(a, c0), acc0);
+        const uint64_t n = static_cast<uint64_t>(a.n);
+        for (int64_t k = k0 + 4 * lane; k < k1; k += 4 * L) {
+            Entries<VT, I> e;
+            e.load(a.vals, ci, k, k1, I(-1));
+            if (e.col(0) < n) acc0 = fma(e.val(0), load_x(a, e.col(0)), acc0);
+            if (e.col(1) < n) acc1 = fma(e.val(1), load_x(a, e.col(1)), acc1);
+            if (e.col(2) < n) acc2 = fma(e.val(2), load_x(a, e.col(2)), acc2);
+            if (e.col(3) < n) acc3 = fma(e.val(3), load_x(a, e.col(3)), acc3);
         }
         double acc = (acc0 + acc1) + (acc2 + acc3);
 #pragma unroll
@@ -598,6 +629,367 @@ void transpose_impl(const CsrMat& A, int64_t panel_rows, void* vals_t, void* ptr
     TOMOS_LAUNCH_CHECK("csr_gather_kernel");
 }
 
+// ---- transpose by counting ---------------------------------------------------
+// Stable counting sort of the entries by (panel, column).  A's rows are cut
+// into tiles of about kTileEntries entries, a block each: it counts its
+// tile's columns in LDS, two scans turn the counts into the tile's first
+// position of every column, and a second kernel sorts the tile's entries by
+// column in LDS and writes them out, so that a column's entries of one tile
+// leave as one run.  (Written straight to their places, four bytes at a
+// time from some thousand open lines per wavefront, they took 3.8 ms.)
+// Entries of one 64-entry step that share a column are ranked by lane and
+// wavefronts take consecutive parts of a tile, so the result is the stable
+// one, whatever the launch shape.
+// Bound: the entries are read twice and written once (20 B an entry for
+// FP32 values and 32-bit indices), and the lane ranking costs about 100 VALU
+// operations per 64 entries.  A radix sort of packed (row, value) pairs,
+// which this replaces for n <= kCountCols, moved them through HBM three
+// times and needed the keys, the packing and the row of every entry besides:
+// 2e6 x 1000 with 1e8 entries 3.55 ms, now 0.87 (count 0.12, scans 0.03,
+// sort 0.71: 2.2 TB/s).
+constexpr int64_t kCountCols = 2048;      // above, a tile's runs are a few entries long
+constexpr int64_t kTileEntries = 6144;    // a chunk of the sorting kernel: two blocks a CU (12288: one, 1.38 ms)
+constexpr int64_t kTileRows = 2048;       // a tile's row starts in LDS
+constexpr int64_t kGroupTiles = 64;       // tiles per scan group
+
+struct CountPlan {
+    int64_t panel_rows, panels;
+    int64_t tile_rows, tiles;    // rows per tile, tiles per panel
+    int64_t groups;              // scan groups per panel
+};
+
+bool count_transpose(const CsrMat& A) {
+    return A.n >= 1 && A.n <= kCountCols && A.nnz < (int64_t(1) << 32);
+}
+
+CountPlan count_plan(const CsrMat& A, int64_t panel_rows) {
+    CountPlan p;
+    p.panel_rows = panel_rows;
+    p.panels = A.m > 0 ? ceil_div(A.m, panel_rows) : 1;
+    // full tiles where they make two rounds over the chip, smaller ones otherwise
+    const int64_t want = std::min(std::max<int64_t>(A.nnz / 512, 1024), kTileEntries);
+    const double mean = A.m > 0 ? static_cast<double>(A.nnz) / static_cast<double>(A.m) : 1.0;
+    const int64_t rows = static_cast<int64_t>(static_cast<double>(want) / std::max(mean, 1e-3));
+    p.tile_rows = std::min(std::min(std::max<int64_t>(rows, 1), kTileRows), panel_rows);
+    p.tiles = ceil_div(std::min(panel_rows, std::max<int64_t>(A.m, 1)), p.tile_rows);
+    p.groups = ceil_div(p.tiles, kGroupTiles);
+    return p;
+}
+
+size_t count_bytes(const CsrMat& A, int64_t panel_rows) {
+    const CountPlan p = count_plan(A, panel_rows);
+    const size_t n = static_cast<size_t>(A.n), pn = static_cast<size_t>(p.panels);
+    return align256(pn * static_cast<size_t>(p.tiles) * n * 4) + align256(pn * static_cast<size_t>(p.groups) * n * 4);
+}
+
+struct CountArgs {
+    int64_t m, n, nnz;
+    int64_t panel_rows, panels, tile_rows, tiles, groups;
+    const void* rp;
+    const void* ci;
+    const void* vals;
+    uint32_t* cnt;   // [panel][tile][column]
+    uint32_t* gcnt;  // [panel][group][column]
+    void* ptr_t;
+    void* idx_t;
+    void* vals_t;
+};
+
+// The block's tile: entries [k0, k1), rows [r0, r1) of panel p.
+struct CountTile {
+    int64_t g, p, t, r0, r1, k0, k1;
+};
+template <class I>
+__device__ __forceinline__ CountTile count_tile(const CountArgs& a) {
+    CountTile q;
+    // block ids go round-robin over the 8 XCDs: an XCD takes consecutive
+    // tiles, so the lines that neighbouring tiles share meet in its L2
+    const int64_t total = a.panels * a.tiles, per = (total + 7) / 8;
+    q.g = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    q.p = q.g / a.tiles;
+    q.t = q.g - q.p * a.tiles;
+    if (q.g >= total) {
+        q.r0 = q.r1 = q.k0 = q.k1 = 0;
+        return q;
+    }
+    const int64_t pend = min(a.m, (q.p + 1) * a.panel_rows);
+    q.r0 = min(q.p * a.panel_rows + q.t * a.tile_rows, pend);
+    q.r1 = min(q.r0 + a.tile_rows, pend);
+    const I* rp = static_cast<const I*>(a.rp);
+    q.k0 = clamp_ptr(rp[q.r0], a.nnz);
+    q.k1 = max(q.k0, clamp_ptr(rp[q.r1], a.nnz));
+    return q;
+}
+
+template <class I>
+__global__ __launch_bounds__(256) void csr_count_kernel(CountArgs a) {
+    __shared__ uint32_t h[kCountCols];
+    for (int64_t c = threadIdx.x; c < a.n; c += 256) h[c] = 0;
+    __syncthreads();
+    const CountTile q = count_tile<I>(a);
+    const I* ci = static_cast<const I*>(a.ci);
+    const uint64_t n = static_cast<uint64_t>(a.n);
+    for (int64_t k = q.k0 + threadIdx.x; k < q.k1; k += 8 * 256) {
+        uint64_t c[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) c[u] = k + u * 256 < q.k1 ? static_cast<uint64_t>(ci[k + u * 256]) : n;
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (c[u] < n) atomicAdd(&h[c[u]], 1u);
+    }
+    __syncthreads();
+    if (q.g >= a.panels * a.tiles) return;
+    uint32_t* out = a.cnt + q.g * a.n;
+    for (int64_t c = threadIdx.x; c < a.n; c += 256) out[c] = h[c];
+}
+
+// Exclusive sums of each column's counts over the tiles of a group, in place;
+// the group's total per column.  grid = (columns / 256, panels * groups).
+__global__ __launch_bounds__(256) void csr_count_scan_kernel(CountArgs a) {
+    const int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (c >= a.n) return;
+    for (int64_t pg = blockIdx.y; pg < a.panels * a.groups; pg += gridDim.y) {
+        const int64_t p = pg / a.groups, g = pg - p * a.groups;
+        const int64_t t0 = g * kGroupTiles, t1 = min(a.tiles, t0 + kGroupTiles);
+        uint32_t* col = a.cnt + p * a.tiles * a.n + c;
+        uint32_t run = 0;
+        for (int64_t t = t0; t < t1; t += 16) {
+            uint32_t v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = t + u < t1 ? col[(t + u) * a.n] : 0u;
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                if (t + u < t1) {
+                    col[(t + u) * a.n] = run;
+                    run += v[u];
+                }
+        }
+        a.gcnt[pg * a.n + c] = run;
+    }
+}
+
+// Per panel: exclusive sums over its groups (in place) and over its columns,
+// starting at the panel's first entry: the blocked transpose's row starts.
+template <class I>
+__global__ __launch_bounds__(1024) void csr_count_ptr_kernel(CountArgs a) {
+    __shared__ uint32_t part[16];
+    const int64_t p = blockIdx.x;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const I* rp = static_cast<const I*>(a.rp);
+    I* ptr = static_cast<I*>(a.ptr_t) + p * a.n;
+    int64_t base = a.m > 0 ? clamp_ptr(rp[p * a.panel_rows], a.nnz) : 0;
+    for (int64_t c0 = 0; c0 < a.n; c0 += 1024) {
+        const int64_t c = c0 + threadIdx.x;
+        uint32_t tot = 0;
+        if (c < a.n) {
+            uint32_t* col = a.gcnt + p * a.groups * a.n + c;
+            for (int64_t g = 0; g < a.groups; g += 8) {
+                uint32_t v[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) v[u] = g + u < a.groups ? col[(g + u) * a.n] : 0u;
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (g + u < a.groups) {
+                        col[(g + u) * a.n] = tot;
+                        tot += v[u];
+                    }
+            }
+        }
+        uint32_t inc = tot;  // inclusive over the wavefront, then over the block's wavefronts
+        for (int o = 1; o < 64; o *= 2) {
+            const uint32_t up = __shfl_up(inc, o);
+            if (lane >= o) inc += up;
+        }
+        if (lane == 63) part[wave] = inc;
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+        for (int w = 0; w < 16; ++w) {
+            before += w < wave ? part[w] : 0u;
+            all += part[w];
+        }
+        if (c < a.n) ptr[c] = static_cast<I>(base + before + inc - tot);
+        base += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && p == a.panels - 1) ptr[a.n] = static_cast<I>(base);
+}
+
+// LDS of the sorting kernel: W wavefronts' 16-bit column counters, two words
+// per column, the tile's row starts, and a chunk of sorted entries.
+template <class V, int W, int Q>
+size_t count_lds_bytes(int64_t n) {
+    return static_cast<size_t>(W * n * 2 + 2 * n * 4 + (kTileRows + 1) * 4 + 64 * W * Q * (4 + static_cast<int64_t>(sizeof(V)))) + 16;
+}
+
+// n <= 2^BITS.  W wavefronts of Q entries a lane sort a chunk of 64 W Q entries at a time
+// (a tile is one chunk unless its rows are much longer than the mean).
+template <class V, class I, int W, int Q, int BITS>
+__global__ __launch_bounds__(64 * W) void csr_count_sort_kernel(CountArgs a) {
+    extern __shared__ __attribute__((aligned(16))) char count_lds[];
+    constexpr uint32_t E = 64 * W * Q;
+    const uint32_t n = static_cast<uint32_t>(a.n);
+    V* sval = reinterpret_cast<V*>(count_lds);
+    uint32_t* base = reinterpret_cast<uint32_t*>(sval + E);  // next position of each column
+    uint32_t* off = base + n;                                // position - place in the chunk
+    uint32_t* start = off + n;                               // the tile's row starts, relative to k0
+    uint16_t* srow = reinterpret_cast<uint16_t*>(start + kTileRows + 1);
+    uint16_t* scol = srow + E;
+    uint16_t* hist = scol + E;  // [W][n]
+    __shared__ uint32_t part[W];
+    const CountTile q = count_tile<I>(a);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const uint32_t len = static_cast<uint32_t>(q.k1 - q.k0), rows = static_cast<uint32_t>(q.r1 - q.r0);
+    if (len == 0) return;
+    {
+        const I* ptr = static_cast<const I*>(a.ptr_t) + q.p * a.n;
+        const uint32_t* cnt = a.cnt + q.g * a.n;
+        const uint32_t* gc = a.gcnt + (q.p * a.groups + q.t / kGroupTiles) * a.n;
+        for (uint32_t c = tid; c < n; c += 64 * W) base[c] = static_cast<uint32_t>(ptr[c]) + gc[c] + cnt[c];
+        const I* rp = static_cast<const I*>(a.rp);
+        for (uint32_t r = tid; r <= rows; r += 64 * W)
+            start[r] = static_cast<uint32_t>(clamp_ptr(rp[q.r0 + r], a.nnz) - q.k0);
+    }
+    const I* ci = static_cast<const I*>(a.ci) + q.k0;
+    const V* vals = static_cast<const V*>(a.vals) + q.k0;
+    uint16_t* h = hist + wave * n;
+    for (uint32_t e0 = 0; e0 < len; e0 += E) {
+        uint32_t c[Q], at[Q];
+        V v[Q];
+        const uint32_t first = e0 + wave * 64 * Q + lane;
+#pragma unroll
+        for (int u = 0; u < Q; ++u) {
+            const uint32_t e = first + u * 64;
+            c[u] = e < len ? static_cast<uint32_t>(ci[e]) : n;
+            if (e < len) v[u] = vals[e];
+        }
+        for (uint32_t i = lane; i < n; i += 64) h[i] = 0;
+        __syncthreads();  // row starts; the last chunk's entries are out of LDS
+        // rank of every entry among its wavefront's entries of the same column
+#pragma unroll
+        for (int u = 0; u < Q; ++u) {
+            const bool in = c[u] < n;
+            uint64_t same = __ballot(in);
+#pragma unroll
+            for (int b = 0; b < BITS; ++b) {
+                const bool bit = (c[u] >> b) & 1u;
+                const uint64_t set = __ballot(bit);
+                same &= bit ? set : ~set;
+            }
+            at[u] = 0;
+            if (in) {
+                const uint32_t rank = __builtin_amdgcn_mbcnt_hi(
+                    static_cast<uint32_t>(same >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(same), 0u));
+                at[u] = __hip_atomic_load(&h[c[u]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) + rank;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // every lane has read before one writes
+                if (rank + 1 == static_cast<uint32_t>(__popcll(same)))
+                    __hip_atomic_store(&h[c[u]], static_cast<uint16_t>(at[u] + 1), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_WORKGROUP);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // and has written before the next step reads
+        }
+        __syncthreads();
+        // places in the chunk: by column, then wavefront
+        uint32_t carry = 0;
+        for (uint32_t c0 = 0; c0 < n; c0 += 64 * W) {
+            const uint32_t col = c0 + tid;
+            uint32_t tot = 0;
+            if (col < n)
+#pragma unroll
+                for (int w = 0; w < W; ++w) tot += hist[w * n + col];
+            uint32_t inc = tot;
+            for (int o = 1; o < 64; o *= 2) {
+                const uint32_t up = __shfl_up(inc, o);
+                if (lane >= o) inc += up;
+            }
+            if (lane == 63) part[wave] = inc;
+            __syncthreads();
+            uint32_t before = carry;
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                before += w < wave ? part[w] : 0u;
+                carry += part[w];
+            }
+            if (col < n) {
+                uint32_t s = before + inc - tot;
+                off[col] = base[col] - s;
+                base[col] += tot;
+#pragma unroll
+                for (int w = 0; w < W; ++w) {
+                    const uint32_t t = hist[w * n + col];
+                    hist[w * n + col] = static_cast<uint16_t>(s);
+                    s += t;
+                }
+            }
+            __syncthreads();
+        }
+        uint32_t r = 0;  // row of the lane's first entry: the last start at or before it
+        for (uint32_t w = kTileRows; w; w >>= 1)
+            if (r + w < rows && start[r + w] <= first) r += w;
+#pragma unroll
+        for (int u = 0; u < Q; ++u) {
+            const uint32_t e = first + u * 64;
+            while (e < len && r + 1 < rows && start[r + 1] <= e) ++r;
+            if (c[u] < n) {
+                const uint32_t i = h[c[u]] + at[u];
+                sval[i] = v[u];
+                srow[i] = static_cast<uint16_t>(r);
+                scol[i] = static_cast<uint16_t>(c[u]);
+            }
+        }
+        __syncthreads();
+        I* idx = static_cast<I*>(a.idx_t);
+        V* out = static_cast<V*>(a.vals_t);
+        for (uint32_t i = tid; i < carry; i += 64 * W) {
+            const uint32_t pos = off[scol[i]] + i;
+            idx[pos] = static_cast<I>(q.r0 + srow[i]);
+            out[pos] = sval[i];
+        }
+    }
+}
+
+template <class I>
+void transpose_count(const CsrMat& A, int64_t panel_rows, void* vals_t, void* ptr_t, void* idx_t, void* scratch,
+                     hipStream_t s) {
+    const CountPlan p = count_plan(A, panel_rows);
+    CountArgs a{A.m, A.n, A.nnz, panel_rows, p.panels, p.tile_rows, p.tiles, p.groups, A.row_ptrs, A.col_idxs, A.vals,
+                static_cast<uint32_t*>(scratch), nullptr, ptr_t, idx_t, vals_t};
+    a.gcnt = reinterpret_cast<uint32_t*>(static_cast<char*>(scratch) +
+                                         align256(static_cast<size_t>(p.panels * p.tiles * A.n) * 4));
+    if (A.m == 0) {
+        TOMOS_HIP_CHECK(hipMemsetAsync(ptr_t, 0, static_cast<size_t>(A.n + 1) * sizeof(I), s));
+        return;
+    }
+    const int64_t blocks = ceil_div(p.panels * p.tiles, 8) * 8;
+    require(blocks < (int64_t(1) << 31), "CSR transpose: too many tiles");
+    csr_count_kernel<I><<<static_cast<unsigned>(blocks), 256, 0, s>>>(a);
+    TOMOS_LAUNCH_CHECK("csr_count_kernel");
+    csr_count_scan_kernel<<<dim3(static_cast<unsigned>(ceil_div(A.n, 256)),
+                                 static_cast<unsigned>(std::min<int64_t>(p.panels * p.groups, 65535))),
+                            256, 0, s>>>(a);
+    TOMOS_LAUNCH_CHECK("csr_count_scan_kernel");
+    csr_count_ptr_kernel<I><<<static_cast<unsigned>(p.panels), 1024, 0, s>>>(a);
+    TOMOS_LAUNCH_CHECK("csr_count_ptr_kernel");
+    if (A.nnz == 0) return;
+    auto launch = [&](auto* k, int threads, size_t lds) {
+        TOMOS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k),
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
+        k<<<static_cast<unsigned>(blocks), threads, lds, s>>>(a);
+    };
+#define TOMOS_COUNT_SORT(V, Q)                                                                   \
+    do {                                                                                         \
+        if (A.n <= 256) launch(csr_count_sort_kernel<V, I, 8, Q, 8>, 512, count_lds_bytes<V, 8, Q>(A.n));  \
+        else if (A.n <= 1024) launch(csr_count_sort_kernel<V, I, 8, Q, 10>, 512, count_lds_bytes<V, 8, Q>(A.n)); \
+        else launch(csr_count_sort_kernel<V, I, 8, Q, 11>, 512, count_lds_bytes<V, 8, Q>(A.n));      \
+    } while (0)
+    switch (csr_value_bytes(A.val_type)) {
+        case 8: TOMOS_COUNT_SORT(uint64_t, 8); break;
+        case 4: TOMOS_COUNT_SORT(uint32_t, 12); break;
+        default: TOMOS_COUNT_SORT(uint16_t, 12); break;
+    }
+#undef TOMOS_COUNT_SORT
+    TOMOS_LAUNCH_CHECK("csr_count_sort_kernel");
+}
+
 }  // namespace
 
 size_t csr_value_bytes(int t) { return t == TOMOS_F64 ? 8 : t == TOMOS_F32 ? 4 : 2; }
@@ -713,6 +1105,7 @@ int64_t csr_panel_rows(const CsrMat& A, int x_type) {
 int64_t csr_panels(const CsrMat& A, int64_t panel_rows) { return A.m > 0 ? ceil_div(A.m, panel_rows) : 1; }
 
 size_t csr_transpose_scratch_bytes(const CsrMat& A, int64_t panel_rows) {
+    if (count_transpose(A)) return count_bytes(A, panel_rows);
     const int64_t nkeys = csr_panels(A, panel_rows) * A.n;
     if (packed_sort(A)) return transpose_bytes_packed(A.nnz, nkeys);
     return A.idx_type == TOMOS_INDEX_INT64 ? transpose_bytes<uint64_t>(A.nnz, nkeys)
@@ -724,6 +1117,11 @@ void csr_transpose(const CsrMat& A, int64_t panel_rows, void* vals_t, void* ptr_
     require(panel_rows >= 1, "csr_transpose: bad panel size");
     require(scratch_bytes >= csr_transpose_scratch_bytes(A, panel_rows), "csr_transpose: scratch too small");
     require(ptr_t != nullptr && ((vals_t && idx_t) || A.nnz == 0), "csr_transpose: null output");
+    if (count_transpose(A)) {
+        if (A.idx_type == TOMOS_INDEX_INT64) transpose_count<int64_t>(A, panel_rows, vals_t, ptr_t, idx_t, scratch, s);
+        else transpose_count<int32_t>(A, panel_rows, vals_t, ptr_t, idx_t, scratch, s);
+        return;
+    }
     // the index buffers hold non-negative values: sorted as unsigned
     if (packed_sort(A)) transpose_packed(A, panel_rows, vals_t, ptr_t, idx_t, scratch, s);
     else if (A.idx_type == TOMOS_INDEX_INT64) transpose_impl<uint64_t>(A, panel_rows, vals_t, ptr_t, idx_t, scratch, s);
