@@ -154,3 +154,26 @@ def test_tier_errors(capi):
                a.ptr, 4, None)
     with pytest.raises(C.TomosError):  # no such tier
         C.call("tomos_gemm", C.FP32_BF16, 7, 0, 0, 1.0, 4, 4, 4, a.ptr, a.ptr, 4, a.ptr, 4, 0.0, a.ptr, 4, None)
+
+
+@pytest.mark.parametrize("a_type,variant,dec_hi,dec_ex", FORMATS)
+@pytest.mark.parametrize("ta,tb", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (128, 128, 64), (129, 127, 65), (256, 130, 63), (255, 33, 1100),
+                                   (100, 100, 520), (100, 100, 4100), (3600, 3300, 72)])
+def test_tile_and_split_edges(capi, orc, a_type, variant, dec_hi, dec_ex, ta, tb, shape):
+    """Both MFMA tiers at the edges of the C tiles (128 and, from 192 tiles,
+    256 wide), of the K slices (32 / 64) and of the K splits, odd leading
+    dimensions, beta != 0.  Integers up to 15 (8 significant bits hold them in
+    every plane, K * 225 < 2^24): every product and FP32 sum is exact, so the
+    result is the FP64 one rounded once."""
+    M, N, K = shape
+    rng = np.random.default_rng(M + 2 * N + 3 * K)
+    A, B, C0 = (np.asfortranarray(np.rint(np.clip(5 * X, -15, 15))) for X in operands(rng, M, N, K, ta, tb, 1))
+    Av, Bv = views(A, B, M, N, K, ta, tb)
+    ref = 2.0 * (Av @ Bv) - 3.0 * C0[:M].astype(np.float64)
+    wh, wr = H.pack(variant, A)
+    for tier in (C.TIER_DEFAULT, C.TIER_MATERIALIZE):
+        print("tiles", a_type, ta, tb, shape, tier, flush=True)
+        got = gemm(a_type, tier, ta, tb, 2.0, M, N, K, wh, wr, A.shape[0], B, B.shape[0], -3.0, C0, M + 1)
+        assert np.array_equal(got[:M], ref.astype(np.float32)), np.abs(got[:M] - ref).max()
+        assert np.array_equal(got[M:], C0[M:])

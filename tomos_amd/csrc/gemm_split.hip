@@ -18,11 +18,14 @@
 //     2^s per operand, chosen from the operand's largest magnitude, so the hi
 //     and lo terms stay clear of fp16 overflow and underflow (C is rescaled
 //     by 2^-(sA+sB) in the epilogue); FP32_BF16 uses bf16 planes.
-//  2. gemm: 512 threads, 256 x 256 C tile, K slice of 32 staged through LDS
-//     (rows padded against bank conflicts); each wave owns 128 x 64 = 4 x 2
-//     MFMA 32x32x16 tiles and issues 1 (hi-only) or 3 (split) MFMAs per
-//     tile per 16-wide k step into one FP32 accumulator.
+//     The planes are stored as the LDS images the GEMM reads: blocks of 128
+//     rows x 32 k, so a K slice of a tile is one contiguous run per operand.
+//  2. gemm: 256 x 256 (or 128 x 128) C tiles, K slices through two LDS
+//     stages by DMA, 1 (hi-only) or 3 (split) MFMA 32x32x16 per tile and
+//     16-wide k step into one FP32 accumulator; splits of K where the tiles
+//     leave the chip idle.
 #include <algorithm>
+#include <type_traits>
 
 #include "codec.hpp"
 #include "common.hpp"
@@ -36,10 +39,20 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
-constexpr int BM = 256, BN = 256, BK = 32;
-constexpr int LDK = BK + 8;  // padded K stride (elements) of an LDS row
-constexpr int kGemmThreads = 512;                     // 8 waves: 2 (M) x 4 (N)
-constexpr int kPlaneElems = BM * LDK;                 // one plane's K slice in LDS (BM == BN)
+constexpr int kPadRows = 256;   // operand rows are padded to the larger tile
+constexpr int kBlockRows = 128, kBlockK = 32;
+constexpr int kBlockElems = kBlockRows * kBlockK;  // one plane's block: 8 KB
+
+// Element offset of the 8-element chunk (row r, k .. k+7) of a staged
+// operand of nk slices.  A slice holds two blocks of every 128-row group, one
+// after the other: the hi and the lo plane of 32 k (TERMS == 3), or the hi
+// plane of two times 32 k (TERMS == 1, `second` = k / 32 % 2).  Inside a block
+// a row is 64 bytes; its four 16-byte chunks are permuted by the row so that
+// the 16 lanes that a 16-byte LDS read serves together touch all banks.
+__host__ __device__ __forceinline__ int64_t chunk_offset(int64_t r, int64_t slice, int second, int64_t nk, int c) {
+    const int row = static_cast<int>(r % kBlockRows);
+    return ((r / kBlockRows * nk + slice) * 2 + second) * kBlockElems + row * kBlockK + ((c ^ ((row >> 2) & 3)) * 8);
+}
 
 // ---------------------------------------------------------------- operands
 // A GEMM operand as the prep kernels read it: X column-major with leading
@@ -57,11 +70,6 @@ __device__ __forceinline__ float decode_exact(int fmt, uint32_t h, uint32_t r) {
     return fmt == TOMOS_FP32_16 ? codec::fp32_16_decode_exact(h, r) : __uint_as_float((h << 16) | r);
 }
 
-// exact value of element idx (split mode)
-__device__ __forceinline__ float src_value(const Src& s, int64_t idx) {
-    return s.f ? s.f[idx] : decode_exact(s.fmt, s.wh[idx], s.wr[idx]);
-}
-
 __device__ __forceinline__ uint16_t bf16_rn(float v) {
     return static_cast<uint16_t>(codec::f32_to_bf16_bits(v));
 }
@@ -69,31 +77,6 @@ __device__ __forceinline__ uint16_t f16_rn(float v) {
     return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
 }
 __device__ __forceinline__ float bf16_val(uint16_t b) { return __uint_as_float(static_cast<uint32_t>(b) << 16); }
-
-// 16-bit MFMA operand bits of element idx (hi-only mode): the packed hi word
-// decoded as the reference's 16-bit tiers read it (FP32_BF16: wh is the
-// bf16 value, fp32_bf16_bf16_only; FP32_16: fp32_16_half_only), or an FP32
-// value rounded to nearest-even bf16 / fp16.
-__device__ __forceinline__ uint16_t src_hi_bits(const Src& s, int64_t idx, bool f16) {
-    if (s.f) return f16 ? f16_rn(s.f[idx]) : bf16_rn(s.f[idx]);
-    const uint32_t h = s.wh[idx];
-    return static_cast<uint16_t>(s.fmt == TOMOS_FP32_16 ? codec::fp32_16_half_bits(h) : h);
-}
-
-// max |x| over an operand (exact values), for the fp16 split scale
-__global__ __launch_bounds__(256) void absmax_kernel(Src s, int64_t rows, int64_t cols,
-                                                     unsigned* __restrict__ out_bits) {
-    float mx = 0.0f;
-    const int64_t total = rows * cols;
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; t < total;
-         t += static_cast<int64_t>(gridDim.x) * 256) {
-        const int64_t j = t / rows, i = t - j * rows;
-        const float v = fabsf(src_value(s, i + j * s.ld));
-        if (v <= 3.0e38f) mx = fmaxf(mx, v);  // ignore Inf/NaN
-    }
-    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
-    if ((threadIdx.x & 63) == 0) atomicMax(out_bits, __float_as_uint(mx));
-}
 
 __device__ __forceinline__ int fp16_scale_exp(bool f16, const unsigned* absmax_bits) {
     // power-of-two scale bringing max |x| to about 2^13 (fp16 max is 65504)
@@ -119,137 +102,170 @@ __device__ __forceinline__ void split16(bool f16, float v, int sc, uint16_t& h16
 
 enum { PREP_HI = 1, PREP_SPLIT = 3 };
 
-// hi (and, for PREP_SPLIT, lo) 16-bit bits of element idx
-template <int MODE>
-__device__ __forceinline__ void prep_elem(const Src& s, int64_t idx, bool valid, bool f16, int sc,
-                                          uint16_t& h16, uint16_t& l16) {
-    if constexpr (MODE == PREP_HI) {
-        h16 = valid ? src_hi_bits(s, idx, f16) : uint16_t(0);
-        l16 = 0;
-    } else {
-        split16(f16, valid ? src_value(s, idx) : 0.0f, sc, h16, l16);
-    }
-}
+typedef u32x4 u32x4_u __attribute__((aligned(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4_u __attribute__((aligned(4)));
 
-// K-contiguous operand (X is K x R column-major): out[r][k] = X(k, r) for
-// r < pad_r, k < pad_k, zero outside X.  hi (and lo) planes have row
-// stride out_ld.
-template <int MODE>
-__global__ __launch_bounds__(256) void prep_k_kernel(Src s, int64_t rows, int64_t cols, int64_t out_ld,
-                                                     uint16_t* __restrict__ hi, uint16_t* __restrict__ lo,
-                                                     const unsigned* __restrict__ absmax_bits, bool f16,
-                                                     int64_t pad_r, int64_t pad_k) {
-    const int sc = MODE == PREP_SPLIT ? fp16_scale_exp(f16, absmax_bits) : 0;
-    const int64_t total = pad_r * pad_k;
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; t < total;
-         t += static_cast<int64_t>(gridDim.x) * 256) {
-        const int64_t r = t / pad_k, k = t - r * pad_k;
-        uint16_t h16, l16;
-        prep_elem<MODE>(s, k + r * s.ld, k < rows && r < cols, f16, sc, h16, l16);
-        hi[r * out_ld + k] = h16;
-        if constexpr (MODE == PREP_SPLIT) lo[r * out_ld + k] = l16;
-    }
-}
-
-// Vector form of prep_k_kernel for operands whose columns are whole 16-byte
-// runs of 16-bit words (rows % 8 == 0, ld % 8 == 0, 16-byte aligned planes)
-// or 32-byte runs of FP32: 8 elements per thread, 16-byte stores.
-template <int MODE>
-__global__ __launch_bounds__(256) void prep_k_vec_kernel(Src s, int64_t rows, int64_t cols, int64_t out_ld,
-                                                         uint16_t* __restrict__ hi, uint16_t* __restrict__ lo,
-                                                         const unsigned* __restrict__ absmax_bits, bool f16,
-                                                         int64_t pad_r, int64_t pad_k) {
-    const int sc = MODE == PREP_SPLIT ? fp16_scale_exp(f16, absmax_bits) : 0;
-    const int64_t cpr = pad_k / 8, total = pad_r * cpr;
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; t < total;
-         t += static_cast<int64_t>(gridDim.x) * 256) {
-        const int64_t r = t / cpr, k = (t - r * cpr) * 8;  // out[r][k..k+7] = X(k..k+7, r)
-        const bool valid = k < rows && r < cols;
-        const int64_t base = k + r * s.ld;
-        uint16_t h[8], l[8];
-        if (s.f) {
-            float v[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-            if (valid) {
-                const float4 v0 = *reinterpret_cast<const float4*>(s.f + base);
-                const float4 v1 = *reinterpret_cast<const float4*>(s.f + base + 4);
-                v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
-                v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
-            }
+// The words of elements idx .. idx+7 of a packed plane, of which the first
+// `count` exist (the others are zero words): one 16-byte load at element
+// alignment for a whole run.
+__device__ __forceinline__ u32x4 words8(const uint16_t* __restrict__ p, int64_t idx, int64_t count) {
+    if (count >= 8) return *reinterpret_cast<const u32x4_u*>(p + idx);
+    u32x4 w = {0u, 0u, 0u, 0u};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if constexpr (MODE == PREP_HI) {
-                    h[e] = f16 ? f16_rn(v[e]) : bf16_rn(v[e]);
-                    l[e] = 0;
-                } else {
-                    split16(f16, v[e], sc, h[e], l[e]);
-                }
-            }
+    for (int e = 0; e < 7; ++e)
+        if (e < count) w[e / 2] |= static_cast<uint32_t>(p[idx + e]) << (16 * (e & 1));
+    return w;
+}
+
+// Exact values of elements idx .. idx+7, zero beyond `count`.
+__device__ __forceinline__ void values8(const Src& s, int64_t idx, int64_t count, float (&v)[8]) {
+    if (s.f) {
+        if (count >= 8) {
+            const f32x4 v0 = *reinterpret_cast<const f32x4_u*>(s.f + idx);
+            const f32x4 v1 = *reinterpret_cast<const f32x4_u*>(s.f + idx + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { v[e] = v0[e]; v[4 + e] = v1[e]; }
         } else {
-            u32x4 wh8 = {0u, 0u, 0u, 0u}, wr8 = {0u, 0u, 0u, 0u};
-            if (valid) {
-                wh8 = *reinterpret_cast<const u32x4*>(s.wh + base);
-                if constexpr (MODE == PREP_SPLIT) wr8 = *reinterpret_cast<const u32x4*>(s.wr + base);
-            }
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int b = 0; b < 2; ++b) {
-                    const uint32_t hw = b ? (wh8[q] >> 16) : (wh8[q] & 0xFFFFu);
-                    const int e = 2 * q + b;
-                    if constexpr (MODE == PREP_HI) {
-                        h[e] = valid ? static_cast<uint16_t>(s.fmt == TOMOS_FP32_16 ? codec::fp32_16_half_bits(hw)
-                                                                                    : hw)
-                                     : uint16_t(0);
-                        l[e] = 0;
-                    } else {
-                        const uint32_t rw = b ? (wr8[q] >> 16) : (wr8[q] & 0xFFFFu);
-                        split16(f16, valid ? decode_exact(s.fmt, hw, rw) : 0.0f, sc, h[e], l[e]);
-                    }
-                }
+            for (int e = 0; e < 8; ++e) v[e] = e < count ? s.f[idx + e] : 0.0f;
         }
-        u32x4 h8, l8;
+        return;
+    }
+    const u32x4 wh = words8(s.wh, idx, count), wr = words8(s.wr, idx, count);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int b = 16 * (e & 1);
+        const float x = decode_exact(s.fmt, (wh[e / 2] >> b) & 0xFFFFu, (wr[e / 2] >> b) & 0xFFFFu);
+        v[e] = e < count ? x : 0.0f;
+    }
+}
+
+// hi (and, for PREP_SPLIT, lo) bits of elements idx .. idx+7, zero beyond `count`.
+template <int MODE>
+__device__ __forceinline__ void prep8(const Src& s, int64_t idx, int64_t count, bool f16, int sc, uint16_t (&h)[8],
+                                      uint16_t (&l)[8]) {
+    if (MODE == PREP_HI && !s.f) {
+        const u32x4 wh = words8(s.wh, idx, count);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            h8[q] = static_cast<uint32_t>(h[2 * q]) | (static_cast<uint32_t>(h[2 * q + 1]) << 16);
-            l8[q] = static_cast<uint32_t>(l[2 * q]) | (static_cast<uint32_t>(l[2 * q + 1]) << 16);
+            // zero words stay zero in both formats' hi decode
+            const uint32_t hb = s.fmt == TOMOS_FP32_16 ? codec::fp32_16_half_bits2(wh[q]) : wh[q];
+            h[2 * q] = static_cast<uint16_t>(hb);
+            h[2 * q + 1] = static_cast<uint16_t>(hb >> 16);
         }
-        *reinterpret_cast<u32x4*>(hi + r * out_ld + k) = h8;
-        if constexpr (MODE == PREP_SPLIT) *reinterpret_cast<u32x4*>(lo + r * out_ld + k) = l8;
+        return;
+    }
+    float v[8];
+    values8(s, idx, count, v);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        if constexpr (MODE == PREP_HI) h[e] = f16 ? f16_rn(v[e]) : bf16_rn(v[e]);
+        else split16(f16, v[e], sc, h[e], l[e]);
     }
 }
 
-// R-contiguous operand (X is R x K column-major): out[r][k] = X(r, k) needs
-// a transpose, done per 64 x 64 tile through LDS so both the reads (r
-// fastest) and the writes (k fastest) are contiguous.
-// grid = (ceil(pad_k/64), ceil(pad_r/64)).
+__global__ void absmax_clear_kernel(unsigned* out) { out[threadIdx.x] = 0; }
+
+// max |x| over an operand (exact values), for the fp16 split scale: runs of 8
+// rows a thread, columns strided over blockIdx.y.
+__global__ __launch_bounds__(256) void absmax_kernel(Src s, int64_t rows, int64_t cols,
+                                                     unsigned* __restrict__ out_bits) {
+    float mx = 0.0f;
+    const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 8;
+    if (i < rows)
+        for (int64_t j = blockIdx.y; j < cols; j += gridDim.y) {
+            float v[8];
+            values8(s, i + j * s.ld, rows - i, v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float a = fabsf(v[e]);
+                if (a <= 3.0e38f) mx = fmaxf(mx, a);  // ignore Inf/NaN
+            }
+        }
+    for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    if ((threadIdx.x & 63) == 0) atomicMax(out_bits, __float_as_uint(mx));
+}
+
+__device__ __forceinline__ u32x4 pack8(const uint16_t (&h)[8]) {
+    u32x4 v;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = static_cast<uint32_t>(h[2 * q]) | (static_cast<uint32_t>(h[2 * q + 1]) << 16);
+    return v;
+}
+
+// Stores the chunk of k .. k+7 (k a multiple of 8) of row r.
 template <int MODE>
-__global__ __launch_bounds__(256) void prep_t_kernel(Src s, int64_t rows, int64_t cols, int64_t out_ld,
-                                                     uint16_t* __restrict__ hi, uint16_t* __restrict__ lo,
-                                                     const unsigned* __restrict__ absmax_bits, bool f16,
-                                                     int64_t pad_r, int64_t pad_k) {
-    __shared__ uint16_t th[64][65];
-    __shared__ uint16_t tl[64][65];
+__device__ __forceinline__ void store_chunk(uint16_t* __restrict__ out, int64_t r, int64_t k, int64_t nk, u32x4 h,
+                                            u32x4 l) {
+    const int c = static_cast<int>(k % kBlockK) / 8;
+    if constexpr (MODE == PREP_HI) {
+        const int second = static_cast<int>(k / kBlockK % 2);
+        *reinterpret_cast<u32x4*>(out + chunk_offset(r, k / (2 * kBlockK), second, nk, c)) = h;
+    } else {
+        *reinterpret_cast<u32x4*>(out + chunk_offset(r, k / kBlockK, 0, nk, c)) = h;
+        *reinterpret_cast<u32x4*>(out + chunk_offset(r, k / kBlockK, 1, nk, c)) = l;
+    }
+}
+
+// K-contiguous operand (X is K x R column-major): row r of the operand is
+// X's column r.  A block takes 32 rows x 64 k: 128 contiguous bytes (or more)
+// of every column in, 64-byte rows out.  grid = (ceil(Kp / 64), pad_r / 32).
+template <int MODE>
+__global__ __launch_bounds__(256) void prep_k_kernel(Src s, int64_t rows, int64_t cols, int64_t pad_r, int64_t nk,
+                                                     int64_t Kp, uint16_t* __restrict__ out,
+                                                     const unsigned* __restrict__ absmax_bits, bool f16) {
+    const int sc = MODE == PREP_SPLIT ? fp16_scale_exp(f16, absmax_bits) : 0;
+    const int64_t k = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x % 8 * 8;
+    if (k >= Kp) return;
+    for (int64_t r = static_cast<int64_t>(blockIdx.y) * 32 + threadIdx.x / 8; r < pad_r;
+         r += static_cast<int64_t>(gridDim.y) * 32) {
+        uint16_t h[8], l[8];
+        prep8<MODE>(s, k + r * s.ld, r < cols ? rows - k : 0, f16, sc, h, l);
+        store_chunk<MODE>(out, r, k, nk, pack8(h), pack8(l));
+    }
+}
+
+// R-contiguous operand (X is R x K column-major): row r of the operand is
+// X's row r, so 64 x 64 tiles are transposed through LDS.  A thread loads 8
+// rows of two adjacent columns and writes their pairs as 32-bit words; rows
+// of 33 words spread both the writes and the reads over the banks.
+// grid = (ceil(Kp / 64), pad_r / 64).
+template <int MODE>
+__global__ __launch_bounds__(256) void prep_t_kernel(Src s, int64_t rows, int64_t cols, int64_t nk, int64_t Kp,
+                                                     uint16_t* __restrict__ out,
+                                                     const unsigned* __restrict__ absmax_bits, bool f16) {
+    constexpr int kPlanes = MODE == PREP_SPLIT ? 2 : 1;
+    __shared__ uint32_t tile[kPlanes][64][33];  // [row][k pair]
     const int sc = MODE == PREP_SPLIT ? fp16_scale_exp(f16, absmax_bits) : 0;
     const int64_t k0 = static_cast<int64_t>(blockIdx.x) * 64, r0 = static_cast<int64_t>(blockIdx.y) * 64;
-    const int tid = threadIdx.x;
-#pragma unroll 4
-    for (int it = 0; it < 16; ++it) {
-        const int idx = tid + it * 256, i = idx & 63, j = idx >> 6;  // i: r, j: k
-        const int64_t r = r0 + i, k = k0 + j;
-        uint16_t h16, l16;
-        prep_elem<MODE>(s, r + k * s.ld, r < rows && k < cols, f16, sc, h16, l16);
-        th[j][i] = h16;
-        if constexpr (MODE == PREP_SPLIT) tl[j][i] = l16;
+    {
+        const int rv = threadIdx.x % 8 * 8, kp = threadIdx.x / 8;  // 8 rows, one k pair
+        uint16_t h[2][8], l[2][8];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int64_t k = k0 + 2 * kp + b;
+            prep8<MODE>(s, r0 + rv + k * s.ld, k < cols ? rows - (r0 + rv) : 0, f16, sc, h[b], l[b]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            tile[0][rv + e][kp] = static_cast<uint32_t>(h[0][e]) | (static_cast<uint32_t>(h[1][e]) << 16);
+            if constexpr (MODE == PREP_SPLIT)
+                tile[kPlanes - 1][rv + e][kp] = static_cast<uint32_t>(l[0][e]) | (static_cast<uint32_t>(l[1][e]) << 16);
+        }
     }
     __syncthreads();
-#pragma unroll 4
-    for (int it = 0; it < 16; ++it) {
-        const int idx = tid + it * 256, j = idx & 63, i = idx >> 6;  // j: k, i: r
-        const int64_t r = r0 + i, k = k0 + j;
-        if (r < pad_r && k < pad_k) {
-            hi[r * out_ld + k] = th[j][i];
-            if constexpr (MODE == PREP_SPLIT) lo[r * out_ld + k] = tl[j][i];
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const int idx = threadIdx.x + it * 256, c = idx % 8, i = idx / 8;  // chunk of 8 k, row
+        if (k0 + 8 * c >= Kp) continue;
+        u32x4 h, l = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            h[q] = tile[0][i][4 * c + q];
+            if constexpr (MODE == PREP_SPLIT) l[q] = tile[kPlanes - 1][i][4 * c + q];
         }
+        store_chunk<MODE>(out, r0 + i, k0 + 8 * c, nk, h, l);
     }
 }
 
@@ -269,9 +285,8 @@ __device__ __forceinline__ void mfma32(const u32x4& a, const u32x4& b, f32x16& c
 // an XCD holds at once cover an 8 x 4 patch of C (8 A row panels and 4 B
 // column panels in that XCD's L2) instead of one whole tile column.
 constexpr int kGroupN = 4;
-__device__ __forceinline__ void tile_of(int64_t tiles_m, int64_t tiles_n, int64_t& tm, int64_t& tn) {
+__device__ __forceinline__ void tile_of(int64_t bid, int64_t tiles_m, int64_t tiles_n, int64_t& tm, int64_t& tn) {
     const int64_t nb = tiles_m * tiles_n;
-    int64_t bid = blockIdx.x;
     if (nb % 8 == 0) bid = (bid % 8) * (nb / 8) + bid / 8;
     const int64_t per_group = tiles_m * kGroupN;
     const int64_t g = bid / per_group, w = bid - g * per_group;
@@ -280,118 +295,151 @@ __device__ __forceinline__ void tile_of(int64_t tiles_m, int64_t tiles_n, int64_
     tm = w / gn;
 }
 
-// Ah/Al: [Mp][Kp], Bh/Bl: [Np][Kp] (K contiguous, padded to tile multiples).
-// NT threads = NT/64 waves as 2 (M) x WN (N); a wave owns 128 x (256/WN)
-// of the 256 x 256 C tile: 4 x TJ MFMA 32x32x16 tiles, 3 MFMAs (lo*hi,
-// hi*lo, hi*hi) per tile per 16-wide k step into one FP32 accumulator.  The
-// B fragment is the MFMA's first operand, so the accumulator is C^T per
-// tile and each lane holds C rows (lane % 32): the column-major stores of a
-// 32-lane half are 128 contiguous bytes.  The K slice (32) of all four
-// planes is staged through LDS (rows padded to 80 bytes: conflict-free
-// 16-byte fragment reads); the next slice is loaded into registers while
-// the current one is multiplied.
-template <bool F16, int NT, int TERMS>
-__global__ __launch_bounds__(NT) void gemm_mfma_kernel(
-    int64_t M, int64_t N, int64_t Kp, const uint16_t* __restrict__ Ah, const uint16_t* __restrict__ Al,
-    const uint16_t* __restrict__ Bh, const uint16_t* __restrict__ Bl, int64_t ldk, double alpha,
-    double beta, float* __restrict__ C, int64_t ldc, const unsigned* __restrict__ absA,
-    const unsigned* __restrict__ absB) {
-    constexpr int WN = NT / 128;      // waves along N
-    constexpr int TJ = 8 / WN;        // 32-wide n tiles per wave
-    constexpr int CH = 1024 / NT;     // 16-byte chunks per plane slice per thread
-    static_assert(TERMS == 1 || TERMS == 3, "hi-only or 3-term split");
-    extern __shared__ __attribute__((aligned(16))) uint16_t gemm_lds[];
-    uint16_t* sAh = gemm_lds;
-    uint16_t* sBh = sAh + kPlaneElems;
-    uint16_t* sAl = sBh + kPlaneElems;  // TERMS == 3 only
-    uint16_t* sBl = sAl + kPlaneElems;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    int64_t tm, tn;
-    tile_of((M + BM - 1) / BM, (N + BN - 1) / BN, tm, tn);
-    const int64_t m0 = tm * BM, n0 = tn * BN;
+// 16 bytes a lane from base + voff into LDS at lds + 16 * lane, without a
+// register in between.  As assembly, so that the compiler does not order
+// every later LDS read behind the DMA (it cannot tell the stages apart): the
+// kernel waits itself, with wait_stage().  No other instruction here uses M0.
+__device__ __forceinline__ void dma16(const void* base, uint32_t voff, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(base)
+                 : "memory");
+}
+// This wave's DMA but the last `LATER` has landed and its LDS reads have
+// returned; then all waves meet.
+template <int LATER>
+__device__ __forceinline__ void wait_stage() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LATER) : "memory");
+}
 
-    f32x16 acc[TJ][4];  // [n tile][m tile]
+// A, B: staged operands (chunk_offset).  WM x WN waves, a wave owns MT x NT
+// MFMA 32x32x16 tiles.  The B fragment is the MFMA's first operand, so the
+// accumulator is C^T per tile and each lane holds C rows (lane % 32): the
+// column-major stores of a 32-lane half are 128 contiguous bytes.
+//
+// A K slice (two blocks per 128 rows of A and B) goes to one of two LDS
+// stages by DMA; a slice is two phases, split by k (TERMS == 3: 16 k, hi and
+// lo; TERMS == 1: 32 k).  The second phase's fragments are read during the
+// first phase's MFMAs and the next slice's first phase during the second's;
+// the one barrier of a slice stands between the two, where this slice's
+// reads are done (its stage is refilled right away, one slice ahead) and the
+// next slice has landed.
+// Bound by the matrix pipes: 8192^3 split, bf16, 3.1 -> 2.33 ms (1.42 PFLOP/s
+// of MFMA work; a plain bf16 library product of that size runs at 1.15).
+// Before, the slices went through registers into padded LDS rows, between two
+// barriers a slice, and the tiles were 256 x 256 whatever their number.
+template <bool F16, int TERMS, int WM, int WN, int MT, int NT>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
+    int64_t M, int64_t N, int64_t nk, int64_t slices, const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
+    double alpha, double beta, float* __restrict__ C, int64_t ldc, const unsigned* __restrict__ absA,
+    const unsigned* __restrict__ absB, float* __restrict__ partial) {
+    static_assert(TERMS == 1 || TERMS == 3, "hi-only or 3-term split");
+    constexpr int BM = 32 * WM * MT, BN = 32 * WN * NT;
+    constexpr int kThreads = 64 * WM * WN;
+    constexpr int GA = BM / kBlockRows, GB = BN / kBlockRows;  // 128-row groups
+    constexpr uint32_t kGroup = 2 * kBlockElems * 2;           // bytes of a group's slice
+    constexpr uint32_t kStage = (GA + GB) * kGroup;
+    constexpr uint32_t kStep = kThreads * 16;                  // bytes per DMA of the block
+    constexpr int kLoads = kStage / kStep;                     // DMAs per thread and slice
+    extern __shared__ __attribute__((aligned(1024))) char gemm_lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave % WM, wn = wave / WM;
+    const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const int64_t split = blockIdx.x / (tiles_m * tiles_n);
+    int64_t tm, tn;
+    tile_of(blockIdx.x - split * tiles_m * tiles_n, tiles_m, tiles_n, tm, tn);
+    const int64_t m0 = tm * BM, n0 = tn * BN;
+    const int64_t s0 = split * slices, s1 = min(nk, s0 + slices);
+
+    f32x16 acc[NT][MT];
 #pragma unroll
-    for (int j = 0; j < TJ; ++j)
+    for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int v = 0; v < 16; ++v) acc[j][i][v] = 0.0f;
 
-    // loader: a plane slice is 256 rows x 32 k = 1024 16-byte chunks, CH per thread
-    int so[CH];
-    int64_t oa[CH], ob[CH];
+    const char* ga = reinterpret_cast<const char*>(A) + tm * GA * nk * kGroup;
+    const char* gb = reinterpret_cast<const char*>(B) + tn * GB * nk * kGroup;
+    const uint32_t lds0 = static_cast<uint32_t>(
+        reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) char*)gemm_lds));
+    const uint32_t voff = tid * 16, wave_lds = __builtin_amdgcn_readfirstlane(lds0 + wave * 1024);
+    auto load_slice = [&](int64_t s, uint32_t stage) {
 #pragma unroll
-    for (int q = 0; q < CH; ++q) {
-        const int ch = tid + q * NT, row = ch >> 2, kc = (ch & 3) * 8;
-        so[q] = row * LDK + kc;
-        oa[q] = (m0 + row) * ldk + kc;
-        ob[q] = (n0 + row) * ldk + kc;
+        for (int g = 0; g < GA; ++g)
+#pragma unroll
+            for (uint32_t x = 0; x < kGroup; x += kStep)
+                dma16(ga + (g * nk + s) * kGroup + x, voff, stage + g * kGroup + x + wave_lds);
+#pragma unroll
+        for (int g = 0; g < GB; ++g)
+#pragma unroll
+            for (uint32_t x = 0; x < kGroup; x += kStep)
+                dma16(gb + (g * nk + s) * kGroup + x, voff, stage + (GA + g) * kGroup + x + wave_lds);
+    };
+    // fragment addresses: row lane % 32 of the wave's first tile, the chunk of
+    // k 8 (lane / 32), permuted as stored; the other chunk of a block is at ^ 32
+    const int sw = (lane >> 2) & 3, row = lane & 31;
+    const uint32_t chunk = (((lane >> 5) ^ sw) * 16);
+    const int am = wm * MT * 32, bn = wn * NT * 32;
+    const uint32_t fa = (am / kBlockRows) * kGroup + (am % kBlockRows + row) * 64 + chunk;
+    const uint32_t fb = (GA + bn / kBlockRows) * kGroup + (bn % kBlockRows + row) * 64 + chunk;
+    // a[x][i], b[x][j]: x = hi / lo plane (split) or the two k steps of the phase
+    struct Frag {
+        u32x4 a[2][MT], b[2][NT];
+    };
+    auto read_phase = [&](Frag& f, uint32_t stage, int phase) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const uint32_t block = (TERMS == 3 ? x : phase) * (kBlockElems * 2);
+            const uint32_t flip = (TERMS == 3 ? phase : x) * 32;
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                f.a[x][i] = *reinterpret_cast<const u32x4*>(gemm_lds + stage + ((fa ^ flip) + block + i * 2048));
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                f.b[x][j] = *reinterpret_cast<const u32x4*>(gemm_lds + stage + ((fb ^ flip) + block + j * 2048));
+        }
+    };
+    auto multiply = [&](const Frag& f) {
+        if constexpr (TERMS == 3) {  // lo*hi, hi*lo, hi*hi
+#pragma unroll
+            for (int t = 0; t < 3; ++t)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i)
+                        mfma32<F16>(f.b[t == 1 ? 1 : 0][j], f.a[t == 0 ? 1 : 0][i], acc[j][i]);
+        } else {
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+#pragma unroll
+                    for (int i = 0; i < MT; ++i) mfma32<F16>(f.b[x][j], f.a[x][i], acc[j][i]);
+        }
+    };
+
+    Frag f0, f1;
+    uint32_t stage = 0;
+    load_slice(s0, 0);
+    if (s0 + 1 < s1) {
+        load_slice(s0 + 1, kStage);
+        wait_stage<kLoads>();
+    } else {
+        wait_stage<0>();
     }
-    // next K slice in flight in registers: A hi/lo and B hi/lo
-    u32x4 pah[CH], pal[CH], pbh[CH], pbl[CH];
-#pragma unroll
-    for (int q = 0; q < CH; ++q) {
-        pah[q] = *reinterpret_cast<const u32x4*>(Ah + oa[q]);
-        pbh[q] = *reinterpret_cast<const u32x4*>(Bh + ob[q]);
-        if constexpr (TERMS == 3) {
-            pal[q] = *reinterpret_cast<const u32x4*>(Al + oa[q]);
-            pbl[q] = *reinterpret_cast<const u32x4*>(Bl + ob[q]);
-        }
-    }
-    for (int64_t k0 = 0; k0 < Kp; k0 += BK) {
-#pragma unroll
-        for (int q = 0; q < CH; ++q) {
-            *reinterpret_cast<u32x4*>(&sAh[so[q]]) = pah[q];
-            *reinterpret_cast<u32x4*>(&sBh[so[q]]) = pbh[q];
-            if constexpr (TERMS == 3) {
-                *reinterpret_cast<u32x4*>(&sAl[so[q]]) = pal[q];
-                *reinterpret_cast<u32x4*>(&sBl[so[q]]) = pbl[q];
-            }
-        }
-        __syncthreads();
-        if (k0 + BK < Kp) {
-            const int64_t k1 = k0 + BK;
-#pragma unroll
-            for (int q = 0; q < CH; ++q) {
-                pah[q] = *reinterpret_cast<const u32x4*>(Ah + oa[q] + k1);
-                pbh[q] = *reinterpret_cast<const u32x4*>(Bh + ob[q] + k1);
-                if constexpr (TERMS == 3) {
-                    pal[q] = *reinterpret_cast<const u32x4*>(Al + oa[q] + k1);
-                    pbl[q] = *reinterpret_cast<const u32x4*>(Bl + ob[q] + k1);
-                }
-            }
-        }
-#pragma unroll
-        for (int ks = 0; ks < BK; ks += 16) {
-            const int kk = ks + 8 * (lane >> 5);
-            u32x4 ah[4], al[4], bh[TJ], bl[TJ];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int r = (wm * 128 + i * 32 + (lane & 31)) * LDK + kk;
-                ah[i] = *reinterpret_cast<const u32x4*>(&sAh[r]);
-                if constexpr (TERMS == 3) al[i] = *reinterpret_cast<const u32x4*>(&sAl[r]);
-            }
-#pragma unroll
-            for (int j = 0; j < TJ; ++j) {
-                const int r = (wn * (32 * TJ) + j * 32 + (lane & 31)) * LDK + kk;
-                bh[j] = *reinterpret_cast<const u32x4*>(&sBh[r]);
-                if constexpr (TERMS == 3) bl[j] = *reinterpret_cast<const u32x4*>(&sBl[r]);
-            }
-#pragma unroll
-            for (int j = 0; j < TJ; ++j)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if constexpr (TERMS == 3) {
-                        mfma32<F16>(bh[j], al[i], acc[j][i]);
-                        mfma32<F16>(bl[j], ah[i], acc[j][i]);
-                    }
-                    mfma32<F16>(bh[j], ah[i], acc[j][i]);
-                }
-        }
-        __syncthreads();
+    read_phase(f0, 0, 0);
+    for (int64_t s = s0; s < s1; ++s) {
+        read_phase(f1, stage, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(f0);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_stage<0>();
+        if (s + 2 < s1) load_slice(s + 2, stage);
+        stage ^= kStage;
+        if (s + 1 < s1) read_phase(f0, stage, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(f1);
+        __builtin_amdgcn_sched_barrier(0);
     }
     // epilogue: acc[j][i][v] is C(row, col) with row = m tile i, lane % 32 and
     // col = n tile j, 8 (v / 4) + 4 (lane / 32) + v % 4
@@ -403,86 +451,135 @@ __global__ __launch_bounds__(NT) void gemm_mfma_kernel(
         scale = ldexp(alpha, -((13 - ea) + (13 - eb)));
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t row = m0 + wm * 128 + i * 32 + (lane & 31);
-        if (row >= M) continue;
+    for (int i = 0; i < MT; ++i) {
+        const int64_t r = m0 + am + i * 32 + row;
+        if (r >= M) continue;
 #pragma unroll
-        for (int j = 0; j < TJ; ++j)
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
-                const int64_t col = n0 + wn * (32 * TJ) + j * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
+                const int64_t col = n0 + bn + j * 32 + 8 * (v / 4) + 4 * (lane >> 5) + (v % 4);
                 if (col < N) {
-                    float* p = C + row + col * ldc;
-                    double r = scale * static_cast<double>(acc[j][i][v]);
-                    if (beta != 0.0) r += beta * static_cast<double>(*p);
-                    *p = static_cast<float>(r);
+                    if (partial) {
+                        partial[(split * N + col) * M + r] = acc[j][i][v];
+                        continue;
+                    }
+                    float* p = C + r + col * ldc;
+                    double t = scale * static_cast<double>(acc[j][i][v]);
+                    if (beta != 0.0) t += beta * static_cast<double>(*p);
+                    *p = static_cast<float>(t);
                 }
             }
     }
 }
 
-// Staged operand planes: absmax words, then A hi [Mp][Kp], B hi [Np][Kp]
-// and, for the split, A lo and B lo.
+// C = scale * (sum of the K splits' partial products, in FP64) + beta C
+__global__ __launch_bounds__(256) void gemm_split_sum_kernel(int64_t M, int64_t N, int splits,
+                                                             const float* __restrict__ partial, double alpha,
+                                                             double beta, float* __restrict__ C, int64_t ldc,
+                                                             const unsigned* __restrict__ absA,
+                                                             const unsigned* __restrict__ absB) {
+    double scale = alpha;
+    if (absA) {
+        int ea = 0, eb = 0;
+        frexpf(fmaxf(__uint_as_float(*absA), 1e-38f), &ea);
+        frexpf(fmaxf(__uint_as_float(*absB), 1e-38f), &eb);
+        scale = ldexp(alpha, -((13 - ea) + (13 - eb)));
+    }
+    const int64_t total = M * N;
+    for (int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; t < total;
+         t += static_cast<int64_t>(gridDim.x) * 256) {
+        double v = 0.0;
+        for (int q = 0; q < splits; ++q) v += static_cast<double>(partial[q * total + t]);
+        float* p = C + t % M + t / M * ldc;
+        v *= scale;
+        if (beta != 0.0) v += beta * static_cast<double>(*p);
+        *p = static_cast<float>(v);
+    }
+}
+
+// Staged operands: absmax words, A, B, then the partial products of K splits.
 struct Planes {
-    int64_t Mp, Np, Kp;
+    int64_t Mp, Np, Kp, nk;  // padded sizes, K slices
     unsigned* absmax;
-    uint16_t *Ah, *Bh, *Al, *Bl;
+    uint16_t *A, *B;
+    float* partial;
 };
+
+int64_t slice_k(int terms) { return terms == 3 ? kBlockK : 2 * kBlockK; }
 
 Planes planes_of(int terms, int64_t M, int64_t N, int64_t K, void* base_ptr) {
     Planes p;
-    p.Mp = ceil_div(M, BM) * BM;
-    p.Np = ceil_div(N, BN) * BN;
-    p.Kp = std::max<int64_t>(ceil_div(K, BK) * BK, BK);
+    p.Mp = ceil_div(M, kPadRows) * kPadRows;
+    p.Np = ceil_div(N, kPadRows) * kPadRows;
+    p.nk = std::max<int64_t>(ceil_div(K, slice_k(terms)), 1);
+    p.Kp = p.nk * slice_k(terms);
     char* base = static_cast<char*>(base_ptr);
     p.absmax = reinterpret_cast<unsigned*>(base);
-    p.Ah = reinterpret_cast<uint16_t*>(base + 256);
-    p.Bh = p.Ah + p.Mp * p.Kp;
-    p.Al = terms == 3 ? p.Bh + p.Np * p.Kp : nullptr;
-    p.Bl = terms == 3 ? p.Al + p.Mp * p.Kp : nullptr;
+    p.A = reinterpret_cast<uint16_t*>(base + 256);
+    p.B = p.A + p.Mp * p.nk * 2 * kBlockK;
+    p.partial = reinterpret_cast<float*>(p.B + p.Np * p.nk * 2 * kBlockK);
     return p;
+}
+
+// Launch shape.  256 x 256 tiles (8 waves) read the LDS least per MFMA and
+// are taken where they about fill the chip; below that 128 x 128 (4 waves,
+// two blocks a CU), and K is split while the tiles are under half the 512
+// blocks the chip holds, as long as a split keeps kMinSlices slices.
+// Measured (hi-only whole call, us, before / now / with 256-wide tiles and
+// splits): 712 x 83 x 5473 178 / 27 / 38; 2451 x 337 x 2714 107 / 36 / 45;
+// 2000^3 88 / 47 / 58; 3001 x 1501 x 6001 223 / 117 / 118; 4096^3 (256 tiles)
+// 173 / 142 / 143.  Splitting for 768 or 1024 blocks: 4950 x 397 x 4895 75 -> 87.
+struct Shape {
+    bool large;
+    int64_t tiles, slices;  // C tiles, K slices per split
+    int splits;
+};
+constexpr int64_t kMinSlices = 8, kLargeTiles = 192, kSplitBlocks = 512;
+Shape shape_of(int64_t M, int64_t N, int64_t nk) {
+    Shape h;
+    const int64_t big = ceil_div(M, 256) * ceil_div(N, 256), small = ceil_div(M, 128) * ceil_div(N, 128);
+    h.large = big >= kLargeTiles;
+    h.tiles = h.large ? big : small;
+    int64_t splits = h.large ? 1 : std::max<int64_t>(1, kSplitBlocks / small);
+    splits = std::max<int64_t>(1, std::min<int64_t>(splits, nk / kMinSlices));
+    h.slices = ceil_div(nk, splits);
+    h.splits = static_cast<int>(ceil_div(nk, h.slices));
+    return h;
 }
 
 // Stage one operand: X is rows x cols column-major; kcontig means the GEMM's
 // K runs down X's columns (X is K x R), otherwise along its rows (X is R x K).
-void stage(int mode, bool f16, const Src& x, bool kcontig, int64_t rows, int64_t cols, int64_t pad_r,
-           int64_t Kp, uint16_t* hi, uint16_t* lo, const unsigned* absmax, hipStream_t s) {
+void stage(int mode, bool f16, const Src& x, bool kcontig, int64_t rows, int64_t cols, int64_t pad_r, int64_t nk,
+           int64_t Kp, uint16_t* out, const unsigned* absmax, hipStream_t s) {
+    require(kcontig || pad_r / 64 < 65536, "gemm: operand too large");
+    const dim3 grid(static_cast<unsigned>(ceil_div(Kp, 64)),
+                    static_cast<unsigned>(kcontig ? std::min<int64_t>(pad_r / 32, 65535) : pad_r / 64));
     if (kcontig) {
-        const bool vec = rows % 8 == 0 && x.ld % 8 == 0 &&
-                         (x.f ? reinterpret_cast<uintptr_t>(x.f) % 16 == 0
-                              : reinterpret_cast<uintptr_t>(x.wh) % 16 == 0 &&
-                                    (mode == PREP_HI || reinterpret_cast<uintptr_t>(x.wr) % 16 == 0));
-        if (vec && rows > 0) {
-            const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(ceil_div(pad_r * Kp / 8, 256), 65536));
-            if (mode == PREP_HI)
-                prep_k_vec_kernel<PREP_HI><<<blocks, 256, 0, s>>>(x, rows, cols, Kp, hi, lo, absmax, f16, pad_r, Kp);
-            else
-                prep_k_vec_kernel<PREP_SPLIT><<<blocks, 256, 0, s>>>(x, rows, cols, Kp, hi, lo, absmax, f16, pad_r,
-                                                                     Kp);
-        } else {
-            const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(ceil_div(pad_r * Kp, 256), 65536));
-            if (mode == PREP_HI)
-                prep_k_kernel<PREP_HI><<<blocks, 256, 0, s>>>(x, rows, cols, Kp, hi, lo, absmax, f16, pad_r, Kp);
-            else
-                prep_k_kernel<PREP_SPLIT><<<blocks, 256, 0, s>>>(x, rows, cols, Kp, hi, lo, absmax, f16, pad_r, Kp);
-        }
-    } else {
-        require(ceil_div(pad_r, 64) < 65536, "gemm: operand too large");
-        const dim3 grid(static_cast<unsigned>(ceil_div(Kp, 64)), static_cast<unsigned>(ceil_div(pad_r, 64)));
         if (mode == PREP_HI)
-            prep_t_kernel<PREP_HI><<<grid, 256, 0, s>>>(x, rows, cols, Kp, hi, lo, absmax, f16, pad_r, Kp);
+            prep_k_kernel<PREP_HI><<<grid, 256, 0, s>>>(x, rows, cols, pad_r, nk, Kp, out, absmax, f16);
         else
-            prep_t_kernel<PREP_SPLIT><<<grid, 256, 0, s>>>(x, rows, cols, Kp, hi, lo, absmax, f16, pad_r, Kp);
+            prep_k_kernel<PREP_SPLIT><<<grid, 256, 0, s>>>(x, rows, cols, pad_r, nk, Kp, out, absmax, f16);
+    } else {
+        if (mode == PREP_HI)
+            prep_t_kernel<PREP_HI><<<grid, 256, 0, s>>>(x, rows, cols, nk, Kp, out, absmax, f16);
+        else
+            prep_t_kernel<PREP_SPLIT><<<grid, 256, 0, s>>>(x, rows, cols, nk, Kp, out, absmax, f16);
     }
     TOMOS_LAUNCH_CHECK("gemm operand staging");
 }
 
 }  // namespace
 
+// Staged planes only (the least a call needs), and with the K splits' partials.
+size_t gemm_planes_bytes(int terms, int64_t M, int64_t N, int64_t K) {
+    const Planes p = planes_of(terms, M, N, K, nullptr);
+    return static_cast<size_t>((p.Mp + p.Np) * p.nk * 2 * kBlockK) * 2 + 256;
+}
 size_t gemm_mfma_scratch_bytes(int terms, int64_t M, int64_t N, int64_t K) {
-    const int64_t Mp = ceil_div(M, BM) * BM, Np = ceil_div(N, BN) * BN;
-    const int64_t Kp = std::max<int64_t>(ceil_div(K, BK) * BK, BK);
-    return static_cast<size_t>((terms == 3 ? 2 : 1) * (Mp + Np) * Kp) * 2 + 256;
+    const Planes p = planes_of(terms, M, N, K, nullptr);
+    const Shape h = shape_of(M, N, p.nk);
+    return gemm_planes_bytes(terms, M, N, K) + (h.splits > 1 ? static_cast<size_t>(h.splits) * M * N * 4 : 0);
 }
 
 size_t gemm_split_scratch_bytes(int64_t M, int64_t N, int64_t K) { return gemm_mfma_scratch_bytes(3, M, N, K); }
@@ -499,41 +596,67 @@ void gemm_mfma(int terms, bool f16, const Src& a, bool a_kcontig, const Src& b, 
                size_t scratch_bytes, hipStream_t s) {
     require(terms == 1 || terms == 3, "gemm_mfma: terms must be 1 or 3");
     if (M == 0 || N == 0) return;
-    const size_t need = gemm_mfma_scratch_bytes(terms, M, N, K);
-    if (!scratch) scratch = fallback_scratch(need);
-    else require(scratch_bytes >= need, "gemm: scratch too small (need " + std::to_string(need) + " bytes)");
+    const size_t least = gemm_planes_bytes(terms, M, N, K), need = gemm_mfma_scratch_bytes(terms, M, N, K);
+    if (!scratch) {
+        scratch = fallback_scratch(need);
+        scratch_bytes = need;
+    }
+    require(scratch_bytes >= least, "gemm: scratch too small (need " + std::to_string(least) + " bytes)");
     const Planes p = planes_of(terms, M, N, K, scratch);
     const int mode = terms == 3 ? PREP_SPLIT : PREP_HI;
     const bool scaled = terms == 3 && f16;
     if (scaled) {
-        TOMOS_HIP_CHECK(hipMemsetAsync(p.absmax, 0, 8, s));
+        absmax_clear_kernel<<<1, 2, 0, s>>>(p.absmax);
         if (K > 0) {
-            absmax_kernel<<<2048, 256, 0, s>>>(a, a_kcontig ? K : M, a_kcontig ? M : K, p.absmax);
-            absmax_kernel<<<2048, 256, 0, s>>>(b, b_kcontig ? K : N, b_kcontig ? N : K, p.absmax + 1);
+            auto absmax = [&](const Src& x, int64_t rows, int64_t cols, unsigned* out) {
+                const int64_t bx = ceil_div(rows, 2048);  // about 2048 blocks in all
+                const dim3 grid(static_cast<unsigned>(bx),
+                                static_cast<unsigned>(std::min(cols, std::max<int64_t>(2048 / bx, 1))));
+                absmax_kernel<<<grid, 256, 0, s>>>(x, rows, cols, out);
+            };
+            absmax(a, a_kcontig ? K : M, a_kcontig ? M : K, p.absmax);
+            absmax(b, b_kcontig ? K : N, b_kcontig ? N : K, p.absmax + 1);
             TOMOS_LAUNCH_CHECK("absmax_kernel");
         }
     }
-    stage(mode, f16, a, a_kcontig, a_kcontig ? K : M, a_kcontig ? M : K, p.Mp, p.Kp, p.Ah, p.Al, p.absmax, s);
-    stage(mode, f16, b, b_kcontig, b_kcontig ? K : N, b_kcontig ? N : K, p.Np, p.Kp, p.Bh, p.Bl, p.absmax + 1, s);
-    const int64_t nblocks = (p.Mp / BM) * (p.Np / BN);
+    stage(mode, f16, a, a_kcontig, a_kcontig ? K : M, a_kcontig ? M : K, p.Mp, p.nk, p.Kp, p.A, p.absmax, s);
+    stage(mode, f16, b, b_kcontig, b_kcontig ? K : N, b_kcontig ? N : K, p.Np, p.nk, p.Kp, p.B, p.absmax + 1, s);
+    Shape h = shape_of(M, N, p.nk);
+    if (scratch_bytes < need) {  // a scratch of the planes alone: no K splits
+        h.splits = 1;
+        h.slices = p.nk;
+    }
+    const int64_t nblocks = h.tiles * h.splits;
     require(nblocks < (int64_t(1) << 31), "gemm: grid too large");
     const unsigned* absA = scaled ? p.absmax : nullptr;
     const unsigned* absB = scaled ? p.absmax + 1 : nullptr;
-    const int lds = (terms == 3 ? 4 : 2) * kPlaneElems * 2;
-    auto launch = [&](auto* k) {
+    float* partial = h.splits > 1 ? p.partial : nullptr;
+    auto launch = [&](auto* k, int threads, int tile) {
+        const int lds = 2 * 2 * (tile / kBlockRows) * 2 * kBlockElems * 2;  // two stages of A and B slices
         TOMOS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                             hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-        k<<<static_cast<unsigned>(nblocks), kGemmThreads, lds, s>>>(M, N, p.Kp, p.Ah, p.Al, p.Bh, p.Bl, p.Kp, alpha,
-                                                                    beta, c, ldc, absA, absB);
+        k<<<static_cast<unsigned>(nblocks), threads, lds, s>>>(M, N, p.nk, h.slices, p.A, p.B, alpha, beta, c, ldc, absA,
+                                                               absB, partial);
     };
-    if (terms == 3) {
-        if (f16) launch(gemm_mfma_kernel<true, kGemmThreads, 3>);
-        else launch(gemm_mfma_kernel<false, kGemmThreads, 3>);
+    auto run = [&](auto f16_, auto terms_) {
+        if (h.large) launch(gemm_mfma_kernel<f16_, terms_, 2, 4, 4, 2>, 512, 256);
+        else launch(gemm_mfma_kernel<f16_, terms_, 2, 2, 2, 2>, 256, 128);
+    };
+    using one = std::integral_constant<int, 1>;
+    using three = std::integral_constant<int, 3>;
+    if (f16) {
+        if (terms == 3) run(std::true_type{}, three{});
+        else run(std::true_type{}, one{});
     } else {
-        if (f16) launch(gemm_mfma_kernel<true, kGemmThreads, 1>);
-        else launch(gemm_mfma_kernel<false, kGemmThreads, 1>);
+        if (terms == 3) run(std::false_type{}, three{});
+        else run(std::false_type{}, one{});
     }
     TOMOS_LAUNCH_CHECK("gemm_mfma_kernel");
+    if (h.splits > 1) {
+        const unsigned blocks = static_cast<unsigned>(std::min<int64_t>(ceil_div(M * N, 256), 16384));
+        gemm_split_sum_kernel<<<blocks, 256, 0, s>>>(M, N, h.splits, partial, alpha, beta, c, ldc, absA, absB);
+        TOMOS_LAUNCH_CHECK("gemm_split_sum_kernel");
+    }
 }
 
 void gemm_split(int a_type, int64_t M, int64_t N, int64_t K, double alpha, const uint16_t* awh,
