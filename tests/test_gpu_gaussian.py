@@ -114,3 +114,20 @@ def test_errors(capi):
     with pytest.raises(C.TomosError, match="F64, F32, F16 or BF16"):
         C.call("tomos_gaussian_fill", C.FP32_16, 2, 2, buf.ptr, 2, 1, None)
     C.call("tomos_gaussian_fill", C.F32, 0, 5, None, 1, 1, None)  # empty: no-op
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 3), (2, 70000), (511, 5), (512, 5), (513, 66000), (4000, 17)])
+def test_transform_accuracy(capi, orc, rows, cols):
+    """Launch edges (one pair, a part block, columns beyond the grid) and the
+    transform's error against FP64: r and the circular function are each
+    within 2 ulp (log 1, square root and rounding 1; polynomial and rounding
+    1.5), |x| <= 5.8, so 4 * 2^-23 * 5.8 = 2.8e-6 bounds the largest error and
+    a fifth of 2^-23 relative in the 2-norm (rms of uniform roundings) 1e-7."""
+    out = C.DeviceBuffer(rows * cols * 4)
+    print("gaussian", rows, cols, flush=True)
+    C.call("tomos_gaussian_fill", C.F32, rows, cols, out.ptr, rows, 12345, None)
+    got = out.to_numpy(np.float32, (rows, cols)).astype(np.float64)
+    ref = np.zeros((rows, cols), np.float64, order="F")
+    orc.lib().orc_gaussian_fill_f64(rows, cols, ref.ctypes.data_as(orc.f64p), rows, 12345)
+    assert np.abs(got - ref).max() <= 2.8e-6
+    assert np.linalg.norm(got - ref) <= 1e-7 * np.linalg.norm(ref) + 1e-12
