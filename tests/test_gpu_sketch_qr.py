@@ -386,3 +386,26 @@ def test_cholqr_graded_columns(capi, k, n, cond):
     sgn = np.sign(np.diag(R)) * np.sign(np.diag(Rn))
     rowerr = np.abs(R - sgn[:, None] * Rn).max(axis=1) / np.abs(np.diag(Rn))
     assert rowerr.max() < 1e-12, rowerr.max()
+
+
+@pytest.mark.parametrize("a_type", [C.F32, C.FP32_16, C.FP32_BF16])
+@pytest.mark.parametrize("m,n,s", [(7, 3, 5), (9, 2, 3), (16391, 5, 40), (20011, 9, 300), (5000, 3, 20000)])
+@pytest.mark.parametrize("pad", [1, 3, 5])
+def test_sketch_does_not_depend_on_alignment(capi, a_type, m, n, s, pad):
+    """The fixed-point sketch depends on the values only: columns at any
+    element alignment give the aligned call's result bit for bit (fewer rows
+    than a vector, ragged tails, both kinds of exponents, one column a block)."""
+    rng = np.random.default_rng(m + pad)
+    A = np.asfortranarray((rng.standard_normal((m, n)) * 2.0 ** rng.integers(-6, 7, (m, n))).astype(np.float32))
+    out = []
+    for lda in ((m + 7) // 8 * 8, (m + 7) // 8 * 8 + pad):
+        print("alignment", a_type, m, n, s, lda, flush=True)
+        if a_type == C.F32:
+            Ap = np.full((lda, n), np.nan, np.float32, order="F")
+            Ap[:m] = A
+            out.append(H.countsketch_apply(a_type, C.TIER_EXACT, m, n, H.dev(Ap), None, lda, s))
+        else:
+            variant = C.PACK_FP32_16 if a_type == C.FP32_16 else C.PACK_FP32_BF16
+            wh, wr = H.pack(variant, A, ld=lda)
+            out.append(H.countsketch_apply(a_type, C.TIER_EXACT, m, n, wh, wr, lda, s))
+    assert np.array_equal(out[0], out[1])

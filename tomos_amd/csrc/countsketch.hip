@@ -16,8 +16,7 @@
 // The LDS slice is written to a per-split partial, and a second pass sums
 // the splits in a fixed order in FP64.  Bucket/sign indices are bit-exact;
 // the values are FP32 sums within a split (order depends on LDS atomic
-// order), FP64 across splits.  A, lda or the split start not 16-byte
-// aligned takes the element-wise kernel.
+// order), FP64 across splits.
 #include <algorithm>
 #include <type_traits>
 #include <vector>
@@ -74,51 +73,14 @@ __device__ __forceinline__ float load_elem(const void* __restrict__ a,
     }
 }
 
-template <int FMT, bool EXACT, int CG>
-__global__ __launch_bounds__(256) void cs_apply_kernel(int64_t m, int64_t n,
-                                                       const void* __restrict__ a,
-                                                       const uint16_t* __restrict__ wr,
-                                                       int64_t lda, int64_t s,
-                                                       const uint32_t* __restrict__ packed,
-                                                       int64_t rows_per_split, int ncg,
-                                                       float* __restrict__ partial) {
-    extern __shared__ float ylds[];  // [s][CG]
-    const int split = blockIdx.x / ncg;
-    const int cg = blockIdx.x - split * ncg;
-    const int64_t c0 = static_cast<int64_t>(cg) * CG;
-    const int ncols = static_cast<int>(min<int64_t>(CG, n - c0));
-    for (int64_t t = threadIdx.x; t < s * CG; t += 256) ylds[t] = 0.0f;
-    __syncthreads();
-
-    const int64_t r0 = static_cast<int64_t>(split) * rows_per_split;
-    const int64_t r1 = min(m, r0 + rows_per_split);
-    for (int64_t i = r0 + threadIdx.x; i < r1; i += 256) {
-        const uint32_t w = packed[i];
-        const int b = static_cast<int>(w & 0x7FFFFFFFu);
-        const float sg = (w & 0x80000000u) ? -1.0f : 1.0f;
-#pragma unroll
-        for (int c = 0; c < CG; ++c) {
-            if (c < ncols) {
-                const float v = load_elem<FMT, EXACT>(a, wr, i + (c0 + c) * lda);
-                atomicAdd(&ylds[b * CG + c], sg * v);
-            }
-        }
-    }
-    __syncthreads();
-    float* out = partial + static_cast<int64_t>(split) * s * n;
-    for (int64_t t = threadIdx.x; t < s * ncols; t += 256) {
-        const int64_t c = t / s;
-        const int64_t b = t - c * s;
-        out[(c0 + c) * s + b] = ylds[b * CG + c];
-    }
-}
-
 template <int FMT>
 constexpr int vec_rows() {
     return FMT == FMT_F64 ? 2 : (FMT == FMT_F32 ? 4 : 8);
 }
 
-template <int FMT, bool EXACT>
+// PAIRS: FP32_16 words two at a time (a vector with a saturated word, all of
+// its words one by one).
+template <int FMT, bool EXACT, bool PAIRS = true>
 __device__ __forceinline__ void decode_rows(const uint4& h, const uint4& l,
                                             float (&v)[vec_rows<FMT>()]) {
     if constexpr (FMT == FMT_F64) {
@@ -132,6 +94,23 @@ __device__ __forceinline__ void decode_rows(const uint4& h, const uint4& l,
     } else {
         const uint32_t hw[4] = {h.x, h.y, h.z, h.w};
         const uint32_t lw[4] = {l.x, l.y, l.z, l.w};
+        if constexpr (FMT == FMT_P16 && PAIRS) {
+            if (!EXACT || (codec::fp32_16_saturated2(h.x) | codec::fp32_16_saturated2(h.y) |
+                           codec::fp32_16_saturated2(h.z) | codec::fp32_16_saturated2(h.w)) == 0) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    if constexpr (EXACT) {
+                        codec::fp32_16_decode_exact2(hw[k], lw[k], v[2 * k], v[2 * k + 1]);
+                    } else {
+                        const uint32_t b = codec::fp32_16_half_bits2(hw[k]);
+                        v[2 * k] = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(b)));
+                        v[2 * k + 1] =
+                            static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(b >> 16)));
+                    }
+                }
+                return;
+            }
+        }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
 #pragma unroll
@@ -153,8 +132,20 @@ __device__ __forceinline__ void decode_rows(const uint4& h, const uint4& l,
 
 constexpr int kVecThreads = 1024;
 
-// Vector path: rows_per_split, lda and the base pointers are multiples of
-// the 16-byte row vector (checked by the host).
+// A vector of rows at element alignment: gfx950 global loads take any, so
+// columns need not start on 16 bytes (an lda that is no multiple of the
+// vector took an element-wise kernel with float atomics before: 250001 x 300
+// FP32_16, s = 1200, 517 us, now 100 with the pair decode and fx_term).
+template <bool NTL>
+__device__ __forceinline__ uint4 load_rows16(const void* p) {
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4), aligned(2)));
+    u32x4 v;
+    if constexpr (NTL) v = __builtin_nontemporal_load(static_cast<const u32x4*>(p));
+    else v = *static_cast<const u32x4*>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+// rows_per_split is a multiple of the row vector (of the index words too).
 template <int FMT, bool EXACT, int CG>
 __global__ __launch_bounds__(kVecThreads) void cs_apply_vec_kernel(
     int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr, int64_t lda,
@@ -194,9 +185,9 @@ __global__ __launch_bounds__(kVecThreads) void cs_apply_vec_kernel(
             for (int c = 0; c < CG; ++c) {
                 if (c < ncols) {
                     const int64_t e = i0 + (c0 + c) * lda;
-                    h[c] = *reinterpret_cast<const uint4*>(abase + e * EB);
+                    h[c] = load_rows16<false>(abase + e * EB);
                     if constexpr (EXACT && (FMT == FMT_P16 || FMT == FMT_PBF))
-                        l[c] = *reinterpret_cast<const uint4*>(wr + e);
+                        l[c] = load_rows16<false>(wr + e);
                     else
                         l[c] = make_uint4(0, 0, 0, 0);
                 }
@@ -277,9 +268,9 @@ __global__ __launch_bounds__(256) void cs_colmax_kernel(int64_t m, const void* _
     for (int64_t i0 = r0 + static_cast<int64_t>(threadIdx.x) * V; i0 < r1; i0 += 256 * V) {
         float v[V];
         if (i0 + V <= r1) {
-            const uint4 h = load_a16<NTL>(col + i0 * EB);
+            const uint4 h = load_rows16<NTL>(col + i0 * EB);
             uint4 l = make_uint4(0, 0, 0, 0);
-            if constexpr (EXACT) l = load_a16<NTL>(wr + i0 + j * lda);
+            if constexpr (EXACT) l = load_rows16<NTL>(wr + i0 + j * lda);
             decode_rows<FMT, EXACT>(h, l, v);
         } else {
             for (int r = 0; r < V; ++r) v[r] = (i0 + r < r1) ? load_elem<FMT, EXACT>(a, wr, i0 + r + j * lda) : 0.0f;
@@ -346,10 +337,10 @@ __device__ __forceinline__ void cs_sample_exp_body(int64_t j, int64_t m, const v
         const int64_t i0 = static_cast<int64_t>(sg) * stride + static_cast<int64_t>(t - sg * vps) * V;
         float v[V];
         if (i0 + V <= m) {
-            const uint4 h = load_a16<false>(col + i0 * EB);
+            const uint4 h = load_rows16<false>(col + i0 * EB);
             uint4 l = make_uint4(0, 0, 0, 0);
-            if constexpr (EXACT) l = load_a16<false>(wr + i0 + j * lda);
-            decode_rows<FMT, EXACT>(h, l, v);
+            if constexpr (EXACT) l = load_rows16<false>(wr + i0 + j * lda);
+            decode_rows<FMT, EXACT, false>(h, l, v);
         } else {
             for (int r = 0; r < V; ++r) v[r] = (i0 + r < m) ? load_elem<FMT, EXACT>(a, wr, i0 + r + j * lda) : 0.0f;
         }
@@ -436,8 +427,19 @@ __global__ __launch_bounds__(256) void cs_group_exp_kernel(const CsGroupDesc* __
                                    q.flags);
 }
 
-template <int FMT, bool EXACT, int CG, bool NTL>
-__device__ __forceinline__ void cs_apply_fx_body(
+// round(v 2^sc) to the nearest even 64-bit integer, |v 2^sc| < 2^50: the FP64
+// sum with 1.5 2^52 leaves it in the low bits (the sum's only rounding; the
+// product is exact).  `scale` = 2^sc.  Five operations against about twenty
+// for ldexpf and the conversion of any float.
+constexpr int kMagicShift = 50;
+__device__ __forceinline__ unsigned long long fx_term(float v, double scale) {
+    const uint64_t d = __builtin_bit_cast(uint64_t, fma(static_cast<double>(v), scale, 0x1.8p52));
+    return (static_cast<uint64_t>(static_cast<uint32_t>(d >> 32) - 0x43380000u) << 32) | static_cast<uint32_t>(d);
+}
+
+// MAGIC: shift <= kMagicShift (m >= 1024), the terms by fx_term.
+template <int FMT, bool EXACT, int CG, bool NTL, bool MAGIC>
+__device__ __forceinline__ void cs_apply_fx_rows(
     int split, int cg, int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
     int64_t lda, int64_t s, const uint32_t* __restrict__ packed, int64_t rows_per_split,
     const int* __restrict__ colexp, int shift, unsigned long long* __restrict__ partial, int* __restrict__ over) {
@@ -448,10 +450,12 @@ __device__ __forceinline__ void cs_apply_fx_body(
     const int ncols = static_cast<int>(min<int64_t>(CG, n - c0));
     for (int64_t t = threadIdx.x; t < s * CG; t += kVecThreads) yfx[t] = 0ull;
     int sc[CG];
+    double scale[CG];
     float bnd[CG];  // |value| < 2^e_c keeps every term below 2^shift (no overflow)
 #pragma unroll
     for (int c = 0; c < CG; ++c) {
         sc[c] = c < ncols ? shift - colexp[c0 + c] : 0;
+        scale[c] = MAGIC ? ldexp(1.0, sc[c]) : 0.0;
         bnd[c] = c < ncols ? ldexpf(1.0f, colexp[c0 + c]) : 0.0f;
     }
     bool beyond = false;  // a value at or above its column's bound (or not finite)
@@ -481,9 +485,9 @@ __device__ __forceinline__ void cs_apply_fx_body(
             for (int c = 0; c < CG; ++c) {
                 if (c < ncols) {
                     const int64_t e = i0 + (c0 + c) * lda;
-                    h[c] = load_a16<NTL>(abase + e * EB);
+                    h[c] = load_rows16<NTL>(abase + e * EB);
                     if constexpr (EXACT && (FMT == FMT_P16 || FMT == FMT_PBF))
-                        l[c] = load_a16<NTL>(wr + e);
+                        l[c] = load_rows16<NTL>(wr + e);
                     else
                         l[c] = make_uint4(0, 0, 0, 0);
                 }
@@ -497,9 +501,14 @@ __device__ __forceinline__ void cs_apply_fx_body(
                     for (int r = 0; r < V; ++r) {
                         const int b = static_cast<int>(w[r] & 0x7FFFFFFFu);
                         beyond = beyond || !(fabsf(v[r]) < bnd[c]);
-                        const long long q = __float2ll_rn(ldexpf(v[r], sc[c]));
-                        atomicAdd(&yfx[c * s + b],
-                                  static_cast<unsigned long long>((w[r] & 0x80000000u) ? -q : q));
+                        if constexpr (MAGIC) {
+                            const float sv = __uint_as_float(__float_as_uint(v[r]) ^ (w[r] & 0x80000000u));
+                            atomicAdd(&yfx[c * s + b], fx_term(sv, scale[c]));
+                        } else {
+                            const long long q = __float2ll_rn(ldexpf(v[r], sc[c]));
+                            atomicAdd(&yfx[c * s + b],
+                                      static_cast<unsigned long long>((w[r] & 0x80000000u) ? -q : q));
+                        }
                     }
                 }
             }
@@ -519,6 +528,19 @@ __device__ __forceinline__ void cs_apply_fx_body(
     if (__syncthreads_or(beyond) && threadIdx.x == 0) atomicOr(over, 1);
     unsigned long long* out = partial + static_cast<int64_t>(split) * s * n + c0 * s;
     for (int64_t t = threadIdx.x; t < s * ncols; t += kVecThreads) out[t] = yfx[t];
+}
+
+template <int FMT, bool EXACT, int CG, bool NTL>
+__device__ __forceinline__ void cs_apply_fx_body(
+    int split, int cg, int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
+    int64_t lda, int64_t s, const uint32_t* __restrict__ packed, int64_t rows_per_split,
+    const int* __restrict__ colexp, int shift, unsigned long long* __restrict__ partial, int* __restrict__ over) {
+    if (shift <= kMagicShift)
+        cs_apply_fx_rows<FMT, EXACT, CG, NTL, true>(split, cg, m, n, a, wr, lda, s, packed, rows_per_split, colexp,
+                                                    shift, partial, over);
+    else
+        cs_apply_fx_rows<FMT, EXACT, CG, NTL, false>(split, cg, m, n, a, wr, lda, s, packed, rows_per_split, colexp,
+                                                     shift, partial, over);
 }
 
 template <int FMT, bool EXACT, int CG, bool NTL>
@@ -605,7 +627,8 @@ CsPlan cs_plan_fx(int64_t m, int64_t n, int64_t s) {
     p.cg = 8;
     while (p.cg > 1 && s * p.cg * 8 > kLdsBytes) p.cg >>= 1;
     p.ncg = static_cast<int>(ceil_div(std::max<int64_t>(n, 1), p.cg));
-    const int64_t want = std::max<int64_t>(1, ceil_div(4 * 256, p.ncg));
+    // rounded down: at two blocks a CU, 1026 blocks take three rounds and 988 two
+    const int64_t want = std::max<int64_t>(1, 4 * 256 / p.ncg);
     const int64_t max_splits = std::max<int64_t>(1, ceil_div(m, 8192));
     p.splits = static_cast<int>(std::min(want, max_splits));
     p.rows_per_split = ceil_div(ceil_div(std::max<int64_t>(m, 1), p.splits), 8) * 8;
@@ -642,8 +665,9 @@ CsLayout cs_layout(int64_t m, int64_t n, int64_t s) {
 
 size_t cs_scratch(int64_t m, int64_t n, int64_t s) { return cs_layout(m, n, s).total; }
 
+// Whether columns start on 16-byte boundaries.
 template <int FMT>
-bool vec_ok(const void* a, const uint16_t* wr, int64_t lda, bool exact) {
+bool aligned16(const void* a, const uint16_t* wr, int64_t lda, bool exact) {
     constexpr int V = vec_rows<FMT>();
     const bool lo = !(exact && (FMT == FMT_P16 || FMT == FMT_PBF)) ||
                     (reinterpret_cast<uintptr_t>(wr) % 16 == 0);
@@ -657,23 +681,13 @@ void launch_apply(const CsPlan& p, int64_t m, int64_t n, const void* a, const ui
     const size_t lds = static_cast<size_t>(s) * CG * 4;
     const int64_t blocks = static_cast<int64_t>(p.splits) * p.ncg;
     require(blocks < (int64_t(1) << 31), "countsketch_apply: grid too large");
-    if (vec_ok<FMT>(a, wr, lda, EXACT)) {
-        auto* k = cs_apply_vec_kernel<FMT, EXACT, CG>;
-        TOMOS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k),
-                                            hipFuncAttributeMaxDynamicSharedMemorySize,
-                                            static_cast<int>(lds)));
-        k<<<dim3(static_cast<unsigned>(blocks)), kVecThreads, lds, st>>>(
-            m, n, a, wr, lda, s, packed, p.rows_per_split, p.ncg, partial);
-        TOMOS_LAUNCH_CHECK("cs_apply_vec_kernel");
-        return;
-    }
-    auto* k = cs_apply_kernel<FMT, EXACT, CG>;
+    auto* k = cs_apply_vec_kernel<FMT, EXACT, CG>;
     TOMOS_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(k),
                                         hipFuncAttributeMaxDynamicSharedMemorySize,
                                         static_cast<int>(lds)));
-    k<<<dim3(static_cast<unsigned>(blocks)), 256, lds, st>>>(m, n, a, wr, lda, s, packed,
-                                                            p.rows_per_split, p.ncg, partial);
-    TOMOS_LAUNCH_CHECK("cs_apply_kernel");
+    k<<<dim3(static_cast<unsigned>(blocks)), kVecThreads, lds, st>>>(
+        m, n, a, wr, lda, s, packed, p.rows_per_split, p.ncg, partial);
+    TOMOS_LAUNCH_CHECK("cs_apply_vec_kernel");
 }
 
 template <int FMT, bool EXACT>
@@ -715,7 +729,8 @@ void fx_enqueue(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t
     // suffices; FP32_16's exact values need their own decode
     constexpr bool kExactMax = EXACT && FMT == FMT_P16;
     constexpr int64_t kElemBytes = (FMT == FMT_F64 ? 8 : FMT == FMT_F32 ? 4 : 2) * (EXACT && (FMT == FMT_P16 || FMT == FMT_PBF) ? 2 : 1);
-    const bool ntl = stream_loads(m * n * kElemBytes);
+    // a vector across two cache lines wants the line kept for its neighbour
+    const bool ntl = aligned16<FMT>(a, wr, lda, EXACT) && stream_loads(m * n * kElemBytes);
     if (clear_flags) TOMOS_HIP_CHECK(hipMemsetAsync(flags, 0, 8, st));
     if (sample) {
         // segments start (m / 32) rounded down to 8 rows apart and are
@@ -773,13 +788,18 @@ void fx_enqueue(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t
 }
 
 // The fixed-point path for one call; returns false (the float path runs)
-// when it does not apply (unaligned A) or a column's max over every row is
-// not finite.
+// when a column's max over every row is not finite.  Reading the flags waits
+// for the stream, which a stream under capture cannot: a call whose columns
+// are not 16-byte aligned takes the float path there, as it always has.
 template <int FMT, bool EXACT>
 bool try_apply_fx(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, int64_t s,
                   const uint32_t* packed, char* scratch, const CsLayout& L, double* y, int64_t ldy,
                   hipStream_t st) {
-    if (!vec_ok<FMT>(a, wr, lda, EXACT)) return false;
+    if (!aligned16<FMT>(a, wr, lda, EXACT)) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        TOMOS_HIP_CHECK(hipStreamIsCapturing(st, &cap));
+        if (cap != hipStreamCaptureStatusNone) return false;
+    }
     int* flags = reinterpret_cast<int*>(scratch + L.flag);
     int h[2] = {0, 0};
     auto read_flags = [&]() {
@@ -865,7 +885,7 @@ void countsketch_apply(int a_type, int tier, int64_t m, int64_t n, const void* a
 }
 
 // Many sketches in one call.  Every problem that the fixed-point path takes
-// (16-byte aligned rows, s <= 16384) runs in grouped launches: one index
+// (s <= 16384) runs in grouped launches: one index
 // launch, one exponent launch, one apply launch per column-group width
 // (8, 4, 2, 1 columns, whichever keep a block's int64 buckets within
 // 128 KB of LDS) whose blocks cover every such problem's splits of up to
@@ -892,10 +912,8 @@ bool group_candidate(const tomos_cs_problem& q) {
 bool group_takes(int a_type, bool exact, const tomos_cs_problem& q) {
     if (!group_candidate(q)) return false;
     const bool packed = a_type == TOMOS_FP32_16 || a_type == TOMOS_FP32_BF16;
-    const int v = a_type == TOMOS_F64 ? 2 : a_type == TOMOS_F32 ? 4 : 8;
     if (!packed && a_type != TOMOS_F32 && a_type != TOMOS_F64) return false;
-    if (exact && packed && (!q.wr || reinterpret_cast<uintptr_t>(q.wr) % 16 != 0)) return false;
-    return reinterpret_cast<uintptr_t>(q.a) % 16 == 0 && q.lda % v == 0;
+    return !(exact && packed) || q.wr;
 }
 
 struct GroupLayout {
@@ -1085,7 +1103,12 @@ void countsketch_apply_batched(int a_type, int tier, int nprob, const tomos_cs_p
     if (!hd.empty()) {
         CsGroupDesc* dd = reinterpret_cast<CsGroupDesc*>(sc + L.desc);
         int* downer = reinterpret_cast<int*>(sc + L.owner);
-        const bool ntl = stream_loads(bytes);
+        bool al = true;  // vectors that straddle cache lines are left cacheable
+        const int64_t v = a_type == TOMOS_F64 ? 2 : a_type == TOMOS_F32 ? 4 : 8;
+        for (const CsGroupDesc& d : hd)
+            al = al && d.lda % v == 0 && reinterpret_cast<uintptr_t>(d.a) % 16 == 0 &&
+                 (!exact || reinterpret_cast<uintptr_t>(d.wr) % 16 == 0);
+        const bool ntl = al && stream_loads(bytes);
         switch (a_type) {
             case TOMOS_F32:
                 group_launch<FMT_F32, false>(hd, cg_first, cg_count, blk_first, blk_count, dd, downer, max_m,
