@@ -942,36 +942,32 @@ __device__ __forceinline__ void cq_wave_inv_unit_lower(const double* lo, double*
 }
 
 // LU without pivoting of v (kNB x kNB): lo gets the unit lower factor, up
-// the upper one.  Step i: lane i publishes its column below the pivot (the
-// multipliers before scaling) in bc and writes the scaled multipliers to
-// lo; every lane j > i then subtracts multiplier x U(i, j) from its column.
-__device__ __forceinline__ void cq_wave_lu(const double* v, double* lo, double* up, double* bc) {
+// the upper one.  Step i: lane i's column below the pivot holds the
+// multipliers before scaling; each comes by readlane, is scaled, and every
+// lane j > i subtracts multiplier x U(i, j) from its column.  Lane i's own
+// entries stay as they are, so both factors are written at the end, a row of
+// all lanes at a time.  Bound by latency, 32 dependent steps: through LDS
+// (lane i writing its column entry by entry, then its multipliers) the second
+// small kernel of a 4000 x 1000 sketch took 34.4 us a panel, so 27.0.
+__device__ __forceinline__ void cq_wave_lu(const double* v, double* lo, double* up) {
     const int l = threadIdx.x & 63, j = l & 31;
     double c[kNB];
 #pragma unroll
     for (int i = 0; i < kNB; ++i) c[i] = v[i * kNB + j];
+    double own = 0.0;  // 1 / the lane's pivot
 #pragma unroll
     for (int i = 0; i < kNB; ++i) {
         const double inv = cq_rcp(read_lane(c[i], i));
-        cq_order();
-        if (j == i) {
-#pragma unroll
-            for (int p = i + 1; p < kNB; ++p) bc[p] = c[p];
-        }
-        cq_order();
+        own = j == i ? inv : own;
         const double uij = j > i ? c[i] : 0.0;
 #pragma unroll
-        for (int p = i + 1; p < kNB; ++p) c[p] -= (bc[p] * inv) * uij;
-        if (l == i) {
-#pragma unroll
-            for (int p = i + 1; p < kNB; ++p) lo[p * kNB + i] = bc[p] * inv;
-        }
+        for (int p = i + 1; p < kNB; ++p) c[p] -= (read_lane(c[p], i) * inv) * uij;
     }
     if (l < kNB) {
 #pragma unroll
         for (int i = 0; i < kNB; ++i) {
             up[i * kNB + j] = i <= j ? c[i] : 0.0;
-            if (i <= j) lo[i * kNB + j] = i == j ? 1.0 : 0.0;
+            lo[i * kNB + j] = i > j ? c[i] * own : (i == j ? 1.0 : 0.0);
         }
     }
 }
@@ -1220,7 +1216,7 @@ __global__ __launch_bounds__(kCqT) void qr_cq_small_kernel(const QrDesc* __restr
         B1[e] = (i < nbp && j < nbp) ? B2[e] * sj - (i == j ? 1.0 : 0.0) : (i == j ? 1.0 : 0.0);
     }
     __syncthreads();
-    if (w == 0) cq_wave_lu(B1, B5, B3, bc);  // L1 -> B5, U -> B3
+    if (w == 0) cq_wave_lu(B1, B5, B3);  // L1 -> B5, U -> B3
     __syncthreads();
     if (w == 0) cq_wave_inv_upper(B3, B1);       // U^-1
     if (w == 1) cq_wave_inv_unit_lower(B5, B2);  // L1^-1
