@@ -153,31 +153,50 @@ __global__ __launch_bounds__(kT) void k_beta_finish(LsqrState* s, const double* 
     }
 }
 
-// beta = |u_raw| (as k_beta_finish) and temp[j] = sum_s tsum[s][j] / beta
-// (A^T u from the single-pass kernel's level-1 sums, fixed order) in one
-// launch: every block forms beta from the same partials in the same order,
-// block 0 stores it, and each block scales its columns by its own copy
-__global__ __launch_bounds__(kT) void k_beta_temp_finish(LsqrState* s, const double* __restrict__ red, int nb,
-                                                         int64_t n, int splits, const double* __restrict__ tsum,
-                                                         void* temp, bool t64) {
+// beta = |u_raw| (as k_beta_finish) and temp[j] = (A^T u_raw)_j / beta from
+// the single-pass kernel's block partials (tpart[nblocks][n]) in one launch:
+// every block forms beta from the same partials in the same order (block 0
+// stores it) and adds 32 columns, 32 slices of the partials each, in slice
+// order, FP64.  Latency-bound: as two launches (partials over up to 32
+// splits by a thread per column, then beta and the splits' sums) it took 8.7
+// + 6.2 us at 60000 x 300 with 512 partials; now 7.1.
+constexpr int kBt = 1024, kBtCols = 32, kBtSlices = kBt / kBtCols;
+__global__ __launch_bounds__(kBt) void k_beta_temp(LsqrState* s, const double* __restrict__ red, int nb, int64_t n,
+                                                   int nblocks, const float* __restrict__ tpart, void* temp, bool t64) {
     if (s->done) return;
+    const int col = threadIdx.x % kBtCols, slice = threadIdx.x / kBtCols;
+    const int64_t j = static_cast<int64_t>(blockIdx.x) * kBtCols + col;
+    double a = 0.0;
+    if (j < n)
+        for (int c = slice; c < nblocks; c += 8 * kBtSlices) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                v[u] = c + u * kBtSlices < nblocks ? tpart[static_cast<int64_t>(c + u * kBtSlices) * n + j] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) a += static_cast<double>(v[u]);
+        }
     double acc = 0.0;
-    for (int i = threadIdx.x; i < nb; i += kT) acc += red[i];
+    for (int i = threadIdx.x; i < nb; i += kBt) acc += red[i];
     for (int o = 32; o >= 1; o >>= 1) acc += __shfl_xor(acc, o);
-    __shared__ double w[4];
+    __shared__ double w[kBt / 64];
+    __shared__ double part[kBtSlices][kBtCols + 1];
     if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = acc;
+    part[slice][col] = a;
     __syncthreads();
-    const double b = sqrt((w[0] + w[1]) + (w[2] + w[3]));
+    if (slice != 0) return;
+    double b2 = 0.0;
+    for (int i = 0; i < kBt / 64; ++i) b2 += w[i];
+    const double b = sqrt(b2);
     const double inv_b = 1.0 / b;
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         s->beta = b;
         s->inv_beta = inv_b;
     }
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * kT + threadIdx.x;
     if (j >= n) return;
-    double a = 0.0;
-    for (int sp = 0; sp < splits; ++sp) a += tsum[static_cast<int64_t>(sp) * n + j];
-    st(temp, t64, j, a * inv_b);
+    double t = 0.0;
+    for (int q = 0; q < kBtSlices; ++q) t += part[q][col];
+    st(temp, t64, j, t * inv_b);
 }
 
 constexpr int kTail = 1024;
@@ -298,7 +317,7 @@ __global__ __launch_bounds__(kTail) void k_tail(LsqrState* S, int init, int pre,
 // history, reduction partials and GEMV partial sums.
 struct Layout {
     size_t u, v, w, t, pv, arena_total;
-    size_t state, hist, red, z, tpart, tsum, scratch, scratch_total;
+    size_t state, hist, red, z, tpart, scratch, scratch_total;
     bool fused_possible;
     FusedPlan fplan;
     size_t gemv_bytes;
@@ -351,10 +370,9 @@ Layout layout_for(const tomos_lsqr_options& o, int64_t m, int64_t n) {
                                             L.fused_possible ? lsqr_fused_max_blocks(m) : 0);
     L.red = off; off = align256(off + static_cast<size_t>(red_n) * 8);
     L.z = off; off = align256(off + static_cast<size_t>(n) * 8);  // z = P w (precond type)
-    L.tpart = L.tsum = off;
+    L.tpart = off;
     if (L.fused_possible) {
         L.tpart = off; off = align256(off + lsqr_fused_max_tpart_bytes(m, n));
-        L.tsum = off; off = align256(off + lsqr_fused_max_tsum_bytes(n));
     }
     size_t sc = 0;
     sc = std::max(sc, gemv_scratch_bytes(o.a_type, o.mv_tier, TOMOS_NO_TRANSPOSE, m, n));
@@ -520,10 +538,9 @@ struct Solver {
         }
         if (use_fused_restart) {
             float* tpart = reinterpret_cast<float*>(sc + L.tpart);
-            double* tsum = reinterpret_cast<double*>(sc + L.tsum);
             lsqr_restart_launch(o.a_type, m, n, a, wr, lda, static_cast<const double*>(x), x_zero, U(), v64,
-                                red(), tpart, tsum, rplan, &S->done, s);
-            k_beta_temp_finish<<<grid_for(n), kT, 0, s>>>(S, red(), rplan.nblocks, n, rplan.splits, tsum, Tm(), v64);
+                                red(), tpart, nullptr, rplan, &S->done, s);
+            beta_temp(rplan.nblocks);
             tail(true, true);
             return;
         }
@@ -533,6 +550,12 @@ struct Solver {
         gemv_a(o.restart_tier, TOMOS_NO_TRANSPOSE, cr, x, r64, U(), v64, &nb);
         k_beta_finish<<<1, kT, 0, s>>>(S, red(), nb);
         tail(true);
+    }
+
+    // beta and temp from the single-pass kernels' partials of nblocks blocks
+    void beta_temp(int nblocks) {
+        k_beta_temp<<<static_cast<unsigned>(ceil_div(n, kBtCols)), kBt, 0, s>>>(
+            state(), red(), nblocks, n, nblocks, reinterpret_cast<const float*>(sc + L.tpart), Tm(), v64);
     }
 
     // temp = A^T u = (A^T u_raw) / beta, then (pre) the R^-T chunk partials,
@@ -569,10 +592,8 @@ struct Solver {
         if (use_fused) {
             // one pass over A: u_raw and the A^T u_raw partials together
             lsqr_fused_launch(o.a_type, m, n, a, lda, xin, x64, U(), v64, &S->u_coef, red(),
-                              reinterpret_cast<float*>(sc + L.tpart),
-                              reinterpret_cast<double*>(sc + L.tsum), L.fplan, &S->done, s);
-            k_beta_temp_finish<<<grid_for(n), kT, 0, s>>>(S, red(), L.fplan.nblocks, n, L.fplan.splits,
-                                                         reinterpret_cast<const double*>(sc + L.tsum), Tm(), v64);
+                              reinterpret_cast<float*>(sc + L.tpart), nullptr, L.fplan, &S->done, s);
+            beta_temp(L.fplan.nblocks);
             tail(false, true);
             return;
         }

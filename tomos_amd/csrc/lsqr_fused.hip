@@ -1019,6 +1019,7 @@ void lsqr_fused_launch(int a_type, int64_t m, int64_t n, const void* a, int64_t 
     TOMOS_HIP_CHECK(hipLaunchKernel(k, dim3(static_cast<unsigned>(plan.nblocks)), dim3(plan.threads), args, 0, s));
     TOMOS_LAUNCH_CHECK("lsqr_fused_kernel");
     if (timed) TOMOS_HIP_CHECK(hipEventRecord(g_timer.ev[2 * g_timer.used++ + 1], s));
+    if (!tsum) return;  // the caller adds the block partials itself
     fused_tsum_kernel<<<dim3(static_cast<unsigned>(ceil_div(n, kThreads)), static_cast<unsigned>(plan.splits)),
                         kThreads, 0, s>>>(n, plan.nblocks, plan.splits, tpart, tsum, skip);
     TOMOS_LAUNCH_CHECK("fused_tsum_kernel");
@@ -1082,6 +1083,7 @@ void lsqr_restart_launch(int a_type, int64_t m, int64_t n, const void* a, const 
                     &u, &u64, &tpb, &sumsq, &tpart, const_cast<int**>(&skip)};
     TOMOS_HIP_CHECK(hipLaunchKernel(k, dim3(static_cast<unsigned>(plan.nblocks)), dim3(kRsNT), args, 0, s));
     TOMOS_LAUNCH_CHECK("lsqr_restart_kernel");
+    if (!tsum) return;  // the caller adds the block partials itself
     fused_tsum_kernel<<<dim3(static_cast<unsigned>(ceil_div(n, kThreads)), static_cast<unsigned>(plan.splits)),
                         kThreads, 0, s>>>(n, plan.nblocks, plan.splits, tpart, tsum, skip);
     TOMOS_LAUNCH_CHECK("fused_tsum_kernel");

@@ -45,8 +45,9 @@ void lsqr_fused_config_clear();
 bool lsqr_fused_config_get(int a_type, int64_t n, int* g, int* blocks_per_cu, int* threads);
 
 // u_raw <- A p + (*u_coef) u_raw for all m rows; sumsq[b] = sum of u_raw^2
-// over block b's rows (plan.nblocks entries); tsum[s][j] = sum over the
-// blocks of split s of (A^T u_raw)_j.  Every launch is a no-op when *skip.
+// over block b's rows (plan.nblocks entries); tpart[b][j] = block b's part of
+// (A^T u_raw)_j, and tsum[s][j] = sum over the blocks of split s (not formed
+// when tsum is null).  Every launch is a no-op when *skip.
 void lsqr_fused_launch(int a_type, int64_t m, int64_t n, const void* a, int64_t lda, const void* p,
                        bool p64, void* u, bool u64, const double* u_coef, double* sumsq,
                        float* tpart, double* tsum, const FusedPlan& plan, const int* skip,
