@@ -242,8 +242,7 @@ def batched_leg(args, C, DeviceBuffer, ev0, ev1):
     qp = (C.QrProblem * P)(*[C.QrProblem(p["s"], p["n"], p["s"], p["sk"].ptr) for p in probs])
     qsb = C.lib().tomos_sketch_qr_precond_batched_scratch_size(P, qp)
     qs = DeviceBuffer(qsb)
-    # the whole solve is one graph launch with blind restarts: the restart cap
-    # bounds the launches enqueued (12 x 8 iterations, over twice what C5 needs)
+    # one graph launch per restart; the cap is over twice what C5 needs
     o = C.LsqrOptions(C.FP32_BF16, C.TIER_DEFAULT, C.TIER_EXACT, C.F32, C.F64, C.F64, 1e-6, 1e-6, args.inner,
                       args.batched_restarts, 8, 1, 1)
     lp = (C.LsqProblem * P)(*[C.LsqProblem(p["m"], p["n"], p["lda"], p["wh"].ptr, p["wr"].ptr, p["b"].ptr,
@@ -382,7 +381,7 @@ def batched_leg(args, C, DeviceBuffer, ev0, ev1):
             "adjoint_iterations_max": max(grp_its), "adjoint_iterations_max_one_problem": max(adj_its),
             "gradient_errors_vs_dense_fp64_qr": grad_err,
             "forward": "forward_ms = tomos_countsketch_apply_batched + tomos_sketch_qr_precond_batched_f64 + "
-                       "tomos_lsqr_batched_solve to relres 1e-6 (one graph launch); tomos_amd.autograd.lstsq_batched "
+                       "tomos_lsqr_batched_solve to relres 1e-6 (one graph launch per restart); tomos_amd.autograd.lstsq_batched "
                        "runs the same and, with its default normal_correction, one more batched adjoint solve "
                        "(about backward_ms without the gradients)",
             "backward": "tomos_lsq_adjoint_batched, workers = 0: every problem's adjoint CG (tol %g) in grouped "

@@ -548,10 +548,10 @@ typedef struct {
  * step of all problems is the same few launches whatever their number and
  * shapes: a grouped exact-residual kernel (restarts), the grouped
  * single-pass A p / A^T u kernel and a tail (per-problem scalars, R^-1
- * products spread over many blocks).  With use_graph the whole solve
- * (opt->restarts restarts of 1 + opt->max_iters steps; problems that have
- * stopped exit at once) is captured once per launch configuration and
- * submitted as one graph launch; a NULL stream then runs on a private
+ * products spread over many blocks).  With use_graph a restart (1 +
+ * opt->max_iters steps; problems that have stopped exit at once) is captured
+ * once per launch configuration and submitted as one graph launch, and the
+ * stop flags are read between restarts; a NULL stream then runs on a private
  * stream ordered after earlier NULL-stream work.
  * Options: a_type F32/FP32_16/FP32_BF16, mv_tier DEFAULT, value_type F32,
  * refine_type F64, precond_type F64 (R^-1 required), n <= 2048, 16-byte

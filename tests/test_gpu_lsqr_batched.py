@@ -144,3 +144,28 @@ def test_batched_confirm_off_keeps_estimate_stop(capi):
             assert r < 1e-6
         relres = np.linalg.norm(p["b"] - p["A"].astype(np.float64) @ x) / np.linalg.norm(p["b"])
         assert relres < 5e-6, relres
+
+
+@pytest.mark.parametrize("inner", [1, 5])
+def test_batched_restart_caps_share_graphs(capi, inner):
+    """Restart by restart, one scratch and so the same kept graphs under any
+    cap (none, the first form alone, the later form many times over): each
+    equals plain launches bit for bit, and a cap that the solve does not
+    reach changes nothing."""
+    batch = make_batch(SHAPES[:3], 10)
+    big = opts(C.FP32_BF16, inner=inner, restarts=100)
+    P = (C.LsqProblem * len(batch))(*[
+        C.LsqProblem(p["m"], p["n"], p["lda"], p["wh"].ptr, p["wr"].ptr, p["bd"].ptr, p["xd"].ptr, p["sk"].ptr,
+                     p["s"]) for p in batch])
+    scr = DeviceBuffer(C.lib().tomos_lsqr_batched_scratch_size(ctypes.byref(big), len(batch), P, 0, 0, 0))
+    done = None
+    for cap in (0, 1, 2, 100, 80, 1):  # the slowest problem stops in its 55th restart of one step
+        o = opts(C.FP32_BF16, inner=inner, restarts=cap)
+        xg, itg, rg = solve_batched(batch, o, use_graph=1, scr=scr)
+        xp, itp, rp = solve_batched(batch, o, use_graph=0)
+        assert itg == itp and rg == rp
+        assert all(np.array_equal(a, b) for a, b in zip(xg, xp))
+        assert max(itg) <= cap * inner
+        if cap >= 80:
+            assert done is None or (itg == done[1] and all(np.array_equal(a, b) for a, b in zip(xg, done[0])))
+            done = (xg, itg)

@@ -18,17 +18,20 @@
 // v, the Givens rotation, z = P w and x updates, the stop test and the
 // next p = R^-1 v.  A converged problem's blocks exit at once.
 //
-// The whole solve (state set-up and `restarts` restarts of 1 + max_iters
-// steps, every launch) is captured as one hipGraph, instantiated once per
-// launch configuration and kept, and submitted as ONE graph launch; a
-// stopped problem's blocks exit at once in the launches that follow, and
-// the host synchronizes once at the end.  The grouped kernels' work lists
+// A restart (1 + max_iters steps, every launch; the first with the state
+// set-up) is captured as one hipGraph, instantiated once per launch
+// configuration and kept, and submitted as ONE graph launch; a stopped
+// problem's blocks exit at once in the launches that follow, and the host
+// reads the stop flags between restarts.  The grouped kernels' work lists
 // (tile ranges per block) are built on the host per call and read by the
 // graph from the scratch; their shape (row groups, tiles per block) is a
 // tunable.
 #include <algorithm>
 #include <cmath>
+#include <memory>
 #include <mutex>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "codec.hpp"
@@ -605,24 +608,25 @@ struct Batched {
         return true;
     }
 
-    // Everything a captured solve depends on: the launch grids, the tail's
+    // Everything a captured segment depends on: the launch grids, the tail's
     // LDS, the scalar arguments and the scratch address (the kernels read
     // their problem tables and work lists from the scratch, rewritten by
-    // upload() before every launch).
+    // upload() before every solve), and whether it is the solve's first.
     struct GraphKey {
-        int device, nprob, nitems, nrow_items, g, threads, rounds, a_type, max_iters, restarts, confirm;
+        int device, nprob, nitems, nrow_items, g, threads, rounds, a_type, max_iters, confirm;
         size_t lds;
         double tol, maxrr;
         const void* scratch;
-        bool stream;
+        bool stream, first;
         bool operator==(const GraphKey& k) const {
             return device == k.device && nprob == k.nprob && nitems == k.nitems && nrow_items == k.nrow_items &&
                    g == k.g && threads == k.threads && rounds == k.rounds && a_type == k.a_type &&
-                   max_iters == k.max_iters && restarts == k.restarts && confirm == k.confirm && lds == k.lds &&
-                   tol == k.tol && maxrr == k.maxrr && scratch == k.scratch && stream == k.stream;
+                   max_iters == k.max_iters && confirm == k.confirm && lds == k.lds &&
+                   tol == k.tol && maxrr == k.maxrr && scratch == k.scratch && stream == k.stream &&
+                   first == k.first;
         }
     };
-    GraphKey key() const {
+    GraphKey key(bool first) const {
         GraphKey k;
         TOMOS_HIP_CHECK(hipGetDevice(&k.device));
         k.nprob = nprob;
@@ -633,99 +637,114 @@ struct Batched {
         k.rounds = L.rounds;
         k.a_type = o.a_type;
         k.max_iters = o.max_iters;
-        k.restarts = o.restarts;
         k.confirm = o.confirm;
         k.lds = static_cast<size_t>(tail_nmax());
         k.tol = o.tol;
         k.maxrr = o.max_relres;
         k.scratch = sc;
         k.stream = L.stream;
+        k.first = first;
         return k;
     }
 
-    // The whole solve: state set-up, then `restarts` restart sequences.
-    // Problems that have stopped turn their blocks of the later launches
-    // into immediate exits, so the sequence can run to its end blindly.
-    void solve_sequence() {
-        k_bstate_init<<<static_cast<unsigned>(ceil_div(nprob, 64)), 64, 0, s>>>(dprobs(), nprob);
-        k_batch_setup<<<static_cast<unsigned>(nprob), kTail, 0, s>>>(dprobs());
-        for (int r = 0; r < o.restarts; ++r) restart_sequence(r == 0);
+    // One restart of every problem, after the state set-up for the first one.
+    // Problems that have stopped turn their blocks of the launches into
+    // immediate exits.
+    void segment(bool first) {
+        if (first) {
+            k_bstate_init<<<static_cast<unsigned>(ceil_div(nprob, 64)), 64, 0, s>>>(dprobs(), nprob);
+            k_batch_setup<<<static_cast<unsigned>(nprob), kTail, 0, s>>>(dprobs());
+        }
+        restart_sequence(first);
+        TOMOS_LAUNCH_CHECK("lsqr_batched restart");
     }
 
+    // The segment as a graph, instantiated once per key and kept
+    // (library-wide cache of the last few keys).
+    using SharedGraph = std::shared_ptr<std::remove_pointer_t<hipGraphExec_t>>;
+    SharedGraph segment_graph(bool first) {
+        const GraphKey k = key(first);
+        if (SharedGraph kept = graph_cache_find(k)) return kept;
+        hipGraphExec_t exec = nullptr;
+        hipGraph_t graph = nullptr;
+        TOMOS_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
+        try {
+            segment(first);
+        } catch (...) {
+            hipGraph_t g2 = nullptr;
+            (void)hipStreamEndCapture(s, &g2);
+            if (g2) (void)hipGraphDestroy(g2);
+            throw;
+        }
+        TOMOS_HIP_CHECK(hipStreamEndCapture(s, &graph));
+        const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(graph);
+        TOMOS_HIP_CHECK(e);
+        SharedGraph made(exec, [](hipGraphExec_t x) { (void)hipGraphExecDestroy(x); });
+        graph_cache_insert(k, made);
+        return made;
+    }
+
+    // Restart by restart until every problem has stopped.  A solve whose
+    // restarts were all enqueued blindly ended in five empty launches a step
+    // (20 problems up to 200000 x 512, a cap of 40 restarts of 30 steps, all
+    // stopped in the third: about 5700 launches; forward and backward 89.4 ms
+    // so, 77.3 ms with the flags read between restarts) and captured as many
+    // nodes for every new scratch.
     void run(bool use_graph, int* iterations, double* final_relres) {
         upload();
         std::vector<BState> h(nprob);
-        if (use_graph && o.restarts > 0) {
-            // one graph launch for the whole solve, instantiated once per key
-            // and kept (library-wide cache of the last few keys)
-            hipGraphExec_t exec = graph_cache_find(key());
-            if (!exec) {
-                hipGraph_t graph = nullptr;
-                TOMOS_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-                try {
-                    solve_sequence();
-                } catch (...) {
-                    hipGraph_t g2 = nullptr;
-                    (void)hipStreamEndCapture(s, &g2);
-                    if (g2) (void)hipGraphDestroy(g2);
-                    throw;
-                }
-                TOMOS_HIP_CHECK(hipStreamEndCapture(s, &graph));
-                const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-                (void)hipGraphDestroy(graph);
-                TOMOS_HIP_CHECK(e);
-                graph_cache_insert(key(), exec);
+        SharedGraph graphs[2];  // held until the solve has synchronized
+        for (int r = 0; r < o.restarts; ++r) {
+            if (r > 0 && all_done(h)) break;
+            if (use_graph) {
+                SharedGraph& graph = graphs[r == 0 ? 0 : 1];
+                if (!graph) graph = segment_graph(r == 0);
+                TOMOS_HIP_CHECK(hipGraphLaunch(graph.get(), s));
+                TOMOS_LAUNCH_CHECK("lsqr_batched graph");
+            } else {
+                segment(r == 0);
             }
-            TOMOS_HIP_CHECK(hipGraphLaunch(exec, s));
-            TOMOS_LAUNCH_CHECK("lsqr_batched graph");
-            all_done(h);
-        } else {
+        }
+        if (o.restarts <= 0) {
             k_bstate_init<<<static_cast<unsigned>(ceil_div(nprob, 64)), 64, 0, s>>>(dprobs(), nprob);
             k_batch_setup<<<static_cast<unsigned>(nprob), kTail, 0, s>>>(dprobs());
             TOMOS_LAUNCH_CHECK("lsqr_batched setup");
-            for (int r = 0; r < o.restarts; ++r) {
-                if (all_done(h)) break;
-                restart_sequence(r == 0);
-                TOMOS_LAUNCH_CHECK("lsqr_batched restart");
-            }
-            all_done(h);
         }
+        all_done(h);
         for (int i = 0; i < nprob; ++i) {
             if (iterations) iterations[i] = h[i].completed;
             if (final_relres) final_relres[i] = h[i].rhsnorm > 0 ? std::fabs(h[i].phi_bar) / h[i].rhsnorm : 0.0;
         }
     }
 
-    // Library-wide cache of instantiated solve graphs (a few keys, oldest
-    // evicted).  Every solve synchronizes before it returns, so an evicted
-    // graph is not running.
-    static constexpr int kGraphCache = 8;
+    // Library-wide cache of instantiated segment graphs (a few keys, oldest
+    // evicted; a solve that still runs an evicted graph holds its own share).
+    static constexpr int kGraphCache = 16;  // two a solve
     struct CacheEntry {
         GraphKey key;
-        hipGraphExec_t exec;
+        SharedGraph exec;
     };
     static std::vector<CacheEntry>& cache() {
-        static std::vector<CacheEntry> c;
-        return c;
+        // never destroyed: at exit the HIP runtime may be gone before it
+        static auto* c = new std::vector<CacheEntry>;
+        return *c;
     }
     static std::mutex& cache_mutex() {
         static std::mutex m;
         return m;
     }
-    static hipGraphExec_t graph_cache_find(const GraphKey& k) {
+    static SharedGraph graph_cache_find(const GraphKey& k) {
         std::lock_guard<std::mutex> lock(cache_mutex());
         for (const CacheEntry& e : cache())
             if (e.key == k) return e.exec;
         return nullptr;
     }
-    static void graph_cache_insert(const GraphKey& k, hipGraphExec_t exec) {
+    static void graph_cache_insert(const GraphKey& k, SharedGraph exec) {
         std::lock_guard<std::mutex> lock(cache_mutex());
         auto& c = cache();
-        if (static_cast<int>(c.size()) >= kGraphCache) {
-            (void)hipGraphExecDestroy(c.front().exec);
-            c.erase(c.begin());
-        }
-        c.push_back(CacheEntry{k, exec});
+        if (static_cast<int>(c.size()) >= kGraphCache) c.erase(c.begin());
+        c.push_back(CacheEntry{k, std::move(exec)});
     }
 };
 
