@@ -169,3 +169,17 @@ def test_batched_restart_caps_share_graphs(capi, inner):
         if cap >= 80:
             assert done is None or (itg == done[1] and all(np.array_equal(a, b) for a, b in zip(xg, done[0])))
             done = (xg, itg)
+
+
+@pytest.mark.parametrize("tiles", [1, 2])
+def test_batched_partial_totals_edges(capi, tiles):
+    """The tail's column totals: one column, the edges of its 64-column
+    blocks, and 64-row tile counts around its 16 slices and 8 loads in
+    flight (15, 16, 17, 128, 129 and 150 items at one tile an item)."""
+    shapes = [(15 * 64, 1, 0), (16 * 64, 63, 1), (17 * 64 - 3, 64, 1), (128 * 64, 65, 1), (129 * 64, 128, 1),
+              (150 * 64 - 1, 129, 1)]
+    batch = make_batch(shapes, 11)
+    xs, its, _ = solve_batched(batch, opts(C.FP32_BF16), tiles=tiles)
+    for p, x, it in zip(batch, xs, its):
+        relres = np.linalg.norm(p["b"] - p["A"].astype(np.float64) @ x) / np.linalg.norm(p["b"])
+        assert relres <= TRUE_TOL and it < 120, (p["m"], p["n"], relres, it)

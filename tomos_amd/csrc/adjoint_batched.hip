@@ -9,15 +9,16 @@
 // grouped is the launch:
 //   iteration: the grouped single-pass kernel (the batched LSQR solver's,
 //              u = A d with a zero u coefficient, A^T u per tile range, |u|^2
-//              per tile range) for all iterating problems, then one
-//              1024-thread block per problem for the n-sized work: alpha =
-//              rho/|q|^2, w += alpha d, res -= alpha A^T q, the stop test;
+//              per tile range) for all iterating problems, then the n-sized
+//              work in 1024-thread blocks: alpha = rho/|q|^2, w += alpha d, res -= alpha A^T q (64 columns a
+//              block), the stop test (one block per problem);
 //              then, over many blocks per problem, y = R^-T res (a wave per
 //              column) and z = R^-1 y (64 rows a block), and one block per
 //              problem for rho' = res.z, d = z + (rho'/rho) d;
 //   restart:   A^T (A w) at the exact tier for every restarting problem
 //              (one grouped launch over row items; a per-problem GEMV pair
-//              when some n > 1024), then one block per problem: res,
+//              when some n > 1024), the row items added 64 columns
+//              a block), then one block per problem: res,
 //              |res|/|g|, the stop test; z, rho and d = z as in a step.
 // Each problem carries a small state machine on the device (restart
 // pending -> iterating -> restart pending ... -> done), so the host never
@@ -42,6 +43,7 @@
 #include "common.hpp"
 #include "gemv.hpp"
 #include "lsqr_fused.hpp"
+#include "partials.hpp"
 #include "tomos_hip.h"
 
 namespace tomos_hip {
@@ -585,6 +587,17 @@ __global__ __launch_bounds__(kRx2Threads) void k_gadj_grad(const GGrad* __restri
     else run(std::integral_constant<int, 8>{});
 }
 
+// rfull = A^T A w from the exact restart's row-item partials, 64 columns a
+// block.  (Added by k_gadj_restart with one block a problem: 38 us there on
+// average over 26 restarts, against 4.8 us here and 4.3 us there now.)
+__global__ __launch_bounds__(kPartThreads) void k_gadj_rx_sum(const GProb* __restrict__ P) {
+    const GProb& p = P[blockIdx.y];
+    const int64_t col0 = static_cast<int64_t>(blockIdx.x) * kPartCols;
+    if (p.st->phase != kPhaseRestart || p.st->restarts_done == 0 || col0 >= p.n) return;
+    const double t = column_total(p.rpart, p.nrx, p.n, col0);
+    if (threadIdx.x < kPartCols && col0 + threadIdx.x < p.n) p.rfull[col0 + threadIdx.x] = t;
+}
+
 // Restart of every problem whose phase is kPhaseRestart: res = g - rfull
 // (rfull = A^T A w, or nothing on the first restart), |g| on the first, the
 // exact-residual stop test (the restart after `max_restarts` earlier ones is
@@ -598,15 +611,7 @@ __global__ __launch_bounds__(kTail) void k_gadj_restart(const GProb* __restrict_
     const bool first = k == 0;
     double gg = 0.0, rr = 0.0;
     for (int64_t j = threadIdx.x; j < p.n; j += kTail) {
-        double rf = 0.0;
-        if (!first) {
-            if (p.nrx > 0) {
-                for (int k2 = 0; k2 < p.nrx; ++k2) rf += p.rpart[static_cast<int64_t>(k2) * p.n + j];
-            } else {
-                rf = p.rfull[j];
-            }
-        }
-        const double rj = p.g[j] - rf;
+        const double rj = p.g[j] - (first ? 0.0 : p.rfull[j]);
         p.res[j] = rj;
         gg += p.g[j] * p.g[j];
         rr += rj * rj;
@@ -633,28 +638,40 @@ __global__ __launch_bounds__(kTail) void k_gadj_restart(const GProb* __restrict_
 // grouped single-pass kernel left |q|^2 and A^T q as per-item partials.
 // The restart's inner loop ends when |res|/|g| < tol, |q| = 0 or after
 // max_iters steps; the problem then waits for its next restart.
+// The step's n-sized part, 64 columns a block: alpha = rho / |A d|^2, w += alpha
+// d, res -= alpha A^T A d from the grouped pass's partials.  (With one block a
+// problem in k_gadj_step, 50-80 us there for 20 problems up to 200000 x 512;
+// 10 us here and 5 us there now.)
+__global__ __launch_bounds__(kTail) void k_gadj_step_cols(const GProb* __restrict__ P) {
+    static_assert(kTail == kPartThreads, "column_total's block");
+    const GProb& p = P[blockIdx.y];
+    const int64_t n = p.n, col0 = static_cast<int64_t>(blockIdx.x) * kPartCols;
+    if (p.st->phase != kPhaseIterate || col0 >= n) return;
+    __shared__ double sh[kTail / 64];
+    double q2 = 0.0;
+    for (int k = threadIdx.x; k < p.nitems; k += kTail) q2 += p.sumsq[k];
+    q2 = gsum(q2, sh);
+    const double alpha = q2 > 0.0 ? p.st->rho / q2 : 0.0;
+    const double t = column_total(p.tpart, p.nitems, n, col0);
+    const int64_t j = col0 + threadIdx.x;
+    if (threadIdx.x >= kPartCols || j >= n) return;
+    p.w[j] += alpha * p.d[j];
+    p.res[j] -= alpha * t;
+}
+
+// Scalars of the step and its stop test.
 __global__ __launch_bounds__(kTail) void k_gadj_step(const GProb* __restrict__ P, double tol, int max_iters,
                                                     double drop) {
     const GProb& p = P[blockIdx.x];
     GState* S = p.st;
     if (S->phase != kPhaseIterate) return;
     __shared__ double sh[kTail / 64];
-    const double rho = S->rho;
     const int iters = S->iters;
     const int64_t n = p.n;
-    double q2 = 0.0;
+    double q2 = 0.0, rr = 0.0;
     for (int k = threadIdx.x; k < p.nitems; k += kTail) q2 += p.sumsq[k];
     q2 = gsum(q2, sh);
-    const double alpha = q2 > 0.0 ? rho / q2 : 0.0;
-    double rr = 0.0;
-    for (int64_t j = threadIdx.x; j < n; j += kTail) {
-        double t = 0.0;
-        for (int k = 0; k < p.nitems; ++k) t += static_cast<double>(p.tpart[static_cast<int64_t>(k) * n + j]);
-        p.w[j] += alpha * p.d[j];
-        const double rj = p.res[j] - alpha * t;
-        p.res[j] = rj;
-        rr += rj * rj;
-    }
+    for (int64_t j = threadIdx.x; j < n; j += kTail) rr += p.res[j] * p.res[j];
     rr = gsum(rr, sh);
     if (threadIdx.x == 0) {
         S->completed += 1;
@@ -1015,6 +1032,9 @@ struct Grouped {
                 else if (o.a_type == TOMOS_F32) k_gadj_rx<0><<<nb, kRxThreads, 0, s>>>(dprobs(), d);
                 else if (o.a_type == TOMOS_FP32_BF16) k_gadj_rx<1><<<nb, kRxThreads, 0, s>>>(dprobs(), d);
                 else k_gadj_rx<2><<<nb, kRxThreads, 0, s>>>(dprobs(), d);
+                k_gadj_rx_sum<<<dim3(static_cast<unsigned>(ceil_div(L.nmax, static_cast<int64_t>(kPartCols))),
+                                     static_cast<unsigned>(nprob)),
+                                kPartThreads, 0, s>>>(dprobs());
                 TOMOS_LAUNCH_CHECK("k_gadj_rx");
             }
             k_gadj_restart<<<static_cast<unsigned>(nprob), kTail, 0, s>>>(dprobs(), o.tol, o.restarts);
@@ -1056,6 +1076,9 @@ struct Grouped {
         for (int it = 0; it < kSegIters; ++it) {
             if (L.nitems)
                 grouped_fused_launch(o.a_type, L.g, L.threads, L.rounds, dgprobs(), ditems(), L.nitems, s, L.stream);
+            k_gadj_step_cols<<<dim3(static_cast<unsigned>(ceil_div(L.nmax, static_cast<int64_t>(kPartCols))),
+                                    static_cast<unsigned>(nprob)),
+                               kTail, 0, s>>>(dprobs());
             k_gadj_step<<<static_cast<unsigned>(nprob), kTail, 0, s>>>(dprobs(), o.tol, o.max_iters,
                                                                       adjoint_inner_drop(o));
             precond_seq();
