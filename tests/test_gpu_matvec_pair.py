@@ -155,3 +155,22 @@ def test_kernel_timer_counts_single_pass_launches(capi):
     # no timer running: end is an error, begin rejects a bad capacity
     assert C.lib().tomos_kernel_timer_end(dur.ctypes.data, 8, ctypes.byref(cnt)) != 0
     assert C.lib().tomos_kernel_timer_begin(0) != 0
+
+
+@pytest.mark.parametrize("a_type", [C.F32, C.FP32_BF16, C.FP32_16])
+@pytest.mark.parametrize("m,n,threads", [(3001, 256, 256), (3001, 257, 512), (3001, 512, 512), (280000, 500, 0)])
+def test_default_shape_edges(capi, a_type, m, n, threads):
+    """The untuned shape at the edges of its rule on n, bit for bit the
+    explicit one of that many threads; above 256 MiB (280000 x 500 in 16
+    bits) the bf16 planes keep 256 threads, the other types take 512."""
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((m, n), dtype=np.float32).T.reshape(m, n, order="F") if m > 10000 else \
+        rng.standard_normal((m, n)).astype(np.float32, order="F")
+    lda, p, u0 = (m + 7) // 8 * 8, rng.standard_normal(n), rng.standard_normal(m).astype(np.float32)
+    got = run_pair(a_type, A, lda, p, u0, 0.5)
+    C.call("tomos_fused_config_set", a_type, n, 8, 0, threads or (256 if a_type == C.FP32_BF16 else 512))
+    try:
+        want = run_pair(a_type, A, lda, p, u0, 0.5)
+    finally:
+        C.call("tomos_fused_config_clear")
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]) and got[2] == want[2]

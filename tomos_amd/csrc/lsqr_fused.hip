@@ -935,15 +935,25 @@ FusedPlan lsqr_fused_plan(int a_type, int64_t m, int64_t n, int g, int blocks_pe
     FusedPlan p;
     if (g <= 0 && blocks_per_cu <= 0 && threads <= 0) lsqr_fused_config_get(a_type, n, &g, &blocks_per_cu, &threads);
     if (threads <= 0) threads = 256;
+    const int64_t bytes = std::max<int64_t>(m, 1) * n * (a_type == TOMOS_F32 ? 4 : 2);
     if (g <= 0 || rounds_for(g, threads, n) == 0) {
         const FusedShape d = lsqr_fused_default_shape(n);
         g = d.g;
         threads = d.threads;
+        // Between 256 and 512 columns twice the threads halve each wave's
+        // rounds: faster except where the pass is bound by streaming bf16
+        // rows from HBM (more than the 256 MiB last-level cache holds).  us per pass, 256 / 512 threads: FP32_BF16
+        // 20000 x 400 22.5 / 18.2, 60000 x 300 30.6 / 24.7, 200000 x 512
+        // 53.3 / 50.3, but 700000 x 300 106 / 110.5 and 700000 x 512 130 /
+        // 137; FP32_16 60000 x 300 39.6 / 34.5, 700000 x 300 250 / 212.
+        // Up to 256 columns 256 threads (700000 x 130 60.6 / 96.4).
+        const bool bf16 = a_type == TOMOS_FP32_BF16 || a_type == TOMOS_BF16;
+        if (n > 256 && n <= 512 && !(bf16 && bytes > (int64_t{256} << 20))) threads = 512;
     }
     p.g = g;
     p.threads = threads;
     p.rounds = rounds_for(g, threads, n);
-    p.stream = stream_loads(std::max<int64_t>(m, 1) * n * (a_type == TOMOS_F32 ? 4 : 2));
+    p.stream = stream_loads(bytes);
     if (blocks_per_cu <= 0) {
         // as many blocks as fit on the device at once: one wave of blocks
         int occ = 0;
