@@ -155,6 +155,12 @@ int tomos_convert(int src_type, int dst_type, int64_t rows, int64_t cols, const 
 int tomos_pack(int variant, int64_t m, int64_t n, const float* src, int64_t ld_src,
                uint16_t* wh, uint16_t* wr, int64_t ld_dst, tomos_stream_t stream);
 
+/* The same planes from a row-major source: element (i, j) at src[i ld_src + j],
+ * ld_src >= n (the layout of a contiguous torch matrix), without a
+ * transposed copy. */
+int tomos_pack_rows(int variant, int64_t m, int64_t n, const float* src, int64_t ld_src,
+                    uint16_t* wh, uint16_t* wr, int64_t ld_dst, tomos_stream_t stream);
+
 /* Replaces cuda::combine_dense_fp32_16 (fp32_16_cuda_kernels.cu:301-323)
  * for every FP32-producing decoder above.  wr may be NULL for the wh-only
  * decoders. */

@@ -4,6 +4,8 @@ Inputs: a strided sweep of 2^26 fp32 bit patterns (every 64-pattern block of
 the 2^32 space, every exponent, signs, zeros, subnormals, Inf, NaN) plus all
 2^16 wh words for the wh-only decoders.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -125,3 +127,32 @@ def test_unpack_runs_and_remainders(capi, orc, m, n, pad):
             exp = orc.unpack(dec, eh, er)
             assert np.array_equal(got[:m].view(np.uint32), np.ascontiguousarray(exp).astype(np.float32).view(np.uint32)), dec
             assert np.all(got[m:] == -7.0)
+
+
+@pytest.mark.parametrize("m,n,pad_src,pad_dst,shift", [(1, 1, 0, 0, 0), (7, 65, 0, 3, 1), (128, 64, 0, 0, 0),
+                                                        (129, 63, 5, 7, 2), (127, 66, 1, 1, 3), (300, 3, 0, 4, 1),
+                                                        (260, 200, 2, 0, 0)])
+def test_pack_rows_equals_pack(capi, orc, m, n, pad_src, pad_dst, shift):
+    """A row-major source packs to the same words as its columns, at tile
+    edges and remainders, odd leading dimensions and a source at any element;
+    nothing is written past row m or column n."""
+    rng = np.random.default_rng(m * n)
+    A = (rng.standard_normal((m, n)) * 2.0 ** rng.integers(-34, 34, (m, n))).astype(np.float32)
+    A.flat[::7] = rng.choice(np.array([0.0, -0.0, np.inf, -np.inf, np.nan, 1e-45, 65520.0], np.float32), A.flat[::7].size)
+    lds, ld = n + pad_src, m + pad_dst
+    flat = np.full(shift + m * lds, 3.0, np.float32)
+    flat[shift:].reshape(m, lds)[:, :n] = A
+    src = H.dev(flat)
+    cols = H.dev(np.asfortranarray(A))
+    for variant in range(5):
+        print("pack_rows", variant, m, n, lds, ld, shift, flush=True)
+        outs = []
+        for entry in ("tomos_pack_rows", "tomos_pack"):
+            wh, wr = (H.dev(np.full(ld * (n + 1), 0x1234, np.uint16)) for _ in range(2))
+            rows = entry == "tomos_pack_rows"
+            C.call(entry, variant, m, n, src.ptr + 4 * shift if rows else cols.ptr, lds if rows else m, wh.ptr, wr.ptr,
+                   ld, None)
+            outs.append([x.to_numpy(np.uint16, (ld * (n + 1),)) for x in (wh, wr)])
+        assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1]), variant
+    assert C.lib().tomos_pack_rows(0, m, n, ctypes.c_void_p(src.ptr), n - 1, ctypes.c_void_p(src.ptr),
+                                   ctypes.c_void_p(src.ptr), ld, None) == 1

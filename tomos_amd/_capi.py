@@ -94,6 +94,7 @@ _SIGS = {
     "tomos_fill_normal_f32": (cint, [vp, i64, i64, i64, ctypes.c_uint64, vp, cint, cint, vp]),
     "tomos_convert": (cint, [cint, cint, i64, i64, vp, i64, vp, i64, vp]),
     "tomos_pack": (cint, [cint, i64, i64, vp, i64, vp, vp, i64, vp]),
+    "tomos_pack_rows": (cint, [cint, i64, i64, vp, i64, vp, vp, i64, vp]),
     "tomos_unpack": (cint, [cint, i64, i64, vp, vp, i64, vp, i64, vp]),
     "tomos_decode_wh": (cint, [cint, i64, vp, vp, vp]),
     "tomos_gemv_scratch_size": (sz, [cint, cint, cint, i64, i64]),

@@ -79,11 +79,17 @@ class PackedProblem:
         # of every column, which then start on cache lines (16 bytes is the
         # minimum; a 64-byte offset made the batched passes fetch ~1.4x)
         self.ld = (m + 63) // 64 * 64
-        acm = A.t().contiguous()    # (n, m) row-major == column-major (m, n)
         self.wh = torch.empty(self.ld * n, dtype=torch.int16, device=dev)
         self.wr = torch.empty(self.ld * n, dtype=torch.int16, device=dev)
         s = _stream()
-        C.call("tomos_pack", C.PACK_FP32_BF16, m, n, _p(acm), m, _p(self.wh), _p(self.wr), self.ld, s)
+        # rows in order are packed as they are; any other layout (and a lazy
+        # negation, which is not in the memory) goes through a column-major copy
+        if A.stride(1) == 1 and A.stride(0) >= n and not A.is_neg():
+            C.call("tomos_pack_rows", C.PACK_FP32_BF16, m, n, _p(A), A.stride(0), _p(self.wh), _p(self.wr),
+                   self.ld, s)
+        else:
+            acm = A.t().contiguous()    # (n, m) row-major == column-major (m, n)
+            C.call("tomos_pack", C.PACK_FP32_BF16, m, n, _p(acm), m, _p(self.wh), _p(self.wr), self.ld, s)
         self.s_rows = max(opts.sketch_factor * n, n)
         self.sketch = torch.empty((n, self.s_rows), dtype=torch.float64, device=dev)
         if precondition:
