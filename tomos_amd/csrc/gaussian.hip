@@ -16,8 +16,9 @@
 // u1 = (b + 1/2) 2^-23 in (0, 1), bits 8..31 give u2 = b 2^-24 in [0, 1),
 // and the Box-Muller transform (Box & Muller 1958) turns them into two
 // independent normals r cos(2 pi u2), r sin(2 pi u2), r = sqrt(-2 ln u1).
-// The transform runs in FP32 (device logf, sqrtf, sincospif), the way the
-// reference computes its values in float before the cast.  The output
+// The transform runs in FP32 (logarithm, root, sine and cosine of exactly
+// these arguments, below), the way the reference computes its values in
+// float before the cast.  The output
 // type's conversion rounds to nearest even.
 //
 // Roofline: each entry is written once and nothing is read, so the kernel

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(256) void pack_kernel(int64_t m, const float* __res
 // as (h, r) words and written along the columns (256 bytes of each plane).
 // HBM-bound like
 // pack_kernel, in place of a transposed copy and a pack of it (20 matrices
-// up to 200000 x 512, on average: 368 + 39 us so, 68 us here, 3.2 TB/s).
+// up to 200000 x 512, on average: 368 + 39 us so, 68 us here, 3.7 TB/s).
 constexpr int kTileRows = 128, kTileCols = 64;
 // Odd: the words that a wave stores at a step (one column of each 4, 16 lanes
 // a row, 4 rows) hit 64 different banks, those that it loads (every eighth
