@@ -329,3 +329,60 @@ def test_transpose_tiles(capi, vt, it, m, n, mean, long_row):
     assert np.array_equal(pt_.to_numpy(idt, (n + 1,)), np.concatenate([[0], np.cumsum(np.bincount(ci, minlength=n))]))
     assert np.array_equal(it_.to_numpy(idt, (nnz,)), rows[order])
     assert np.array_equal(vt_.to_numpy(bits.dtype, (nnz,)), bits[order])
+
+
+def _count_cells(m, n, nnz, panel_rows):
+    """32-bit words of the counting transpose: a count per column of every row
+    tile (about nnz / 512 entries, 1024..6144) and of every 64 tiles."""
+    def up(a, b):
+        return -(-a // b)
+    panels, want = up(m, panel_rows), min(max(nnz // 512, 1024), 6144)
+    rows = min(min(max(int(want / max(nnz / m, 1e-3)), 1), 2048), panel_rows)
+    tiles = up(min(panel_rows, m), rows)
+    return panels, panels * tiles * n, panels * up(tiles, 64) * n
+
+
+@pytest.mark.parametrize("it", [C.INDEX_INT32, C.INDEX_INT64])
+def test_mv_scratch_holds_either_x_type(capi, it):
+    """The advertised scratch of A^T x holds the transpose's working space for
+    FP32 and FP64 x: the number of panels differs, and the space, rounded up
+    per panel, is not always larger with more of them."""
+    rng = np.random.default_rng(5)
+    shapes = [(18466, 1295, 1000943), (20625, 500, 130392)]
+    shapes += [(int(m), int(n), int(m * k)) for m, n, k in zip(np.exp(rng.uniform(np.log(100), np.log(3e6), 3000)),
+                                                               rng.integers(1, 2049, 3000), rng.uniform(0.1, 60, 3000))]
+    ib = 8 if it == C.INDEX_INT64 else 4
+    for m, n, nnz in shapes:
+        size = C.lib().tomos_csr_mv_scratch_size(C.F32, it, 1, m, n, nnz)
+        for xb in (4, 8):
+            pr = 65536 // xb
+            pr = m if m <= pr else -(-m // -(-m // pr))
+            panels, cells, groups = _count_cells(m, n, nnz, pr)
+            need = nnz * 4 + nnz * ib + (panels * n + 1) * ib + 4 * (cells + groups)
+            assert size >= need, (m, n, nnz, xb, size, need)
+
+
+@pytest.mark.parametrize("xt", [C.F32, C.F64])
+@pytest.mark.parametrize("m,n,nnz", [(18466, 1295, 1000943), (20625, 500, 130392)])
+def test_mv_transposed_stays_in_scratch(capi, xt, m, n, nnz):
+    """A^T x in a scratch of exactly the advertised size, between guard bytes,
+    at shapes where FP32 x has fewer panels and the larger working space."""
+    rng = np.random.default_rng(n)
+    rp = np.concatenate([[0], np.sort(rng.integers(0, nnz + 1, m - 1)), [nnz]]).astype(np.int32)
+    ci, v = rng.integers(0, n, nnz).astype(np.int32), rng.standard_normal(nnz).astype(np.float32)
+    xdt = np.float32 if xt == C.F32 else np.float64
+    x = rng.standard_normal(m).astype(xdt)
+    size, guard = C.lib().tomos_csr_mv_scratch_size(C.F32, C.INDEX_INT32, 1, m, n, nnz), 1 << 16
+    assert size % 256 == 0
+    sc = H.dev(np.full(guard + size + guard, 0xA5, np.uint8))
+    rpd, cid, vd, xd, yd = H.dev(rp), H.dev(ci), H.dev(v), H.dev(x), C.DeviceBuffer(n * 8)
+    print("csr mv T", xt, m, n, nnz, flush=True)
+    C.call("tomos_csr_mv", C.F32, C.INDEX_INT32, 1, 1.0, m, n, nnz, vd.ptr, rpd.ptr, cid.ptr, xt, xd.ptr, 0.0, C.F64,
+           yd.ptr, sc.ptr + guard, size, None)
+    raw = sc.to_numpy(np.uint8, (guard + size + guard,))
+    assert np.all(raw[:guard] == 0xA5) and np.all(raw[guard + size:] == 0xA5)
+    ref, scale = np.zeros(n), np.zeros(n)
+    p = v.astype(np.float64) * x[np.repeat(np.arange(m), np.diff(rp))]
+    np.add.at(ref, ci, p)
+    np.add.at(scale, ci, np.abs(p))
+    assert np.all(np.abs(yd.to_numpy(np.float64, (n,)) - ref) <= 1e-13 * scale)

@@ -1268,6 +1268,26 @@ CsrMat make_csr(int val_type, int idx_type, int64_t m, int64_t n, int64_t nnz, c
     A.col_idxs = ci;
     return A;
 }
+
+// Scratch of A^T x: A^T by panels, then the working space that the transpose
+// and the product use one after the other.
+struct TmvLayout {
+    int64_t panel_rows, panels;
+    size_t vals, idx, ptr, work, total;
+};
+TmvLayout tmv_layout(const CsrMat& A, int x_type) {
+    TmvLayout L;
+    L.panel_rows = csr_panel_rows(A, x_type);
+    L.panels = csr_panels(A, L.panel_rows);
+    const size_t e = static_cast<size_t>(std::max<int64_t>(A.nnz, 1));
+    const CsrMat T = make_csr(A.val_type, A.idx_type, L.panels * A.n, A.m, A.nnz, nullptr, nullptr, nullptr);
+    L.vals = 0;
+    L.idx = align256(e * csr_value_bytes(A.val_type));
+    L.ptr = L.idx + align256(e * csr_index_bytes(A.idx_type));
+    L.work = L.ptr + align256(static_cast<size_t>(L.panels * A.n + 1) * csr_index_bytes(A.idx_type));
+    L.total = L.work + std::max(csr_transpose_scratch_bytes(A, L.panel_rows), csr_tmv_scratch_bytes(T, L.panels, A.n));
+    return L;
+}
 }  // namespace
 
 extern "C" {
@@ -1314,13 +1334,9 @@ size_t tomos_csr_mv_scratch_size(int val_type, int idx_type, int trans, int64_t 
     const CsrMat A = make_csr(val_type, idx_type, m, n, nnz, nullptr, nullptr, nullptr);
     if (!trans) return std::max<size_t>(256, csr_mv_scratch_bytes(A));
     try {
-        // sized for FP64 x: the most panels
-        const int64_t pr = csr_panel_rows(A, TOMOS_F64), panels = csr_panels(A, pr);
-        const CsrMat T = make_csr(val_type, idx_type, panels * n, m, nnz, nullptr, nullptr, nullptr);
-        const size_t e = static_cast<size_t>(std::max<int64_t>(nnz, 1));
-        return align256(e * csr_value_bytes(val_type)) + align256(e * csr_index_bytes(idx_type)) +
-               align256(static_cast<size_t>(panels * n + 1) * csr_index_bytes(idx_type)) +
-               std::max(csr_transpose_scratch_bytes(A, pr), csr_tmv_scratch_bytes(T, panels, n));
+        // for either type of x: FP64 x has more panels, but the transpose's
+        // working space is rounded up per panel and may be larger with fewer
+        return std::max(tmv_layout(A, TOMOS_F64).total, tmv_layout(A, TOMOS_F32).total);
     } catch (...) {
         return 0;
     }
@@ -1349,18 +1365,14 @@ int tomos_csr_mv(int val_type, int idx_type, int trans, double alpha, int64_t m,
         // A^T x: transpose into scratch, then the row kernels on A^T
         csr_check(A, scratch, scratch_bytes, st);
         require(x_type == TOMOS_F32 || x_type == TOMOS_F64, "tomos_csr_mv: x must be F32 or F64");
-        const int64_t pr = csr_panel_rows(A, x_type), panels = csr_panels(A, pr);
-        const size_t e = static_cast<size_t>(std::max<int64_t>(nnz, 1));
+        const TmvLayout L = tmv_layout(A, x_type);
+        require(scratch_bytes >= L.work, "tomos_csr_mv: scratch too small");
         char* sc = static_cast<char*>(scratch);
-        void* vt = sc;
-        sc += align256(e * csr_value_bytes(val_type));
-        void* it = sc;
-        sc += align256(e * csr_index_bytes(idx_type));
-        void* pt = sc;
-        sc += align256(static_cast<size_t>(panels * n + 1) * csr_index_bytes(idx_type));
-        csr_transpose(A, pr, vt, pt, it, sc, csr_transpose_scratch_bytes(A, pr), st);
-        const CsrMat T = make_csr(val_type, idx_type, panels * n, m, nnz, vt, pt, it);
-        csr_tmv(T, panels, pr, n, c, x_type, x, y_type, y, sc, csr_tmv_scratch_bytes(T, panels, n), st);
+        void* work = sc + L.work;
+        const size_t work_bytes = scratch_bytes - L.work;
+        csr_transpose(A, L.panel_rows, sc + L.vals, sc + L.ptr, sc + L.idx, work, work_bytes, st);
+        const CsrMat T = make_csr(val_type, idx_type, L.panels * n, m, nnz, sc + L.vals, sc + L.ptr, sc + L.idx);
+        csr_tmv(T, L.panels, L.panel_rows, n, c, x_type, x, y_type, y, work, work_bytes, st);
     });
 }
 
