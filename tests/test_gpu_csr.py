@@ -386,3 +386,31 @@ def test_mv_transposed_stays_in_scratch(capi, xt, m, n, nnz):
     np.add.at(ref, ci, p)
     np.add.at(scale, ci, np.abs(p))
     assert np.all(np.abs(yd.to_numpy(np.float64, (n,)) - ref) <= 1e-13 * scale)
+
+
+@pytest.mark.parametrize("it", [C.INDEX_INT32, C.INDEX_INT64])
+@pytest.mark.parametrize("m,n,mean,head,long_rows", [
+    (30000, 900, 0.05, 0, 0), (30000, 900, 0.2, 0, 0), (9000, 2048, 1.0, 0, 0), (100000, 2, 0.001, 0, 0),
+    (700, 300, 20, 1, 24000), (700, 300, 20, 1, 26000), (40000, 500, 1, 600, 400)])
+def test_transpose_sparse_and_skewed(capi, it, m, n, mean, head, long_rows):
+    """The stable transpose where the rows are far apart (the search for every
+    entry's row, counts that outnumber the entries) and where a few rows hold
+    most entries (both sides of the limit on a tile's length)."""
+    rng = np.random.default_rng(m + n)
+    ln = rng.poisson(mean, m)
+    ln[:head] = long_rows
+    rp = np.concatenate([[0], np.cumsum(ln)])
+    nnz = int(rp[-1])
+    ci, v = rng.integers(0, n, nnz), rng.standard_normal(nnz).astype(np.float32)
+    idt = np.int64 if it == C.INDEX_INT64 else np.int32
+    rpd, cid, vd = H.dev(rp.astype(idt)), H.dev(ci.astype(idt)), H.dev(v)
+    vt_, pt_, it_ = C.DeviceBuffer(nnz * 4), C.DeviceBuffer((n + 1) * idt().itemsize), C.DeviceBuffer(nnz * idt().itemsize)
+    need = C.lib().tomos_csr_transpose_scratch_size(C.F32, it, m, n, nnz)
+    sc = C.DeviceBuffer(need)
+    print("transpose", it, m, n, nnz, head, flush=True)
+    C.call("tomos_csr_transpose", C.F32, it, m, n, nnz, vd.ptr, rpd.ptr, cid.ptr, vt_.ptr, pt_.ptr, it_.ptr, sc.ptr,
+           need, None)
+    order = np.argsort(ci, kind="stable")
+    assert np.array_equal(pt_.to_numpy(idt, (n + 1,)), np.concatenate([[0], np.cumsum(np.bincount(ci, minlength=n))]))
+    assert np.array_equal(it_.to_numpy(idt, (nnz,)), np.repeat(np.arange(m), ln)[order])
+    assert np.array_equal(vt_.to_numpy(np.float32, (nnz,)), v[order])

@@ -409,10 +409,12 @@ void launch_mv(int vt, const MvArgs& a, int lanes, unsigned blocks, hipStream_t 
 }
 
 // ---- validation -------------------------------------------------------------
-// flag bits: 1 row_ptrs[0] != 0, 2 decreasing row_ptrs, 4 row_ptrs[m] != nnz,
-// 8 column index out of range
+// flag[0] bits: 1 row_ptrs[0] != 0, 2 decreasing row_ptrs, 4 row_ptrs[m] !=
+// nnz, 8 column index out of range.  flag[1]: the most entries that
+// `tile_rows` rows of one panel hold (tile_rows > 0; `tiles` a panel).
 template <class I>
-__global__ void csr_check_kernel(int64_t m, int64_t n, int64_t nnz, const I* rp, const I* ci, unsigned* flag) {
+__global__ void csr_check_kernel(int64_t m, int64_t n, int64_t nnz, const I* rp, const I* ci, int64_t panel_rows,
+                                 int64_t panels, int64_t tile_rows, int64_t tiles, unsigned* flag) {
     const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
     unsigned f = 0;
     for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i <= m; i += stride) {
@@ -426,6 +428,16 @@ __global__ void csr_check_kernel(int64_t m, int64_t n, int64_t nnz, const I* rp,
         if (c < 0 || c >= n) f |= 8u;
     }
     if (f) atomicOr(flag, f);
+    if (tile_rows > 0) {
+        unsigned most = 0;
+        for (int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; g < panels * tiles; g += stride) {
+            const int64_t p = g / tiles, end = min(m, (p + 1) * panel_rows);
+            const int64_t r0 = min(p * panel_rows + (g - p * tiles) * tile_rows, end), r1 = min(r0 + tile_rows, end);
+            const int64_t e = static_cast<int64_t>(rp[r1]) - static_cast<int64_t>(rp[r0]);
+            most = max(most, static_cast<unsigned>(min(max(e, int64_t(0)), int64_t(0xFFFFFFFF))));
+        }
+        if (most) atomicMax(flag + 1, most);
+    }
 }
 
 // ---- transpose ----------------------------------------------------------------
@@ -651,6 +663,7 @@ constexpr int64_t kCountCols = 2048;      // above, a tile's runs are a few entr
 constexpr int64_t kTileEntries = 6144;    // a chunk of the sorting kernel: two blocks a CU (12288: one, 1.38 ms)
 constexpr int64_t kTileRows = 2048;       // a tile's row starts in LDS
 constexpr int64_t kGroupTiles = 64;       // tiles per scan group
+constexpr int64_t kXcdRun = 64;           // consecutive tiles on one XCD
 
 struct CountPlan {
     int64_t panel_rows, panels;
@@ -658,9 +671,6 @@ struct CountPlan {
     int64_t groups;              // scan groups per panel
 };
 
-bool count_transpose(const CsrMat& A) {
-    return A.n >= 1 && A.n <= kCountCols && A.nnz < (int64_t(1) << 32);
-}
 
 CountPlan count_plan(const CsrMat& A, int64_t panel_rows) {
     CountPlan p;
@@ -674,6 +684,29 @@ CountPlan count_plan(const CsrMat& A, int64_t panel_rows) {
     p.tiles = ceil_div(std::min(panel_rows, std::max<int64_t>(A.m, 1)), p.tile_rows);
     p.groups = ceil_div(p.tiles, kGroupTiles);
     return p;
+}
+
+// Whether the counts fit LDS and the positions 32 bits, and the counts are no
+// more than kCellsPerEntry words an entry: with fewer entries the tiles are
+// mostly counts, and a radix sort of the entries moves less (2e6 x 2000 with
+// 1e5 entries: 0.71 ms by counting, 0.12 by radix; with 5e5, 4 words an entry,
+// 0.14 and 0.21).
+constexpr int64_t kCellsPerEntry = 4;
+bool count_possible(const CsrMat& A, int64_t panel_rows) {
+    if (A.n < 1 || A.n > kCountCols || A.nnz >= (int64_t(1) << 32)) return false;
+    const CountPlan p = count_plan(A, panel_rows);
+    return p.panels * p.tiles * A.n <= std::max<int64_t>(kCellsPerEntry * A.nnz, int64_t(1) << 18);
+}
+
+// Whether no tile is so much longer than the others that the block that sorts
+// it, 24 us for every kTileEntries entries, outlasts a radix sort of them all
+// (1e6 x 2000 with 3e6 entries, two thirds of them in the first 1000 rows:
+// 7.9 ms by counting, 0.19 ms by radix; 4.8e7 entries falling off by a power
+// law from the first row, the longest tile 254000: 1.71 and 1.36 ms).  Tiles
+// of one row stay with the counting: the radix sort writes a row's index to
+// its entries with 16 lanes (5 rows of 200000: 0.68 and 1.93 ms).
+bool count_even(const CsrMat& A, int64_t panel_rows, int64_t longest_tile) {
+    return longest_tile <= 4 * kTileEntries + A.nnz / 256 || count_plan(A, panel_rows).tile_rows == 1;
 }
 
 size_t count_bytes(const CsrMat& A, int64_t panel_rows) {
@@ -702,10 +735,12 @@ struct CountTile {
 template <class I>
 __device__ __forceinline__ CountTile count_tile(const CountArgs& a) {
     CountTile q;
-    // block ids go round-robin over the 8 XCDs: an XCD takes consecutive
-    // tiles, so the lines that neighbouring tiles share meet in its L2
-    const int64_t total = a.panels * a.tiles, per = (total + 7) / 8;
-    q.g = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    // block ids go round-robin over the 8 XCDs: an XCD takes kXcdRun
+    // consecutive tiles at a time, so the lines that neighbouring tiles share
+    // meet in its L2 (with an eighth of all tiles each, the power law of
+    // count_even left seven XCDs waiting for the first: 2.90 ms, not 1.71)
+    const int64_t total = a.panels * a.tiles, i = blockIdx.x / 8;
+    q.g = (i / kXcdRun * 8 + blockIdx.x % 8) * kXcdRun + i % kXcdRun;
     q.p = q.g / a.tiles;
     q.t = q.g - q.p * a.tiles;
     if (q.g >= total) {
@@ -922,13 +957,24 @@ __global__ __launch_bounds__(64 * W) void csr_count_sort_kernel(CountArgs a) {
             }
             __syncthreads();
         }
-        uint32_t r = 0;  // row of the lane's first entry: the last start at or before it
-        for (uint32_t w = kTileRows; w; w >>= 1)
-            if (r + w < rows && start[r + w] <= first) r += w;
+        // an entry's row: the last start at or before it, searched for the
+        // lane's first entry and then walked to from there, or searched for
+        // every entry where 64 entries lie more than about 13 rows apart
+        // (2e6 x 2000, an entry in every fourth row: 0.92 -> 0.14 ms)
+        auto find = [&](uint32_t e) {
+            uint32_t r = 0;
+            for (uint32_t w = kTileRows; w; w >>= 1)
+                if (r + w < rows && start[r + w] <= e) r += w;
+            return r;
+        };
+        const bool sparse = 5 * rows > len;
+        uint32_t r = sparse ? 0 : find(first);
 #pragma unroll
         for (int u = 0; u < Q; ++u) {
             const uint32_t e = first + u * 64;
-            while (e < len && r + 1 < rows && start[r + 1] <= e) ++r;
+            if (sparse) r = find(e);
+            else
+                while (e < len && r + 1 < rows && start[r + 1] <= e) ++r;
             if (c[u] < n) {
                 const uint32_t i = h[c[u]] + at[u];
                 sval[i] = v[u];
@@ -959,7 +1005,7 @@ void transpose_count(const CsrMat& A, int64_t panel_rows, void* vals_t, void* pt
         TOMOS_HIP_CHECK(hipMemsetAsync(ptr_t, 0, static_cast<size_t>(A.n + 1) * sizeof(I), s));
         return;
     }
-    const int64_t blocks = ceil_div(p.panels * p.tiles, 8) * 8;
+    const int64_t blocks = ceil_div(p.panels * p.tiles, 8 * kXcdRun) * 8 * kXcdRun;
     require(blocks < (int64_t(1) << 31), "CSR transpose: too many tiles");
     csr_count_kernel<I><<<static_cast<unsigned>(blocks), 256, 0, s>>>(a);
     TOMOS_LAUNCH_CHECK("csr_count_kernel");
@@ -1069,25 +1115,31 @@ void csr_mv(const CsrMat& A, const Coef& c, int x_type, const void* x, int y_typ
 
 size_t csr_check_scratch_bytes() { return 256; }
 
-void csr_check(const CsrMat& A, void* scratch, size_t scratch_bytes, hipStream_t s) {
+int64_t csr_check(const CsrMat& A, void* scratch, size_t scratch_bytes, hipStream_t s, int64_t panel_rows) {
     require(scratch_bytes >= csr_check_scratch_bytes(), "csr_check: scratch too small");
     unsigned* flag = static_cast<unsigned*>(scratch);
-    TOMOS_HIP_CHECK(hipMemsetAsync(flag, 0, sizeof(unsigned), s));
+    TOMOS_HIP_CHECK(hipMemsetAsync(flag, 0, 2 * sizeof(unsigned), s));
+    CountPlan p{};
+    if (panel_rows > 0 && A.m > 0 && count_possible(A, panel_rows)) p = count_plan(A, panel_rows);
     const unsigned g = grid_1d(std::max<int64_t>(A.m + 1, A.nnz));
     if (A.idx_type == TOMOS_INDEX_INT64)
         csr_check_kernel<int64_t><<<g, 256, 0, s>>>(A.m, A.n, A.nnz, static_cast<const int64_t*>(A.row_ptrs),
-                                                    static_cast<const int64_t*>(A.col_idxs), flag);
+                                                    static_cast<const int64_t*>(A.col_idxs), p.panel_rows, p.panels,
+                                                    p.tile_rows, p.tiles, flag);
     else
         csr_check_kernel<int32_t><<<g, 256, 0, s>>>(A.m, A.n, A.nnz, static_cast<const int32_t*>(A.row_ptrs),
-                                                    static_cast<const int32_t*>(A.col_idxs), flag);
+                                                    static_cast<const int32_t*>(A.col_idxs), p.panel_rows, p.panels,
+                                                    p.tile_rows, p.tiles, flag);
     TOMOS_LAUNCH_CHECK("csr_check_kernel");
-    unsigned f = 0;
-    TOMOS_HIP_CHECK(hipMemcpyAsync(&f, flag, sizeof(unsigned), hipMemcpyDeviceToHost, s));
+    unsigned h[2] = {0, 0};
+    TOMOS_HIP_CHECK(hipMemcpyAsync(h, flag, sizeof(h), hipMemcpyDeviceToHost, s));
     TOMOS_HIP_CHECK(hipStreamSynchronize(s));
+    const unsigned f = h[0];
     require(!(f & 1u), "CSR: row_ptrs[0] must be 0");
     require(!(f & 2u), "CSR: row_ptrs must be non-decreasing");
     require(!(f & 4u), "CSR: row_ptrs[m] must equal nnz");
     require(!(f & 8u), "CSR: column index out of range");
+    return h[1];
 }
 
 int64_t csr_panel_rows(const CsrMat& A, int x_type) {
@@ -1105,19 +1157,20 @@ int64_t csr_panel_rows(const CsrMat& A, int x_type) {
 int64_t csr_panels(const CsrMat& A, int64_t panel_rows) { return A.m > 0 ? ceil_div(A.m, panel_rows) : 1; }
 
 size_t csr_transpose_scratch_bytes(const CsrMat& A, int64_t panel_rows) {
-    if (count_transpose(A)) return count_bytes(A, panel_rows);
+    // either sort may run: which, the entries decide (count_even)
     const int64_t nkeys = csr_panels(A, panel_rows) * A.n;
-    if (packed_sort(A)) return transpose_bytes_packed(A.nnz, nkeys);
-    return A.idx_type == TOMOS_INDEX_INT64 ? transpose_bytes<uint64_t>(A.nnz, nkeys)
-                                           : transpose_bytes<uint32_t>(A.nnz, nkeys);
+    const size_t radix = packed_sort(A) ? transpose_bytes_packed(A.nnz, nkeys)
+                         : A.idx_type == TOMOS_INDEX_INT64 ? transpose_bytes<uint64_t>(A.nnz, nkeys)
+                                                           : transpose_bytes<uint32_t>(A.nnz, nkeys);
+    return count_possible(A, panel_rows) ? std::max(radix, count_bytes(A, panel_rows)) : radix;
 }
 
-void csr_transpose(const CsrMat& A, int64_t panel_rows, void* vals_t, void* ptr_t, void* idx_t, void* scratch,
-                   size_t scratch_bytes, hipStream_t s) {
+void csr_transpose(const CsrMat& A, int64_t panel_rows, int64_t longest_tile, void* vals_t, void* ptr_t, void* idx_t,
+                   void* scratch, size_t scratch_bytes, hipStream_t s) {
     require(panel_rows >= 1, "csr_transpose: bad panel size");
     require(scratch_bytes >= csr_transpose_scratch_bytes(A, panel_rows), "csr_transpose: scratch too small");
     require(ptr_t != nullptr && ((vals_t && idx_t) || A.nnz == 0), "csr_transpose: null output");
-    if (count_transpose(A)) {
+    if (count_possible(A, panel_rows) && count_even(A, panel_rows, longest_tile)) {
         if (A.idx_type == TOMOS_INDEX_INT64) transpose_count<int64_t>(A, panel_rows, vals_t, ptr_t, idx_t, scratch, s);
         else transpose_count<int32_t>(A, panel_rows, vals_t, ptr_t, idx_t, scratch, s);
         return;
@@ -1319,13 +1372,14 @@ int tomos_csr_transpose(int val_type, int idx_type, int64_t m, int64_t n, int64_
     return guarded([&] {
         const CsrMat A = make_csr(val_type, idx_type, m, n, nnz, vals, row_ptrs, col_idxs);
         csr_require_valid_types(A, "tomos_csr_transpose");
-        csr_check(A, fallback_scratch(csr_check_scratch_bytes()), csr_check_scratch_bytes(), st);
-        const size_t need = csr_transpose_scratch_bytes(A, std::max<int64_t>(m, 1));
+        const int64_t pr = std::max<int64_t>(m, 1);
+        const int64_t longest = csr_check(A, fallback_scratch(csr_check_scratch_bytes()), csr_check_scratch_bytes(), st, pr);
+        const size_t need = csr_transpose_scratch_bytes(A, pr);
         if (!scratch) {
             scratch = fallback_scratch(need);
             scratch_bytes = need;
         }
-        csr_transpose(A, std::max<int64_t>(m, 1), vals_t, row_ptrs_t, col_idxs_t, scratch, scratch_bytes, st);
+        csr_transpose(A, pr, longest, vals_t, row_ptrs_t, col_idxs_t, scratch, scratch_bytes, st);
     });
 }
 
@@ -1363,14 +1417,14 @@ int tomos_csr_mv(int val_type, int idx_type, int trans, double alpha, int64_t m,
             return;
         }
         // A^T x: transpose into scratch, then the row kernels on A^T
-        csr_check(A, scratch, scratch_bytes, st);
         require(x_type == TOMOS_F32 || x_type == TOMOS_F64, "tomos_csr_mv: x must be F32 or F64");
         const TmvLayout L = tmv_layout(A, x_type);
+        const int64_t longest = csr_check(A, scratch, scratch_bytes, st, L.panel_rows);
         require(scratch_bytes >= L.work, "tomos_csr_mv: scratch too small");
         char* sc = static_cast<char*>(scratch);
         void* work = sc + L.work;
         const size_t work_bytes = scratch_bytes - L.work;
-        csr_transpose(A, L.panel_rows, sc + L.vals, sc + L.ptr, sc + L.idx, work, work_bytes, st);
+        csr_transpose(A, L.panel_rows, longest, sc + L.vals, sc + L.ptr, sc + L.idx, work, work_bytes, st);
         const CsrMat T = make_csr(val_type, idx_type, L.panels * n, m, nnz, sc + L.vals, sc + L.ptr, sc + L.idx);
         csr_tmv(T, L.panels, L.panel_rows, n, c, x_type, x, y_type, y, work, work_bytes, st);
     });

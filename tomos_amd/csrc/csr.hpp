@@ -37,21 +37,24 @@ int64_t csr_sumsq_blocks_max(int64_t m);
 
 // Device-side validation: row_ptrs[0] = 0, non-decreasing, row_ptrs[m] =
 // nnz, 0 <= col_idxs < n.  Synchronous; throws Error(kErrInvalidArgument).
-void csr_check(const CsrMat& A, void* scratch, size_t scratch_bytes, hipStream_t s);
+// With panel_rows > 0, returns what csr_transpose by such panels has to know
+// of the row lengths (the entries of its longest row tile).
+int64_t csr_check(const CsrMat& A, void* scratch, size_t scratch_bytes, hipStream_t s, int64_t panel_rows = 0);
 size_t csr_check_scratch_bytes();
 
 // Panel-blocked transpose of A: A's rows are cut into panels of
 // panel_rows rows and row p*n + c of the result (a CSR matrix of
 // panels*n rows over A's m columns) holds column c of panel p, in A's row
 // order; panel_rows >= m gives plain A^T (n x m).  Products with it are
-// deterministic.  A must be valid (csr_check).  csr_panel_rows(A, x_type)
+// deterministic.  A must be valid (csr_check, whose longest_tile chooses the
+// sort).  csr_panel_rows(A, x_type)
 // picks panels whose slice of the gathered vector (of x_type) fits the
 // 64 KB of LDS a product block stages it in.
 int64_t csr_panel_rows(const CsrMat& A, int x_type);
 int64_t csr_panels(const CsrMat& A, int64_t panel_rows);
 size_t csr_transpose_scratch_bytes(const CsrMat& A, int64_t panel_rows);
-void csr_transpose(const CsrMat& A, int64_t panel_rows, void* vals_t, void* ptr_t, void* idx_t, void* scratch,
-                   size_t scratch_bytes, hipStream_t s);
+void csr_transpose(const CsrMat& A, int64_t panel_rows, int64_t longest_tile, void* vals_t, void* ptr_t, void* idx_t,
+                   void* scratch, size_t scratch_bytes, hipStream_t s);
 
 // y (nout) = alpha * A^T x + beta * y from the blocked transpose Tb
 // (panels * nout rows): per-panel products, then each output's panel

@@ -773,8 +773,8 @@ void lsqr_solve_csr(const tomos_lsqr_options& o, const CsrMat& A, int ref_type, 
     sv.r64 = o.refine_type == TOMOS_F64;
     sv.p64 = o.precond_type >= 0 ? o.precond_type == TOMOS_F64 : sv.v64;
     // indices validated once (synchronous), then A^T built in the scratch
-    csr_check(A, sv.sc + sv.L.csr_tmp, sv.L.csr_tmp_bytes, s);
-    csr_transpose(A, sv.L.csr_panel_rows, sv.sc + sv.L.csr_vals, sv.sc + sv.L.csr_ptr, sv.sc + sv.L.csr_idx,
+    const int64_t longest = csr_check(A, sv.sc + sv.L.csr_tmp, sv.L.csr_tmp_bytes, s, sv.L.csr_panel_rows);
+    csr_transpose(A, sv.L.csr_panel_rows, longest, sv.sc + sv.L.csr_vals, sv.sc + sv.L.csr_ptr, sv.sc + sv.L.csr_idx,
                   sv.sc + sv.L.csr_tmp, sv.L.csr_tmp_bytes, s);
     sv.csr = &A;
     sv.csr_t = A;
