@@ -231,3 +231,60 @@ def test_gemv_edges(capi, orc, a_type, shape):
             fin = np.isfinite(ref)
             assert np.array_equal(got[~fin], ref[~fin], equal_nan=True)
             check_close(got[fin], ref[fin], scale[fin], rtol)
+
+
+@pytest.mark.parametrize("a_type", [C.F32, C.F64, C.BF16, C.FP32_16, C.FP32_BF16])
+@pytest.mark.parametrize("m,n", [(1, 4097), (3, 9000), (9, 4103), (300, 5001), (1025, 4100), (2050, 8193), (12300, 8200)])
+def test_gemv_t_many_columns(capi, orc, a_type, m, n):
+    """A^T x of many short columns (a wave owns 8): fewer rows than a vector,
+    the last vector moved back over its neighbour's rows with an Inf beside
+    it, column counts around the wave's 8, both sides of the rules on a
+    column's bytes.  Products of small integers, |sum| < 2^24: exact."""
+    rng = np.random.default_rng(m + n)
+    A = rng.integers(-8, 9, (m, n)).astype(np.float32)
+    A[m - 1, n // 2] = np.inf
+    x = rng.integers(-8, 9, m).astype(np.float64)
+    x[m - 1] = 2.0
+    lda = m + 3
+    store = np.full((lda, n), np.nan, np.float32, order="F")
+    store[:m] = A
+    if a_type in FORMATS:
+        wh, wr = H.pack(FORMATS[a_type][0], store)
+    else:
+        st = store.astype(np.float64) if a_type == C.F64 else bf16_bits_rne(store) if a_type == C.BF16 else store
+        wh, wr = H.dev(st), None
+    with np.errstate(invalid="ignore"):
+        ref = A.T.astype(np.float64) @ x
+    for tier in (C.TIER_DEFAULT, C.TIER_FAST, C.TIER_EXACT):
+        print("many columns", a_type, m, n, tier, flush=True)
+        got = H.gemv(a_type, tier, 1, 1.0, m, n, wh, wr, lda, x, 0.0, None, C.F64, C.F64)
+        fin = np.isfinite(ref)
+        assert np.array_equal(got[fin], ref[fin])
+        assert np.array_equal(got[~fin], ref[~fin])
+
+
+def test_gemv_t_beyond_one_grid(capi):
+    """More column groups than the wave kernel's grid holds, and more columns
+    than a launch of 512 threads for every four has work items for (2^32)."""
+    n = (1 << 25) + 5
+    A = (np.arange(n) % 251).astype(np.float32).reshape(1, n)
+    got = H.gemv(C.F32, C.TIER_DEFAULT, 1, 1.0, 1, n, H.dev(A), None, 1, np.array([3.0]))
+    assert np.array_equal(got, 3.0 * A[0])
+
+
+@pytest.mark.parametrize("a_type", [C.F32, C.F64, C.BF16, C.FP32_16])
+@pytest.mark.parametrize("n", [1, 5, 64, 300, 2000])
+def test_gemv_t_in_place(capi, a_type, n):
+    """y = A^T x with y over x (a square A): every product before any store."""
+    rng = np.random.default_rng(n)
+    A, x = rng.integers(-8, 9, (n, n)).astype(np.float32), rng.integers(-8, 9, n).astype(np.float64)
+    if a_type == C.FP32_16:
+        wh, wr = H.pack(C.PACK_FP32_16, A)
+    else:
+        wh, wr = H.dev(A.astype(np.float64) if a_type == C.F64 else bf16_bits_rne(A) if a_type == C.BF16 else A), None
+    xd = H.dev(x)
+    for tier in (C.TIER_DEFAULT, C.TIER_EXACT):
+        C.call("tomos_memcpy_htod", xd.ptr, x.ctypes.data, x.nbytes, None)
+        C.call("tomos_gemv", a_type, tier, 1, 1.0, n, n, wh.ptr, wr.ptr if wr else None, n, C.F64, xd.ptr, 0.0, C.F64,
+               xd.ptr, None, 0, None)
+        assert np.array_equal(xd.to_numpy(np.float64, (n,)), A.T.astype(np.float64) @ x)

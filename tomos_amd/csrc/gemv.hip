@@ -409,19 +409,20 @@ struct WaveTR<1, OFF, T> {
     }
 };
 
-// Replaces the first `lo` rows of a vector by words that decode to zero
-// (their x is zero too, but they may hold Inf).  On the raw words, so that
-// the decode stays next to its FMA (one v_fma_mix for a half).
+// Replaces the first `lo` rows of a vector by zero words: their x is zero,
+// but they may hold Inf.  On the raw words, so that the decode stays next to
+// its FMA (one v_fma_mix for a half).  A zero word is finite in every format
+// and not one of FP32_16's saturated words, which would send the last vector
+// of every column through dot_rows' slow path (300 x 4000 EXACT: 24 -> 13 us).
 template <int FMT, int DEC, int VEC>
 __device__ __forceinline__ void clear_rows(Raw<FMT, DEC, VEC>& R, int lo) {
     if (VEC == 1) return;
-    constexpr uint32_t zero = FMT == FMT_P16 ? 0x3801u : 0u;  // FP32_16: the saturated underflow word
 #pragma unroll
     for (int v = 0; v < VEC - 1; ++v)
         if (v < lo) {
             if constexpr (is16<FMT>()) {
                 const uint32_t keep = 0xFFFF0000u >> (16 * (v & 1));
-                R.h[v / 2] = (R.h[v / 2] & keep) | (zero << (16 * (v & 1)));
+                R.h[v / 2] &= keep;
                 if constexpr (DEC == DEC_EXACT) R.r[v / 2] &= keep;
             } else if constexpr (FMT == FMT_F32) {
                 R.h[v] = 0;
@@ -586,6 +587,52 @@ __global__ __launch_bounds__(kColThreads) void gemv_t_cols_kernel(
     }
 }
 
+// Short columns and many of them: a wave owns CG whole columns (a strided
+// loop over the column groups bounds the grid), so that lanes without a row
+// cost a wave and not a block of 512, and the loads of CG columns are in
+// flight together; sums as in gemv_t_cols_kernel.  Bound by HBM: 4000 x
+// 60000 bf16 hi 76 us (6.3 TB/s; that kernel 106, row chunks of 64 columns
+// 82), 64 x 1000000 62 us (1195, 228).
+constexpr int kWaveCols = 8;
+constexpr int64_t kWaveBlocks = int64_t(1) << 18;
+template <int FMT, int DEC, int VEC, class ACC, int CG, bool NTL>
+__global__ __launch_bounds__(kThreads) void gemv_t_wave_kernel(
+    int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr, int64_t lda,
+    const void* __restrict__ x, bool x64, ACC* __restrict__ partial, void* __restrict__ y, bool y64, Coef coef) {
+    if (coef.skip && *coef.skip) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t waves = static_cast<int64_t>(gridDim.x) * (kThreads / 64);
+    for (int64_t c0 = (static_cast<int64_t>(blockIdx.x) * (kThreads / 64) + wave) * CG; c0 < n; c0 += waves * CG) {
+        const int ncols = static_cast<int>(min<int64_t>(CG, n - c0));
+        double acc[CG];
+#pragma unroll
+        for (int c = 0; c < CG; ++c) acc[c] = 0.0;
+        for (int64_t ir = static_cast<int64_t>(lane) * VEC; ir < m; ir += 64 * VEC) {
+            const int64_t i = first_row<VEC>(ir, m);
+            const int lo = static_cast<int>(ir - i);
+            Raw<FMT, DEC, VEC> R[CG];
+#pragma unroll
+            for (int c = 0; c < CG; ++c)
+                load_raw<FMT, DEC, VEC, NTL>(a, wr, i + (c0 + min(c, ncols - 1)) * lda, R[c]);
+            ACC xv[VEC];
+            load_x_rows<VEC, ACC>(x, x64, i, lo, xv);
+            const bool edge = __any(lo != 0);
+#pragma unroll
+            for (int c = 0; c < CG; ++c)
+                acc[c] += static_cast<double>(dot_rows<FMT, DEC, VEC, ACC>(R[c], xv, lo, edge, ACC(0)));
+        }
+        WaveTR<CG, 32, double>::run(acc, lane);
+        const int c = lane / (64 / CG);
+        if (lane % (64 / CG) == 0 && c < ncols) {
+            if (partial) partial[c0 + c] = static_cast<ACC>(acc[0]);
+            else
+                store_y(y, y64, c0 + c, read_coef(coef.alpha, coef.dalpha, coef.alpha_mul), acc[0],
+                        read_coef(coef.beta, coef.dbeta, coef.beta_mul));
+        }
+    }
+}
+
 // Adds the chunk partials of 32 columns: 8 chunk slices per column (a slice
 // takes every eighth chunk, four loads in flight), added in slice order
 // (64 chunks x 501: 7.0 us with a thread per column, 5.1 with the slices).
@@ -691,9 +738,21 @@ PlanT plan_t(const Kind& k, int64_t m, int64_t n) {
     return p;
 }
 
-// TRANSPOSE: whole columns per block (gemv_t_cols_kernel) up to this many
-// bytes a column; longer ones are cut into row chunks.
+// TRANSPOSE: whole columns up to kColBytes bytes each, longer ones are cut
+// into row chunks.  A block of 512 threads takes them (gemv_t_cols_kernel),
+// or a wave (gemv_t_wave_kernel) where there are enough for every CU: above
+// 4096 columns of up to 4 KB, which leave most of a block's lanes without a
+// row (1000 x 5000 FP32_16 EXACT 16.8 us by blocks, 9.6 by waves), above 8192
+// of up to 24 KB (4000 x 5000 hi 11.9 and 15.1, 4000 x 60000 118 and 81); of
+// longer ones a block's loads are as many (16000 x 10000 66 and 78).
 constexpr int64_t kColBytes = int64_t(128) << 10;
+bool t_waves(int64_t col_bytes, int64_t n) {
+    return col_bytes <= (int64_t(24) << 10) && n > (col_bytes <= 4096 ? 4096 : 8192);
+}
+template <int FMT, int DEC>
+constexpr int64_t elem_bytes() {
+    return FMT == FMT_F64 ? 8 : (FMT == FMT_F32 || DEC == DEC_EXACT ? 4 : 2);
+}
 bool t_cols(const Kind& k, int64_t m) {
     const int64_t esz = k.fmt == FMT_F64 ? 8 : (k.fmt == FMT_F32 || k.dec == DEC_EXACT ? 4 : 2);
     return m * esz <= kColBytes;
@@ -724,8 +783,7 @@ size_t scratch_for(const Kind& k, int trans, int64_t m, int64_t n) {
 // non-temporal, 77 us cacheable).
 template <int FMT, int DEC>
 bool streams(int64_t m, int64_t n, int64_t lda) {
-    const int64_t esz = FMT == FMT_F64 ? 8 : (FMT == FMT_F32 ? 4 : (DEC == DEC_EXACT ? 4 : 2));
-    return lda % vec_full<FMT>() == 0 && stream_loads(m * n * esz);
+    return lda % vec_full<FMT>() == 0 && stream_loads(m * n * elem_bytes<FMT, DEC>());
 }
 
 template <int FMT, int DEC, int VEC, class ACC, bool NTL>
@@ -765,7 +823,11 @@ template <int FMT, int DEC, int VEC, class ACC, bool NTL>
 void launch_t_cols(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x, bool x64,
                    ACC* part, void* y, bool y64, const Coef& coef, hipStream_t s) {
     // one column a block while that fills the chip about twice, then two, then four
-    if (n <= 512)
+    if (t_waves(m * elem_bytes<FMT, DEC>(), n))
+        gemv_t_wave_kernel<FMT, DEC, VEC, ACC, kWaveCols, NTL>
+            <<<static_cast<unsigned>(std::min(ceil_div(n, kWaveCols * (kThreads / 64)), kWaveBlocks)), kThreads, 0, s>>>(
+                m, n, a, wr, lda, x, x64, part, y, y64, coef);
+    else if (n <= 512)
         gemv_t_cols_kernel<FMT, DEC, VEC, ACC, 1, NTL><<<static_cast<unsigned>(n), kColThreads, 0, s>>>(
             m, n, a, wr, lda, x, x64, part, y, y64, coef);
     else if (n <= 1024)
@@ -786,10 +848,13 @@ int run_t(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, 
     constexpr int CB = sizeof(ACC) == 8 ? 32 : 64;
     ACC* part = static_cast<ACC*>(scratch);
     if (cols && m > 0) {
-        require(n < (int64_t(1) << 31), "gemv: grid too large");
         ACC* one = finish ? nullptr : part;
         if (m < VF)
             launch_t_cols<FMT, DEC, 1, ACC, false>(m, n, a, wr, lda, x, x64, one, y, y64, coef, s);
+        // non-temporal above what the last-level cache holds (60000 x 2000
+        // bf16 hi, 240 MB, again and again: 36 us cacheable, 41 not)
+        else if (DEC != DEC_EXACT && m * n * elem_bytes<FMT, DEC>() > (int64_t(256) << 20) && streams<FMT, DEC>(m, n, lda))
+            launch_t_cols<FMT, DEC, VF, ACC, true>(m, n, a, wr, lda, x, x64, one, y, y64, coef, s);
         else
             launch_t_cols<FMT, DEC, VF, ACC, false>(m, n, a, wr, lda, x, x64, one, y, y64, coef, s);
         return 1;
@@ -800,11 +865,14 @@ int run_t(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, 
         const dim3 grid(static_cast<unsigned>(blocks));
         // the EXACT tier reads A with cacheable loads: its non-temporal form
         // needs 256 VGPRs (one wave per SIMD), the cacheable one ~140
-        if (DEC != DEC_EXACT && streams<FMT, DEC>(m, n, lda))
+        if (DEC != DEC_EXACT && m >= VF && streams<FMT, DEC>(m, n, lda))
             gemv_t_kernel<FMT, DEC, VF, ACC, CB, true><<<grid, kThreads, 0, s>>>(
                 m, n, a, wr, lda, x, x64, p.rows_per_chunk, p.ncg, part, coef.skip);
-        else  // m > kColBytes / 8, so at least a vector
+        else if (m >= VF)
             gemv_t_kernel<FMT, DEC, VF, ACC, CB, false><<<grid, kThreads, 0, s>>>(
+                m, n, a, wr, lda, x, x64, p.rows_per_chunk, p.ncg, part, coef.skip);
+        else  // in place only: otherwise whole columns
+            gemv_t_kernel<FMT, DEC, 1, ACC, CB, false><<<grid, kThreads, 0, s>>>(
                 m, n, a, wr, lda, x, x64, p.rows_per_chunk, p.ncg, part, coef.skip);
         TOMOS_LAUNCH_CHECK("gemv_t_kernel");
     }
@@ -816,6 +884,13 @@ int run_t(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, 
 }
 
 }  // namespace
+
+// Whether x (nx entries) and y (ny entries) share memory.
+static bool overlap(const void* x, int x_type, int64_t nx, const void* y, int y_type, int64_t ny) {
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+    return x0 < y0 + static_cast<uintptr_t>(ny) * (y_type == TOMOS_F64 ? 8 : 4) &&
+           y0 < x0 + static_cast<uintptr_t>(nx) * (x_type == TOMOS_F64 ? 8 : 4);
+}
 
 size_t gemv_scratch_bytes(int a_type, int tier, int trans, int64_t m, int64_t n) {
     return scratch_for(kind_for(a_type, tier, trans), trans, m, n);
@@ -846,7 +921,8 @@ void gemv(int a_type, int tier, int trans, const Coef& coef, int64_t m, int64_t 
     if (inner > 0) require(a != nullptr && x != nullptr, "gemv: null A or x");
     if (k.dec == DEC_EXACT) require(wr != nullptr || inner == 0, "gemv: EXACT tier needs the wr plane");
     const size_t need = scratch_for(k, trans, m, n);
-    const bool cols = trans == TOMOS_TRANSPOSE && m > 0 && t_cols(k, m);
+    // y over x: the products of the row chunks are complete before y is written
+    const bool cols = trans == TOMOS_TRANSPOSE && m > 0 && t_cols(k, m) && !overlap(x, x_type, m, y, y_type, n);
     if (need > 0) {
         if (scratch == nullptr) {
             if (trans == TOMOS_TRANSPOSE && !cols) scratch = fallback_scratch(need);
