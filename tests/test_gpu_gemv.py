@@ -288,3 +288,59 @@ def test_gemv_t_in_place(capi, a_type, n):
         C.call("tomos_gemv", a_type, tier, 1, 1.0, n, n, wh.ptr, wr.ptr if wr else None, n, C.F64, xd.ptr, 0.0, C.F64,
                xd.ptr, None, 0, None)
         assert np.array_equal(xd.to_numpy(np.float64, (n,)), A.T.astype(np.float64) @ x)
+
+
+@pytest.mark.parametrize("a_type", [C.F32, C.F64, C.BF16, C.FP32_16, C.FP32_BF16])
+@pytest.mark.parametrize("m,n", [(1, 300001), (7, 90001), (130, 33333), (300, 20011), (1000, 6007), (4099, 3001)])
+def test_gemv_n_wide(capi, orc, a_type, m, n):
+    """A x of a wide matrix, whose columns are split over the grid: fewer rows
+    than a vector, ragged rows and columns, an Inf, beta != 0, the caller's
+    scratch of exactly the advertised size.  Entries are +-1 or 0 and |x| <= 8,
+    so every sum stays below 2^24: exact."""
+    rng = np.random.default_rng(m + n)
+    A, x = rng.integers(-1, 2, (m, n)).astype(np.float32), rng.integers(-8, 9, n).astype(np.float64)
+    A[m - 1, n - 1], x[n - 1] = np.inf, 2.0
+    y0 = rng.integers(-8, 9, m).astype(np.float64)
+    if a_type in FORMATS:
+        wh, wr = H.pack(FORMATS[a_type][0], A)
+    else:
+        wh, wr = H.dev(A.astype(np.float64) if a_type == C.F64 else bf16_bits_rne(A) if a_type == C.BF16 else A), None
+    with np.errstate(invalid="ignore"):
+        ref = 2.0 * (A.astype(np.float64) @ x) - y0
+    for tier in (C.TIER_DEFAULT, C.TIER_FAST, C.TIER_EXACT):
+        print("wide", a_type, m, n, tier, flush=True)
+        got = H.gemv(a_type, tier, 0, 2.0, m, n, wh, wr, m, x, -1.0, y0, C.F64, C.F64, scratch="explicit")
+        assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("a_type", [C.F32, C.BF16, C.FP32_16])
+def test_gemv_n_error_of_fp32_sums(capi, orc, a_type):
+    """FP32 sums of the DEFAULT tier run over at most L = 32 columns here and
+    meet in FP64.  A rounding is 2^-24 / sqrt(3) rms of its partial sum at most,
+    partial sums grow as sqrt(k), so a chain's error is 2^-24 sqrt(L^2 / 6)
+    terms and the whole sum's, relative, 2^-24 sqrt(L / 6) = 1.38e-7."""
+    m, n = 60000, 1000
+    rng = np.random.default_rng(1)
+    A, x = rng.standard_normal((m, n), dtype=np.float32), rng.standard_normal(n).astype(np.float32)
+    if a_type == C.FP32_16:
+        wh, wr = H.pack(C.PACK_FP32_16, A)
+        A = orc.unpack(orc.DEC16_HALF, *orc.pack(C.PACK_FP32_16, A)).astype(np.float32)
+    else:
+        st = bf16_bits_rne(A) if a_type == C.BF16 else A
+        wh, wr = H.dev(st), None
+        A = (st.astype(np.uint32) << 16).view(np.float32) if a_type == C.BF16 else A
+    got = H.gemv(a_type, C.TIER_DEFAULT, 0, 1.0, m, n, wh, wr, m, x, 0.0, None, C.F32, C.F64)
+    ref = A.astype(np.float64) @ x.astype(np.float64)
+    assert np.linalg.norm(got - ref) <= 2.0 ** -24 * np.sqrt(32 / 6) * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("n", [17, 64, 300, 2000])
+def test_gemv_n_in_place(capi, n):
+    """y = A x with y over x (a square A): every product before any store."""
+    rng = np.random.default_rng(n)
+    A, x = rng.integers(-8, 9, (n, n)).astype(np.float32), rng.integers(-8, 9, n).astype(np.float64)
+    wh, xd = H.dev(A), H.dev(x)
+    for tier in (C.TIER_DEFAULT, C.TIER_EXACT):
+        C.call("tomos_memcpy_htod", xd.ptr, x.ctypes.data, x.nbytes, None)
+        C.call("tomos_gemv", C.F32, tier, 0, 1.0, n, n, wh.ptr, None, n, C.F64, xd.ptr, 0.0, C.F64, xd.ptr, None, 0, None)
+        assert np.array_equal(xd.to_numpy(np.float64, (n,)), A.astype(np.float64) @ x)

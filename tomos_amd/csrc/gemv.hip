@@ -11,7 +11,8 @@
 //           16-B loads are in flight per lane.  x[j] is wave-uniform and is
 //           read through the scalar cache.  When m is too small to fill the
 //           chip, the waves of a block split the columns and add their sums
-//           through LDS in a fixed order.
+//           through LDS in a fixed order; a wide matrix of few rows is split
+//           over the grid too, with partial sums that a second pass adds.
 // z = A^T y (TRANSPOSE): a block owns a chunk of rows and a group of CB
 //           columns; each lane keeps CB column accumulators in VGPRs and
 //           walks the chunk in 16-B row vectors (loads coalesced along the
@@ -19,7 +20,7 @@
 //           butterfly (CB-1 shuffles per lane instead of 6*CB), the four
 //           waves combine through LDS, and the per-chunk partials are summed
 //           in a fixed order by a second pass.  Short columns are owned whole
-//           by a block, without partials.  No atomics anywhere: results are
+//           by a block or a wave, without partials.  No atomics anywhere: results are
 //           bit-reproducible run to run.
 #include <algorithm>
 
@@ -185,22 +186,22 @@ __device__ __forceinline__ double read_coef(double host, const double* dev, doub
     return dev ? mul * (*dev) : host;
 }
 
-// x[j .. j+U), a wave's U columns; entries at j1 and beyond repeat x[j1-1].
-// One branch on the type for all of them, so that their scalar loads are in
-// flight together.
-template <int U, class ACC>
+// x[j .. j+U), a wave's U columns.  One branch on the type for all of them,
+// so that their scalar loads are in flight together.  LAST: entries at j1 and
+// beyond repeat x[j1-1].
+template <int U, class ACC, bool LAST>
 __device__ __forceinline__ void load_x_cols(const void* __restrict__ x, bool x64, int64_t j, int64_t j1,
                                             ACC (&xs)[U]) {
     if (x64) {
         double t[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) t[u] = static_cast<const double*>(x)[min(j + u, j1 - 1)];
+        for (int u = 0; u < U; ++u) t[u] = static_cast<const double*>(x)[LAST ? min(j + u, j1 - 1) : j + u];
 #pragma unroll
         for (int u = 0; u < U; ++u) xs[u] = static_cast<ACC>(t[u]);
     } else {
         float t[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) t[u] = static_cast<const float*>(x)[min(j + u, j1 - 1)];
+        for (int u = 0; u < U; ++u) t[u] = static_cast<const float*>(x)[LAST ? min(j + u, j1 - 1) : j + u];
 #pragma unroll
         for (int u = 0; u < U; ++u) xs[u] = static_cast<ACC>(t[u]);
     }
@@ -260,39 +261,70 @@ __device__ __forceinline__ void block_sumsq_out(double v, double* out) {
 }
 
 // ------------------------------------------------------------ NO_TRANSPOSE
+// Columns whose loads are in flight together (EXACT: two planes, and 8 would
+// take 256 VGPRs).
+template <int DEC>
+constexpr int kBatchCols = DEC == DEC_EXACT ? 4 : 8;
+
 // acc += A[i0 .. i0+VEC, j0 .. j1) x[j0 .. j1): U columns' loads in flight.
+// The indices of whole batches need no clamping: with it, its scalar
+// operations ahead of every batch's loads took 1050000 x 300 bf16 hi from 110
+// to 126 us.
 template <int FMT, int DEC, int VEC, class ACC, bool NTL>
 __device__ __forceinline__ void sweep_columns(const void* __restrict__ a, const uint16_t* __restrict__ wr,
                                               int64_t lda, const void* __restrict__ x, bool x64, int64_t i0,
                                               int64_t j0, int64_t j1, ACC (&acc)[VEC]) {
-    constexpr int U = DEC == DEC_EXACT ? 4 : 8;  // EXACT: two planes, and 8 would take 256 VGPRs
-    for (int64_t j = j0; j < j1; j += U) {
+    constexpr int U = kBatchCols<DEC>;
+    int64_t j = j0;
+    for (; j + U <= j1; j += U) {
         Raw<FMT, DEC, VEC> R[U];
         ACC xs[U];
-        load_x_cols<U, ACC>(x, x64, j, j1, xs);
-        if (j + U <= j1) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) load_raw<FMT, DEC, VEC, NTL>(a, wr, i0 + (j + u) * lda, R[u]);
+        for (int u = 0; u < U; ++u) load_raw<FMT, DEC, VEC, NTL>(a, wr, i0 + (j + u) * lda, R[u]);
+        load_x_cols<U, ACC, false>(x, x64, j, j1, xs);
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
+        for (int u = 0; u < U; ++u) {
+            ACC av[VEC];
+            decode<FMT, DEC, VEC, ACC>(R[u], av);
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) acc[v] = fma(av[v], xs[u], acc[v]);
+        }
+    }
+    if (j < j1) {  // the last columns, their loads in flight together as well
+        Raw<FMT, DEC, VEC> R[U];
+        ACC xs[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (j + u < j1) load_raw<FMT, DEC, VEC, NTL>(a, wr, i0 + (j + u) * lda, R[u]);
+        load_x_cols<U, ACC, true>(x, x64, j, j1, xs);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (j + u < j1) {
                 ACC av[VEC];
                 decode<FMT, DEC, VEC, ACC>(R[u], av);
 #pragma unroll
                 for (int v = 0; v < VEC; ++v) acc[v] = fma(av[v], xs[u], acc[v]);
             }
-        } else {  // the last columns, their loads in flight together as well
+        }
+    }
+}
+
+// The same sum in FP64 from ACC sums over at most `chain` columns (a multiple
+// of the batch) each; FP64 sums throughout when ACC is double.
+template <int FMT, int DEC, int VEC, class ACC, bool NTL>
+__device__ __forceinline__ void sweep_chains(const void* __restrict__ a, const uint16_t* __restrict__ wr,
+                                             int64_t lda, const void* __restrict__ x, bool x64, int64_t i0,
+                                             int64_t j0, int64_t j1, int64_t chain, double (&sum)[VEC]) {
+    if constexpr (sizeof(ACC) == 8) {
+        sweep_columns<FMT, DEC, VEC, ACC, NTL>(a, wr, lda, x, x64, i0, j0, j1, sum);
+    } else {
+        for (int64_t c0 = j0; c0 < j1; c0 += chain) {
+            ACC acc[VEC];
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (j + u < j1) load_raw<FMT, DEC, VEC, NTL>(a, wr, i0 + (j + u) * lda, R[u]);
+            for (int v = 0; v < VEC; ++v) acc[v] = ACC(0);
+            sweep_columns<FMT, DEC, VEC, ACC, NTL>(a, wr, lda, x, x64, i0, c0, min(j1, c0 + chain), acc);
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (j + u < j1) {
-                    ACC av[VEC];
-                    decode<FMT, DEC, VEC, ACC>(R[u], av);
-#pragma unroll
-                    for (int v = 0; v < VEC; ++v) acc[v] = fma(av[v], xs[u], acc[v]);
-                }
-            }
+            for (int v = 0; v < VEC; ++v) sum[v] += static_cast<double>(acc[v]);
         }
     }
 }
@@ -310,14 +342,14 @@ __device__ __forceinline__ int64_t first_row(int64_t i, int64_t m) {
 template <int FMT, int DEC, int VEC, class ACC, bool NTL>
 __global__ __launch_bounds__(kThreads) void gemv_n_kernel(
     int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
-    int64_t lda, const void* __restrict__ x, bool x64, void* __restrict__ y, bool y64, Coef coef) {
+    int64_t lda, const void* __restrict__ x, bool x64, void* __restrict__ y, bool y64, Coef coef, int64_t chain) {
     if (coef.skip && *coef.skip) return;
     const int64_t ir = (static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x) * VEC;
-    ACC acc[VEC];
+    double acc[VEC];
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) acc[v] = ACC(0);
+    for (int v = 0; v < VEC; ++v) acc[v] = 0.0;
     const int64_t i0 = first_row<VEC>(ir, m);
-    if (ir < m) sweep_columns<FMT, DEC, VEC, ACC, NTL>(a, wr, lda, x, x64, i0, 0, n, acc);
+    if (ir < m) sweep_chains<FMT, DEC, VEC, ACC, NTL>(a, wr, lda, x, x64, i0, 0, n, chain, acc);
     const double al = read_coef(coef.alpha, coef.dalpha, coef.alpha_mul);
     const double be = read_coef(coef.beta, coef.dbeta, coef.beta_mul);
     double sq = 0.0;
@@ -325,7 +357,7 @@ __global__ __launch_bounds__(kThreads) void gemv_n_kernel(
 #pragma unroll
         for (int v = 0; v < VEC; ++v)
             if (i0 + v >= ir) {
-                const double r = store_y(y, y64, i0 + v, al, static_cast<double>(acc[v]), be);
+                const double r = store_y(y, y64, i0 + v, al, acc[v], be);
                 sq += r * r;
             }
     }
@@ -334,33 +366,34 @@ __global__ __launch_bounds__(kThreads) void gemv_n_kernel(
 
 // The rows alone do not fill the chip: a block takes RL x VEC rows and its
 // column groups (64 / RL in each wave) split the columns; their sums meet in
-// lane shuffles and LDS and are added in group order, in FP64 across waves.
-// No partials in memory (m x splits accumulators written and read back by a
-// second launch): 20000 x 200 bf16 hi 5.2 + 4.1 -> 5.5 us in one launch,
-// 1e6 x 1000 FP32_16 hi 389 + 5 -> 347 us (5.8 TB/s).  RL = 16, 256-byte runs of a column, where even 64-lane
-// rows times 16 waves are few.  VEC * sizeof(ACC) * waves is at most 512
-// bytes per row lane (32 KB of LDS).
-constexpr int kSplitLds = 512;
+// lane shuffles and LDS and are added in group order, in FP64.  One launch
+// and no partials in memory: 20000 x 200 bf16 hi 5.2 + 4.1 -> 5.5 us,
+// 1e6 x 1000 FP32_16 hi 389 + 5 -> 347 us (5.8 TB/s).  RL = 16, 256-byte runs
+// of a column, where there are few row blocks.  A wide matrix is split by
+// columns over gridDim.y as well, the sums go to partial[split][m] and
+// gemv_n_finish adds them (plan_n).
+constexpr int kSplitLds = 512;  // VEC * sizeof(ACC) * waves at most
 template <int FMT, int DEC, int VEC, class ACC, int RL, bool NTL>
 __global__ __launch_bounds__(kSplitLds / VEC / sizeof(ACC) >= 16 ? 1024 : 64 * (kSplitLds / VEC / sizeof(ACC)))
 void gemv_n_split_kernel(int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
                          int64_t lda, const void* __restrict__ x, bool x64, void* __restrict__ y, bool y64,
-                         Coef coef, int64_t col_chunk) {
+                         Coef coef, int64_t split_cols, int64_t col_chunk, int64_t chain, ACC* __restrict__ partial) {
     if (coef.skip && *coef.skip) return;
     constexpr int kStride = RL + 1;  // v-major slots, odd stride: reads of consecutive rows spread over the banks
-    __shared__ ACC red[kSplitLds / sizeof(ACC) * kStride];
+    extern __shared__ double red[];  // [waves][VEC][kStride]
     const int lane = threadIdx.x & 63, rl = lane % RL;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int waves = blockDim.x >> 6;
     const int64_t b0 = static_cast<int64_t>(blockIdx.x) * RL * VEC;
     const int64_t ir = b0 + rl * VEC;
-    ACC acc[VEC];
+    double acc[VEC];
 #pragma unroll
-    for (int v = 0; v < VEC; ++v) acc[v] = ACC(0);
+    for (int v = 0; v < VEC; ++v) acc[v] = 0.0;
     const int64_t i0 = first_row<VEC>(ir, m);
     if (ir < m) {
-        const int64_t j0 = RL == 64 ? wave * col_chunk : (wave * (64 / RL) + lane / RL) * col_chunk;
-        sweep_columns<FMT, DEC, VEC, ACC, NTL>(a, wr, lda, x, x64, i0, j0, min(n, j0 + col_chunk), acc);
+        const int64_t c0 = blockIdx.y * split_cols, c1 = min(n, c0 + split_cols);
+        const int64_t j0 = c0 + (RL == 64 ? wave * col_chunk : (wave * (64 / RL) + lane / RL) * col_chunk);
+        sweep_chains<FMT, DEC, VEC, ACC, NTL>(a, wr, lda, x, x64, i0, j0, min(c1, j0 + col_chunk), chain, acc);
     }
 #pragma unroll
     for (int o = RL; o < 64; o *= 2)
@@ -378,9 +411,37 @@ void gemv_n_split_kernel(int64_t m, int64_t n, const void* __restrict__ a, const
     double sq = 0.0;
     for (int r = threadIdx.x; r < RL * VEC && b0 + r < m; r += blockDim.x) {
         double s = 0.0;
-        for (int w = 0; w < waves; ++w) s += static_cast<double>(red[(w * VEC + r % VEC) * kStride + r / VEC]);
-        const double t = store_y(y, y64, b0 + r, al, s, be);
-        sq += t * t;
+        for (int w = 0; w < waves; ++w) s += red[(w * VEC + r % VEC) * kStride + r / VEC];
+        if (partial) {
+            partial[blockIdx.y * m + b0 + r] = static_cast<ACC>(s);
+        } else {
+            const double t = store_y(y, y64, b0 + r, al, s, be);
+            sq += t * t;
+        }
+    }
+    if (coef.sumsq && !partial) block_sumsq_out(sq, coef.sumsq + blockIdx.x);
+}
+
+// y from the column splits' partial sums, in split order, FP64.
+template <class ACC>
+__global__ __launch_bounds__(kThreads) void gemv_n_finish(int64_t m, int splits, const ACC* __restrict__ partial,
+                                                          void* __restrict__ y, bool y64, Coef coef) {
+    if (coef.skip && *coef.skip) return;
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+    double sq = 0.0;
+    if (i < m) {
+        double s = 0.0;
+        for (int c = 0; c < splits; c += 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                v[u] = c + u < splits ? static_cast<double>(partial[static_cast<int64_t>(c + u) * m + i]) : 0.0;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) s += v[u];
+        }
+        const double r = store_y(y, y64, i, read_coef(coef.alpha, coef.dalpha, coef.alpha_mul), s,
+                                 read_coef(coef.beta, coef.dbeta, coef.beta_mul));
+        sq = r * r;
     }
     if (coef.sumsq) block_sumsq_out(sq, coef.sumsq + blockIdx.x);
 }
@@ -688,36 +749,80 @@ Kind classify(int a_type, int tier) {
 }
 
 int vec_full_of(int fmt) { return fmt == FMT_F64 ? 2 : (fmt == FMT_F32 ? 4 : 8); }
+// Bytes of A that an element's product reads.
+constexpr int64_t elem_bytes(int fmt, int dec) {
+    return fmt == FMT_F64 ? 8 : (fmt == FMT_F32 || dec == DEC_EXACT ? 4 : 2);
+}
 int cb_of(const Kind& k) { return k.acc64 ? 32 : 64; }
 constexpr int64_t kTargetBlocks = 1024;
 
-// NO_TRANSPOSE: `waves` = 1 gives every lane its own rows (gemv_n_kernel);
-// more split the columns over the waves of a block (gemv_n_split_kernel)
-// until about kTargetWaves waves share the work, two columns a wave at least.
-constexpr int64_t kTargetWaves = 4096;
-int n_waves(const Kind& k, int64_t m, int64_t n) {
-    const int64_t v = m >= vec_full_of(k.fmt) ? vec_full_of(k.fmt) : 1;
-    const int64_t row_waves = ceil_div(m, 64 * v);
-    const int64_t most = std::min<int64_t>(16, kSplitLds / (v * (k.acc64 ? 8 : 4)));
-    int64_t w = 1;
-    while (w < most && row_waves * w < kTargetWaves && n >= 4 * w) w *= 2;
-    return static_cast<int>(w);
-}
-
-// Row lanes of a split block: 16 while 64-lane blocks are under a quarter of
-// the wanted waves and every column group still has a column.
-int n_row_lanes(int64_t waves64, int64_t n, int waves) {
-    return waves64 < kTargetWaves / 4 && n >= 4 * waves ? 16 : 64;
-}
-
-// Scratch columns of the NO_TRANSPOSE size contract: callers size their
-// scratch by it, the kernels need none.
+// Column splits that the scratch of a NO_TRANSPOSE call holds partial sums
+// of (0: none).
 int n_scratch_splits(const Kind& k, int64_t m, int64_t n) {
     const int64_t bx = ceil_div(m, static_cast<int64_t>(kThreads) * vec_full_of(k.fmt));
     if (bx >= kTargetBlocks / 2 || n <= 16) return 0;
     const int64_t s = std::min(ceil_div(kTargetBlocks, bx), std::min<int64_t>(ceil_div(n, 8), 32));
     const int64_t splits = ceil_div(n, ceil_div(n, s));
     return splits > 1 ? static_cast<int>(splits) : 0;
+}
+
+// NO_TRANSPOSE.  waves = 1: a lane's rows to itself (gemv_n_kernel), from
+// kTargetWaves / 2 waves of rows up (530000 x 50 F32 23.6 us with two waves a
+// block that split the columns, 19.3 without).  Below, the waves of a block
+// split the columns (gemv_n_split_kernel) until about kTargetWaves waves
+// share the work, two columns a wave at least; blocks of 16 row lanes while
+// 64-lane blocks are under a quarter of the wanted waves.  splits > 1: the
+// columns are split over the grid as well (split_pays).
+struct PlanN {
+    int waves, row_lanes, splits;
+    int64_t blocks, split_cols, col_chunk, chain;
+};
+constexpr int64_t kTargetWaves = 4096;
+// Whether `bytes` of A in few blocks are read sooner by more of them, at the
+// cost of a second launch (10 us with the partial sums).  A block reads 75 GB/s
+// of a matrix that the caches hold and 36 (16 row lanes) or 40 of one that
+// they do not, FP32_16's decode bounds it to 28 (hi) and 26 or 40 (EXACT); the
+// chip reads 5.5, 6.2 and 4.8 TB/s.  us, one launch / two: 300 x 100000 F32
+// 390 / 36, 16384 x 10000 bf16 hi 76 / 58, but 16384 x 4000 24 / 32 and 60000 x
+// 1000 EXACT 50 / 62 (these two stay at one).
+bool split_pays(const Kind& k, int64_t blocks, int row_lanes, double bytes) {
+    if (blocks >= 200) return false;
+    const bool cached = bytes <= static_cast<double>(kStreamLoadBytes), p16 = k.fmt == FMT_P16;
+    const double wide = row_lanes == 64 ? 40e3 : 36e3;  // bytes per us
+    const double block = !p16 ? (cached ? 75e3 : wide) : (k.dec == DEC_HI ? 28e3 : row_lanes == 64 ? 40e3 : 26e3);
+    const double chip = p16 ? 4.8e6 : (cached ? 5.5e6 : 6.2e6);
+    return bytes / std::min(static_cast<double>(blocks) * block, chip) > bytes / chip + 10.0;
+}
+constexpr int64_t kSplitWork = int64_t(64) << 10;  // bytes of A for a block of a split at least
+PlanN plan_n(const Kind& k, int64_t m, int64_t n) {
+    PlanN p;
+    const int64_t v = m >= vec_full_of(k.fmt) ? vec_full_of(k.fmt) : 1;
+    const int64_t row_waves = ceil_div(m, 64 * v);
+    const int64_t most = std::min<int64_t>(16, kSplitLds / (v * (k.acc64 ? 8 : 4)));
+    int64_t w = 1;
+    if (row_waves < kTargetWaves / 2)
+        while (w < most && row_waves * w < kTargetWaves && n >= 4 * w) w *= 2;
+    p.waves = static_cast<int>(w);
+    p.row_lanes = row_waves * w < kTargetWaves / 4 && n >= 4 * w ? 16 : 64;
+    p.blocks = w > 1 ? ceil_div(m, p.row_lanes * v) : ceil_div(m, kThreads * v);
+    // FP32 sums run over 8 to 64 columns and meet in FP64: the fewer rows, the
+    // fewer columns, down to n / 32, what a split of the scratch stands for
+    const int64_t parts = n_scratch_splits(k, m, n);
+    p.chain = std::min<int64_t>(std::max<int64_t>(n / std::max<int64_t>(parts, 1) / 8 * 8, 8), 64);
+    p.splits = 1;
+    const int64_t eb = elem_bytes(k.fmt, k.dec);
+    if (w > 1 && split_pays(k, p.blocks, p.row_lanes, static_cast<double>(m) * static_cast<double>(n * eb))) {
+        if (row_waves * parts >= 512) {  // enough blocks with whole 1 KB runs of a column
+            p.row_lanes = 64;
+            p.blocks = row_waves;
+        }
+        const int64_t most_splits = std::min(ceil_div(kTargetBlocks, p.blocks), p.row_lanes * v * n * eb / kSplitWork);
+        p.splits = static_cast<int>(std::max<int64_t>(std::min(parts, most_splits), 1));
+    }
+    p.split_cols = ceil_div(std::max<int64_t>(n, 1), p.splits);
+    p.splits = static_cast<int>(ceil_div(std::max<int64_t>(n, 1), p.split_cols));
+    p.col_chunk = ceil_div(p.split_cols, w * (64 / p.row_lanes));
+    return p;
 }
 
 struct PlanT {
@@ -749,13 +854,8 @@ constexpr int64_t kColBytes = int64_t(128) << 10;
 bool t_waves(int64_t col_bytes, int64_t n) {
     return col_bytes <= (int64_t(24) << 10) && n > (col_bytes <= 4096 ? 4096 : 8192);
 }
-template <int FMT, int DEC>
-constexpr int64_t elem_bytes() {
-    return FMT == FMT_F64 ? 8 : (FMT == FMT_F32 || DEC == DEC_EXACT ? 4 : 2);
-}
 bool t_cols(const Kind& k, int64_t m) {
-    const int64_t esz = k.fmt == FMT_F64 ? 8 : (k.fmt == FMT_F32 || k.dec == DEC_EXACT ? 4 : 2);
-    return m * esz <= kColBytes;
+    return m * elem_bytes(k.fmt, k.dec) <= kColBytes;
 }
 
 // The kind a GEMV runs with: F32 GEMV^T accumulates in FP64 in every tier
@@ -783,47 +883,52 @@ size_t scratch_for(const Kind& k, int trans, int64_t m, int64_t n) {
 // non-temporal, 77 us cacheable).
 template <int FMT, int DEC>
 bool streams(int64_t m, int64_t n, int64_t lda) {
-    return lda % vec_full<FMT>() == 0 && stream_loads(m * n * elem_bytes<FMT, DEC>());
+    return lda % vec_full<FMT>() == 0 && stream_loads(m * n * elem_bytes(FMT, DEC));
 }
 
 template <int FMT, int DEC, int VEC, class ACC, bool NTL>
 int launch_n(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x, bool x64,
-             void* y, bool y64, const Coef& coef, int waves, hipStream_t s) {
-    if (waves > 1) {
-        const int rl = n_row_lanes(ceil_div(m, 64 * VEC) * waves, n, waves);
-        const unsigned blocks = static_cast<unsigned>(ceil_div(m, rl * VEC));
-        const int64_t chunk = ceil_div(n, waves * (64 / rl));
-        if (rl == 16)
-            gemv_n_split_kernel<FMT, DEC, VEC, ACC, 16, NTL><<<blocks, 64 * waves, 0, s>>>(
-                m, n, a, wr, lda, x, x64, y, y64, coef, chunk);
-        else
-            gemv_n_split_kernel<FMT, DEC, VEC, ACC, 64, NTL><<<blocks, 64 * waves, 0, s>>>(
-                m, n, a, wr, lda, x, x64, y, y64, coef, chunk);
-        TOMOS_LAUNCH_CHECK("gemv_n_split_kernel");
+             void* y, bool y64, const Coef& coef, ACC* partial, const PlanN& p, hipStream_t s) {
+    const unsigned blocks = static_cast<unsigned>(p.blocks);
+    if (p.waves == 1) {
+        gemv_n_kernel<FMT, DEC, VEC, ACC, NTL><<<blocks, kThreads, 0, s>>>(m, n, a, wr, lda, x, x64, y, y64, coef,
+                                                                           p.chain);
+        TOMOS_LAUNCH_CHECK("gemv_n_kernel");
         return static_cast<int>(blocks);
     }
-    const unsigned blocks = static_cast<unsigned>(ceil_div(m, static_cast<int64_t>(kThreads) * VEC));
-    gemv_n_kernel<FMT, DEC, VEC, ACC, NTL><<<blocks, kThreads, 0, s>>>(m, n, a, wr, lda, x, x64, y, y64, coef);
-    TOMOS_LAUNCH_CHECK("gemv_n_kernel");
-    return static_cast<int>(blocks);
+    const dim3 grid(blocks, static_cast<unsigned>(p.splits));
+    const size_t lds = static_cast<size_t>(p.waves) * VEC * (p.row_lanes + 1) * sizeof(double);
+    if (p.row_lanes == 16)
+        gemv_n_split_kernel<FMT, DEC, VEC, ACC, 16, NTL><<<grid, 64 * p.waves, lds, s>>>(
+            m, n, a, wr, lda, x, x64, y, y64, coef, p.split_cols, p.col_chunk, p.chain, partial);
+    else
+        gemv_n_split_kernel<FMT, DEC, VEC, ACC, 64, NTL><<<grid, 64 * p.waves, lds, s>>>(
+            m, n, a, wr, lda, x, x64, y, y64, coef, p.split_cols, p.col_chunk, p.chain, partial);
+    TOMOS_LAUNCH_CHECK("gemv_n_split_kernel");
+    if (!partial) return static_cast<int>(blocks);
+    const unsigned fb = static_cast<unsigned>(ceil_div(m, kThreads));
+    gemv_n_finish<ACC><<<fb, kThreads, 0, s>>>(m, p.splits, partial, y, y64, coef);
+    TOMOS_LAUNCH_CHECK("gemv_n_finish");
+    return static_cast<int>(fb);
 }
 
 template <int FMT, int DEC, class ACC>
 int run_n(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x,
-          bool x64, void* y, bool y64, const Coef& coef, int waves, hipStream_t s) {
+          bool x64, void* y, bool y64, const Coef& coef, void* scratch, const PlanN& p, hipStream_t s) {
     constexpr int VF = vec_full<FMT>();
+    ACC* part = static_cast<ACC*>(scratch);
     if (m < VF)
-        return launch_n<FMT, DEC, 1, ACC, false>(m, n, a, wr, lda, x, x64, y, y64, coef, waves, s);
+        return launch_n<FMT, DEC, 1, ACC, false>(m, n, a, wr, lda, x, x64, y, y64, coef, part, p, s);
     if (streams<FMT, DEC>(m, n, lda))
-        return launch_n<FMT, DEC, VF, ACC, true>(m, n, a, wr, lda, x, x64, y, y64, coef, waves, s);
-    return launch_n<FMT, DEC, VF, ACC, false>(m, n, a, wr, lda, x, x64, y, y64, coef, waves, s);
+        return launch_n<FMT, DEC, VF, ACC, true>(m, n, a, wr, lda, x, x64, y, y64, coef, part, p, s);
+    return launch_n<FMT, DEC, VF, ACC, false>(m, n, a, wr, lda, x, x64, y, y64, coef, part, p, s);
 }
 
 template <int FMT, int DEC, int VEC, class ACC, bool NTL>
 void launch_t_cols(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, const void* x, bool x64,
                    ACC* part, void* y, bool y64, const Coef& coef, hipStream_t s) {
     // one column a block while that fills the chip about twice, then two, then four
-    if (t_waves(m * elem_bytes<FMT, DEC>(), n))
+    if (t_waves(m * elem_bytes(FMT, DEC), n))
         gemv_t_wave_kernel<FMT, DEC, VEC, ACC, kWaveCols, NTL>
             <<<static_cast<unsigned>(std::min(ceil_div(n, kWaveCols * (kThreads / 64)), kWaveBlocks)), kThreads, 0, s>>>(
                 m, n, a, wr, lda, x, x64, part, y, y64, coef);
@@ -853,7 +958,7 @@ int run_t(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, 
             launch_t_cols<FMT, DEC, 1, ACC, false>(m, n, a, wr, lda, x, x64, one, y, y64, coef, s);
         // non-temporal above what the last-level cache holds (60000 x 2000
         // bf16 hi, 240 MB, again and again: 36 us cacheable, 41 not)
-        else if (DEC != DEC_EXACT && m * n * elem_bytes<FMT, DEC>() > (int64_t(256) << 20) && streams<FMT, DEC>(m, n, lda))
+        else if (DEC != DEC_EXACT && m * n * elem_bytes(FMT, DEC) > (int64_t(256) << 20) && streams<FMT, DEC>(m, n, lda))
             launch_t_cols<FMT, DEC, VF, ACC, true>(m, n, a, wr, lda, x, x64, one, y, y64, coef, s);
         else
             launch_t_cols<FMT, DEC, VF, ACC, false>(m, n, a, wr, lda, x, x64, one, y, y64, coef, s);
@@ -921,11 +1026,15 @@ void gemv(int a_type, int tier, int trans, const Coef& coef, int64_t m, int64_t 
     if (inner > 0) require(a != nullptr && x != nullptr, "gemv: null A or x");
     if (k.dec == DEC_EXACT) require(wr != nullptr || inner == 0, "gemv: EXACT tier needs the wr plane");
     const size_t need = scratch_for(k, trans, m, n);
-    // y over x: the products of the row chunks are complete before y is written
-    const bool cols = trans == TOMOS_TRANSPOSE && m > 0 && t_cols(k, m) && !overlap(x, x_type, m, y, y_type, n);
+    // y over x: by partial sums, which are complete before y is written
+    const bool in_place = overlap(x, x_type, inner, y, y_type, rows_out);
+    const bool cols = trans == TOMOS_TRANSPOSE && m > 0 && t_cols(k, m) && !in_place;
+    PlanN pn{};
+    if (trans == TOMOS_NO_TRANSPOSE) pn = plan_n(k, m, n);
+    const bool parts = pn.splits > 1 || (in_place && pn.waves > 1 && need > 0);
     if (need > 0) {
         if (scratch == nullptr) {
-            if (trans == TOMOS_TRANSPOSE && !cols) scratch = fallback_scratch(need);
+            if (trans == TOMOS_TRANSPOSE ? !cols : parts) scratch = fallback_scratch(need);
         } else {
             require(scratch_bytes >= need, "gemv: scratch too small (need " + std::to_string(need) +
                                                " bytes)");
@@ -935,9 +1044,8 @@ void gemv(int a_type, int tier, int trans, const Coef& coef, int64_t m, int64_t 
 
     if (trans == TOMOS_NO_TRANSPOSE) {
         // n == 0 falls through with an empty column range: y = beta*y.
-        const int waves = n_waves(k, m, n);
         int nb = 0;
-#define RUN_N(F, D, A) nb = run_n<F, D, A>(m, n, a, wr, lda, x, x64, y, y64, coef, waves, s)
+#define RUN_N(F, D, A) nb = run_n<F, D, A>(m, n, a, wr, lda, x, x64, y, y64, coef, parts ? scratch : nullptr, pn, s)
         if (k.fmt == FMT_F32) { if (k.acc64) RUN_N(FMT_F32, DEC_NATIVE, double); else RUN_N(FMT_F32, DEC_NATIVE, float); }
         else if (k.fmt == FMT_F64) RUN_N(FMT_F64, DEC_NATIVE, double);
         else if (k.fmt == FMT_H16) { if (k.acc64) RUN_N(FMT_H16, DEC_HI, double); else RUN_N(FMT_H16, DEC_HI, float); }
