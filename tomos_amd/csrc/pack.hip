@@ -9,6 +9,8 @@
 // column.  Grid = (row runs, columns): coalesced along rows, HBM-bound (8 B
 // moved per element).  500000 x 301 FP32_16: pack 221 -> 212 us (5.7 TB/s),
 // exact unpack 400 (2-byte loads, scalar decode) -> 213 us (5.7 TB/s).
+#include <algorithm>
+
 #include "codec.hpp"
 #include "common.hpp"
 #include "tomos_hip.h"
@@ -82,64 +84,65 @@ constexpr int kTileRows = 128, kTileCols = 64;
 // a row, 4 rows) hit 64 different banks, those that it loads (every eighth
 // row, 16 lanes a column, 4 columns) 32.
 constexpr int kTilePitch = kTileRows + 1;
+constexpr int64_t kTileBlocks = int64_t(1) << 20;  // further tiles in a loop: 2^32 work items bound a launch
 
 template <int VARIANT>
 __global__ __launch_bounds__(256) void pack_rows_kernel(int64_t m, int64_t n, const float* __restrict__ src,
                                                         int64_t ld_src, uint16_t* __restrict__ wh,
                                                         uint16_t* __restrict__ wr, int64_t ld_dst,
-                                                        int64_t col_tiles) {
+                                                        int64_t row_tiles, int64_t col_tiles) {
     __shared__ uint32_t tile[kTileCols * kTilePitch];
-    const int64_t rt = blockIdx.x / col_tiles;
-    const int64_t i0 = rt * kTileRows, j0 = (blockIdx.x - rt * col_tiles) * kTileCols;
     const int t = threadIdx.x;
-    {
-        const int c = (t & 15) * 4, r = t >> 4;
-        const bool whole = j0 + c + 4 <= n;
+    for (int64_t g = blockIdx.x; g < row_tiles * col_tiles; g += gridDim.x) {
+        const int64_t rt = g / col_tiles;
+        const int64_t i0 = rt * kTileRows, j0 = (g - rt * col_tiles) * kTileCols;
+        const int c0 = (t & 15) * 4, r = t >> 4;
+        const bool whole = j0 + c0 + 4 <= n;
         f32x4 v[kTileRows / 16];
 #pragma unroll
         for (int q = 0; q < kTileRows / 16; ++q) {
             const int64_t i = i0 + r + 16 * q;
             v[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             if (i >= m) continue;
-            const float* s = src + i * ld_src + j0 + c;
+            const float* s = src + i * ld_src + j0 + c0;
             if (whole) {
                 v[q] = load16<f32x4>(s);
             } else {
 #pragma unroll
                 for (int k = 0; k < 4; ++k)
-                    if (j0 + c + k < n) v[q][k] = s[k];
+                    if (j0 + c0 + k < n) v[q][k] = s[k];
             }
         }
+        if (g != static_cast<int64_t>(blockIdx.x)) __syncthreads();  // the last tile has been read
 #pragma unroll
         for (int q = 0; q < kTileRows / 16; ++q)
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 uint16_t h, l;
                 encode<VARIANT>(v[q][k], h, l);
-                tile[(c + k) * kTilePitch + r + 16 * q] = h | (uint32_t(l) << 16);
+                tile[(c0 + k) * kTilePitch + r + 16 * q] = h | (uint32_t(l) << 16);
             }
-    }
-    __syncthreads();
-    const int i = (t & 15) * kRun;
-    const int64_t left = m - i0 - i;
-    if (left <= 0) return;
-    for (int c = t >> 4; c < kTileCols && j0 + c < n; c += 16) {
-        const uint32_t* w = tile + c * kTilePitch + i;
-        uint16_t* h = wh + (j0 + c) * ld_dst + i0 + i;
-        uint16_t* r = wr + (j0 + c) * ld_dst + i0 + i;
-        if (left >= kRun) {
-            u32x4 ph, pr;
+        __syncthreads();
+        const int i = (t & 15) * kRun;
+        const int64_t left = m - i0 - i;
+        for (int c = t >> 4; c < kTileCols && j0 + c < n && left > 0; c += 16) {
+            const uint32_t* w = tile + c * kTilePitch + i;
+            uint16_t* h = wh + (j0 + c) * ld_dst + i0 + i;
+            uint16_t* l = wr + (j0 + c) * ld_dst + i0 + i;
+            if (left >= kRun) {
+                u32x4 ph, pl;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                ph[k] = (w[2 * k] & 0xFFFFu) | (w[2 * k + 1] << 16);
-                pr[k] = (w[2 * k] >> 16) | (w[2 * k + 1] & 0xFFFF0000u);
-            }
-            store16(h, ph);
-            store16(r, pr);
-        } else {
-            for (int k = 0; k < static_cast<int>(left); ++k) {
-                h[k] = static_cast<uint16_t>(w[k] & 0xFFFFu);
-                r[k] = static_cast<uint16_t>(w[k] >> 16);
+                for (int k = 0; k < 4; ++k) {
+                    ph[k] = (w[2 * k] & 0xFFFFu) | (w[2 * k + 1] << 16);
+                    pl[k] = (w[2 * k] >> 16) | (w[2 * k + 1] & 0xFFFF0000u);
+                }
+                store16(h, ph);
+                store16(l, pl);
+            } else {
+                for (int k = 0; k < static_cast<int>(left); ++k) {
+                    h[k] = static_cast<uint16_t>(w[k] & 0xFFFFu);
+                    l[k] = static_cast<uint16_t>(w[k] >> 16);
+                }
             }
         }
     }
@@ -225,9 +228,19 @@ __global__ __launch_bounds__(256) void decode_wh_kernel(int64_t count,
 
 // A matrix whose columns follow each other without padding on both sides is
 // one column of m * n rows: whole runs throughout and aligned ones if the
-// first is.
+// first is.  Not where one launch dimension cannot hold that column: HIP takes
+// fewer than 2^32 work items in each (2^35 rows here).
+constexpr bool one_column(int64_t m, int64_t n, int64_t ld_src, int64_t ld_dst) {
+    return ld_src == m && ld_dst == m && n <= (int64_t(1) << 35) / m &&
+           (m * n + 256 * kRun - 1) / (256 * kRun) * 256 < (int64_t(1) << 32);
+}
+static_assert(one_column(2000000, 1000, 2000000, 2000000) && one_column(1 << 20, (1 << 15) - 1, 1 << 20, 1 << 20) &&
+                  !one_column(1 << 20, 1 << 15, 1 << 20, 1 << 20) && !one_column(35000000, 1000, 35000000, 35000000) &&
+                  !one_column(int64_t(1) << 40, int64_t(1) << 30, int64_t(1) << 40, int64_t(1) << 40) &&
+                  !one_column(8, 3, 9, 8),
+              "an unpadded matrix is one column up to 2^35 elements");
 void flatten(int64_t& m, int64_t& n, int64_t& ld_src, int64_t& ld_dst) {
-    if (ld_src == m && ld_dst == m && m * n < (int64_t(1) << 40)) {
+    if (one_column(m, n, ld_src, ld_dst)) {
         m *= n;
         n = 1;
         ld_src = ld_dst = m;
@@ -238,8 +251,8 @@ template <int VARIANT>
 void launch_pack_rows(int64_t m, int64_t n, const float* src, int64_t ld_src, uint16_t* wh, uint16_t* wr,
                       int64_t ld_dst, hipStream_t s) {
     const int64_t ct = ceil_div(n, static_cast<int64_t>(kTileCols)), rt = ceil_div(m, static_cast<int64_t>(kTileRows));
-    require(rt <= 2147483647 / ct, "tomos_pack_rows: too many tiles");
-    pack_rows_kernel<VARIANT><<<static_cast<unsigned>(rt * ct), 256, 0, s>>>(m, n, src, ld_src, wh, wr, ld_dst, ct);
+    const unsigned blocks = static_cast<unsigned>(std::min(rt * ct, kTileBlocks));
+    pack_rows_kernel<VARIANT><<<blocks, 256, 0, s>>>(m, n, src, ld_src, wh, wr, ld_dst, rt, ct);
     TOMOS_LAUNCH_CHECK("pack_rows_kernel");
 }
 
