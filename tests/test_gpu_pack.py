@@ -156,3 +156,30 @@ def test_pack_rows_equals_pack(capi, orc, m, n, pad_src, pad_dst, shift):
         assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1]), variant
     assert C.lib().tomos_pack_rows(0, m, n, ctypes.c_void_p(src.ptr), n - 1, ctypes.c_void_p(src.ptr),
                                    ctypes.c_void_p(src.ptr), ld, None) == 1
+
+
+@pytest.mark.parametrize("m", [1, 7, 8, 9, 16, 17, 100, 1024, 1025])
+@pytest.mark.parametrize("n", [2, 31, 257])
+def test_short_padded_columns(capi, orc, m, n):
+    """Several columns a block: row counts around the powers of two that halve
+    a column's share of the block, column counts that leave part of one, odd
+    leading dimensions; nothing is written past row m."""
+    rng = np.random.default_rng(m * n)
+    A = (rng.standard_normal((m, n)) * 2.0 ** rng.integers(-30, 30, (m, n))).astype(np.float32)
+    lds, ld = m + 3, m + 5
+    src = np.full((lds, n), 5.0, np.float32, order="F")
+    src[:m] = A
+    print("short columns", m, n, flush=True)
+    for variant, dec in ((0, 0), (3, 4)):
+        eh, er = orc.pack(variant, A)
+        wh, wr = H.dev(np.full((ld, n), 0x1111, np.uint16)), H.dev(np.full((ld, n), 0x1111, np.uint16))
+        sd = H.dev(src)
+        C.call("tomos_pack", variant, m, n, sd.ptr, lds, wh.ptr, wr.ptr, ld, None)
+        gh, gr = H.from_dev16(wh, ld, n), H.from_dev16(wr, ld, n)
+        assert np.array_equal(gh[:m], eh) and np.array_equal(gr[:m], er)
+        assert np.all(gh[m:] == 0x1111) and np.all(gr[m:] == 0x1111)
+        out = H.dev(np.full((lds, n), -7.0, np.float32))
+        C.call("tomos_unpack", dec, m, n, wh.ptr, wr.ptr, ld, out.ptr, lds, None)
+        got = out.to_numpy(np.float32, (lds, n))
+        assert np.array_equal(got[:m].view(np.uint32), orc.unpack(dec, eh, er).astype(np.float32).view(np.uint32))
+        assert np.all(got[m:] == -7.0)

@@ -45,12 +45,12 @@ __device__ __forceinline__ void store16(void* p, V v) {
 }
 
 template <int VARIANT>
-__global__ __launch_bounds__(256) void pack_kernel(int64_t m, const float* __restrict__ src,
+__global__ __launch_bounds__(256) void pack_kernel(int64_t m, int64_t n, const float* __restrict__ src,
                                                    int64_t ld_src, uint16_t* __restrict__ wh,
                                                    uint16_t* __restrict__ wr, int64_t ld_dst) {
-    const int64_t j = blockIdx.y;
+    const int64_t j = static_cast<int64_t>(blockIdx.y) * blockDim.y + threadIdx.y;
     const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * kRun;
-    if (i0 >= m) return;
+    if (i0 >= m || j >= n) return;
     const float* s = src + j * ld_src + i0;
     uint16_t* h = wh + j * ld_dst + i0;
     uint16_t* r = wr + j * ld_dst + i0;
@@ -172,13 +172,13 @@ constexpr bool needs_wr() {
 }
 
 template <int DEC>
-__global__ __launch_bounds__(256) void unpack_kernel(int64_t m, const uint16_t* __restrict__ wh,
+__global__ __launch_bounds__(256) void unpack_kernel(int64_t m, int64_t n, const uint16_t* __restrict__ wh,
                                                      const uint16_t* __restrict__ wr,
                                                      int64_t ld_src, float* __restrict__ dst,
                                                      int64_t ld_dst) {
-    const int64_t j = blockIdx.y;
+    const int64_t j = static_cast<int64_t>(blockIdx.y) * blockDim.y + threadIdx.y;
     const int64_t i0 = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * kRun;
-    if (i0 >= m) return;
+    if (i0 >= m || j >= n) return;
     const uint16_t* h = wh + j * ld_src + i0;
     const uint16_t* r = needs_wr<DEC>() ? wr + j * ld_src + i0 : nullptr;
     float* d = dst + j * ld_dst + i0;
@@ -247,6 +247,19 @@ void flatten(int64_t& m, int64_t& n, int64_t& ld_src, int64_t& ld_dst) {
     }
 }
 
+// A block's 256 threads take runs of one column, or of several where the
+// columns are short: padded columns of 100 rows left 243 threads without a
+// run (unpack of 100 x 100000, exact FP32_16: 74 -> 24 us).
+struct RunShape {
+    dim3 grid, block;
+};
+RunShape run_shape(int64_t m, int64_t n) {
+    unsigned tx = 256;
+    while (tx > 1 && n > 1 && static_cast<int64_t>(tx / 2) * kRun >= m) tx /= 2;
+    const unsigned ty = 256 / tx;
+    return {dim3(static_cast<unsigned>(ceil_div(m, tx * kRun)), static_cast<unsigned>(ceil_div(n, ty))), dim3(tx, ty)};
+}
+
 template <int VARIANT>
 void launch_pack_rows(int64_t m, int64_t n, const float* src, int64_t ld_src, uint16_t* wh, uint16_t* wr,
                       int64_t ld_dst, hipStream_t s) {
@@ -260,8 +273,8 @@ template <int VARIANT>
 void launch_pack(int64_t m, int64_t n, const float* src, int64_t ld_src, uint16_t* wh,
                  uint16_t* wr, int64_t ld_dst, hipStream_t s) {
     flatten(m, n, ld_src, ld_dst);
-    const dim3 grid(static_cast<unsigned>(ceil_div(m, 256 * kRun)), static_cast<unsigned>(n));
-    pack_kernel<VARIANT><<<grid, 256, 0, s>>>(m, src, ld_src, wh, wr, ld_dst);
+    const RunShape r = run_shape(m, n);
+    pack_kernel<VARIANT><<<r.grid, r.block, 0, s>>>(m, n, src, ld_src, wh, wr, ld_dst);
     TOMOS_LAUNCH_CHECK("pack_kernel");
 }
 
@@ -269,8 +282,8 @@ template <int DEC>
 void launch_unpack(int64_t m, int64_t n, const uint16_t* wh, const uint16_t* wr, int64_t ld_src,
                    float* dst, int64_t ld_dst, hipStream_t s) {
     flatten(m, n, ld_src, ld_dst);
-    const dim3 grid(static_cast<unsigned>(ceil_div(m, 256 * kRun)), static_cast<unsigned>(n));
-    unpack_kernel<DEC><<<grid, 256, 0, s>>>(m, wh, wr, ld_src, dst, ld_dst);
+    const RunShape r = run_shape(m, n);
+    unpack_kernel<DEC><<<r.grid, r.block, 0, s>>>(m, n, wh, wr, ld_src, dst, ld_dst);
     TOMOS_LAUNCH_CHECK("unpack_kernel");
 }
 
