@@ -409,3 +409,22 @@ def test_sketch_does_not_depend_on_alignment(capi, a_type, m, n, s, pad):
             wh, wr = H.pack(variant, A, ld=lda)
             out.append(H.countsketch_apply(a_type, C.TIER_EXACT, m, n, wh, wr, lda, s))
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("s", [20448, 20449, 32768])
+@pytest.mark.parametrize("pad", [0, 1])
+def test_sketch_bucket_limits(capi, orc, s, pad):
+    """Both sides of the bucket count that fits LDS as 64-bit integers, and
+    the largest: columns at any alignment.  Few rows a bucket: FP32 sums of
+    small integers are exact on either path."""
+    m, n = 30001, 3
+    rng = np.random.default_rng(s)
+    lda = (m + 7) // 8 * 8 + pad
+    A = np.zeros((lda, n), np.float32, order="F")
+    A[:m] = rng.integers(-100, 101, (m, n))
+    print("buckets", s, pad, flush=True)
+    got = H.countsketch_apply(C.F32, C.TIER_DEFAULT, m, n, H.dev(A), None, lda, s)
+    bucket, sign = H.countsketch_indices(m, s)
+    ref = np.zeros((s, n))
+    np.add.at(ref, bucket, sign[:, None] * A[:m].astype(np.float64))
+    assert np.array_equal(got, ref)

@@ -711,6 +711,9 @@ void launch_apply_cg(const CsPlan& p, int64_t m, int64_t n, const void* a, const
 constexpr int64_t kSampleSegs = 32;
 constexpr int64_t kSampleMinRows = 16384;  // the sample is at most 1/8 of the rows
 constexpr int kSampleMargin = 12;           // 2^-31 of the sampled max per term at 2e6 rows, 4 splits
+// Buckets of one column that fit LDS as 64-bit integers, next to the kernel's
+// own 256 bytes; more take the float path.
+constexpr int64_t kFxMaxBuckets = (160 * 1024 - 256) / 8;
 
 // Enqueue the fixed-point path with the exponents from a sample (sample)
 // or from every row, reading nothing back: flags[0] is set if a column's
@@ -795,6 +798,7 @@ template <int FMT, bool EXACT>
 bool try_apply_fx(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, int64_t s,
                   const uint32_t* packed, char* scratch, const CsLayout& L, double* y, int64_t ldy,
                   hipStream_t st) {
+    if (s > kFxMaxBuckets) return false;
     if (!aligned16<FMT>(a, wr, lda, EXACT)) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         TOMOS_HIP_CHECK(hipStreamIsCapturing(st, &cap));
