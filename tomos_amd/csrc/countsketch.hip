@@ -452,11 +452,14 @@ __device__ __forceinline__ void cs_apply_fx_rows(
     int sc[CG];
     double scale[CG];
     float bnd[CG];  // |value| < 2^e_c keeps every term below 2^shift (no overflow)
+    // uniform, and kept in SGPRs: in VGPRs, 24 for 8 columns, they made FP32_BF16
+    // EXACT spill 40 (1000000 x 50 147 us, so 120)
 #pragma unroll
     for (int c = 0; c < CG; ++c) {
-        sc[c] = c < ncols ? shift - colexp[c0 + c] : 0;
-        scale[c] = MAGIC ? ldexp(1.0, sc[c]) : 0.0;
-        bnd[c] = c < ncols ? ldexpf(1.0f, colexp[c0 + c]) : 0.0f;
+        sc[c] = __builtin_amdgcn_readfirstlane(c < ncols ? shift - colexp[c0 + c] : 0);
+        scale[c] = __builtin_bit_cast(double, static_cast<uint64_t>(1023 + sc[c]) << 52);  // -111 <= sc <= 209
+        bnd[c] = codec::u2f(
+            __builtin_amdgcn_readfirstlane(codec::f2u(c < ncols ? ldexpf(1.0f, colexp[c0 + c]) : 0.0f)));
     }
     bool beyond = false;  // a value at or above its column's bound (or not finite)
     __syncthreads();
