@@ -378,6 +378,8 @@ int tomos_csr_sketch(int kind, int val_type, int idx_type, int64_t rows, int64_t
  * A m x n in any a_type/tier (packed A is decoded per tier).  Y is
  * overwritten.  Replaces countsketch_apply_matrix_hashed
  * (countsketch_cuda_kernels.cu:253-285, host :435-450) and the CPU apply.
+ * Asynchronous on `stream` (with a scratch buffer it can be captured); with
+ * NULL scratch and columns on 16-byte boundaries it waits for the stream.
  * scratch: tomos_countsketch_scratch_size() bytes or NULL. */
 size_t tomos_countsketch_scratch_size(int64_t m, int64_t n, int64_t s);
 int tomos_countsketch_apply(int a_type, int tier, int64_t m, int64_t n, const void* a,

@@ -428,3 +428,55 @@ def test_sketch_bucket_limits(capi, orc, s, pad):
     ref = np.zeros((s, n))
     np.add.at(ref, bucket, sign[:, None] * A[:m].astype(np.float64))
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("m", [1001, 20001])
+@pytest.mark.parametrize("pad", [0, 1])
+def test_sketch_is_asynchronous(capi, m, pad):
+    """The call reads nothing back, whatever the columns' alignment: it can be
+    captured, and replays equal plain calls on values that the first attempt's
+    exponents hold for, that they do not (an outlier outside the sampled
+    rows) and that are not finite (the float path: its sums of these integers
+    are exact)."""
+    torch = pytest.importorskip("torch")
+    n, s = 9, 300
+    lda = (m + 7) // 8 * 8 + pad
+    g = torch.Generator(device="cuda").manual_seed(m)
+    plain = torch.randint(-100, 101, (n, lda), generator=g, device="cuda").float()
+    outlier, inf = plain.clone(), plain.clone()
+    outlier[4, 70] = 2.0 ** 22  # segments of 64..1024 rows start every m / 32 rows: 70 is past the first
+    outlier[4, 600] = 2.0 ** 22
+    inf[2, m - 1] = float("inf")
+    a, y = plain.clone(), torch.zeros((n, s), dtype=torch.float64, device="cuda")
+    nb = C.lib().tomos_countsketch_scratch_size(m, n, s)
+    sc = torch.empty(nb, dtype=torch.uint8, device="cuda")
+
+    def call():
+        C.call("tomos_countsketch_apply", C.F32, C.TIER_DEFAULT, m, n, a.data_ptr(), None, lda, s, y.data_ptr(), s,
+               sc.data_ptr(), nb, torch.cuda.current_stream().cuda_stream)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for values in (plain, outlier, inf, plain, inf, outlier, plain):
+        a.copy_(values)
+        y.fill_(-1.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = y.clone()
+        y.fill_(-2.0)
+        call()
+        torch.cuda.synchronize()
+        assert torch.equal(torch.nan_to_num(replayed, nan=7.0), torch.nan_to_num(y, nan=7.0))
+        bad = ~torch.isfinite(y)
+        assert bool(bad.any()) == (values is inf)
+        bucket, sign = H.countsketch_indices(m, s)
+        ref = np.zeros((s, n))
+        with np.errstate(invalid="ignore"):
+            np.add.at(ref, bucket, sign[:, None] * values[:, :m].t().double().cpu().numpy())
+        assert np.array_equal(y.t().cpu().numpy(), ref, equal_nan=True)

@@ -14,9 +14,10 @@
 // and adds sign*A[i,j] into LDS: CG (or 2 CG) independent 16-byte loads per
 // lane are in flight, and the index words are read once per column group.
 // The LDS slice is written to a per-split partial, and a second pass sums
-// the splits in a fixed order in FP64.  Bucket/sign indices are bit-exact;
-// the values are FP32 sums within a split (order depends on LDS atomic
-// order), FP64 across splits.
+// the splits in a fixed order.  Bucket/sign indices are bit-exact; the values
+// are exact fixed-point sums or, where those do not apply (a column that is
+// not finite, more buckets than LDS holds as 64-bit integers), FP32 sums
+// within a split (order depends on LDS atomic order) and FP64 across splits.
 #include <algorithm>
 #include <type_traits>
 #include <vector>
@@ -38,12 +39,16 @@ __device__ __forceinline__ uint64_t splitmix64(uint64_t x) {
     return x ^ (x >> 31);
 }
 
-// packed word: bucket in bits 0..30, bit 31 set for sign -1
+// packed word: bucket in bits 0..30, bit 31 set for sign -1; the call's
+// kFlags flags are cleared on the way
+constexpr int kFlags = 4;
 __global__ __launch_bounds__(256) void cs_index_kernel(int64_t m, int64_t s,
                                                        int32_t* __restrict__ bucket,
                                                        int8_t* __restrict__ sign,
-                                                       uint32_t* __restrict__ packed) {
+                                                       uint32_t* __restrict__ packed,
+                                                       int* __restrict__ flags) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (flags && i < kFlags) flags[i] = 0;
     if (i >= m) return;
     const uint64_t hb = splitmix64(static_cast<uint64_t>(i) ^ kBucketSeed);
     const uint64_t hs = splitmix64(static_cast<uint64_t>(i) ^ kSignSeed);
@@ -145,12 +150,17 @@ __device__ __forceinline__ uint4 load_rows16(const void* p) {
     return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+// Whether a launch with this gate (nullptr, or the two flags of an earlier
+// attempt) has nothing to do: the attempt held.
+__device__ __forceinline__ bool gated_off(const int* __restrict__ gate) { return gate && !(gate[0] | gate[1]); }
+
 // rows_per_split is a multiple of the row vector (of the index words too).
 template <int FMT, bool EXACT, int CG>
 __global__ __launch_bounds__(kVecThreads) void cs_apply_vec_kernel(
     int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr, int64_t lda,
     int64_t s, const uint32_t* __restrict__ packed, int64_t rows_per_split, int ncg,
-    float* __restrict__ partial) {
+    float* __restrict__ partial, const int* __restrict__ gate) {
+    if (gated_off(gate)) return;
     constexpr int V = vec_rows<FMT>();
     constexpr int EB = 16 / V;  // bytes per element of the a plane
     extern __shared__ float ylds[];  // [CG][s]
@@ -225,7 +235,9 @@ __global__ __launch_bounds__(kVecThreads) void cs_apply_vec_kernel(
 
 __global__ __launch_bounds__(256) void cs_finish_kernel(int64_t s, int64_t n, int splits,
                                                         const float* __restrict__ partial,
-                                                        double* __restrict__ y, int64_t ldy) {
+                                                        double* __restrict__ y, int64_t ldy,
+                                                        const int* __restrict__ gate) {
+    if (gated_off(gate)) return;
     const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (t >= s * n) return;
     const int64_t c = t / s;
@@ -237,9 +249,9 @@ __global__ __launch_bounds__(256) void cs_finish_kernel(int64_t s, int64_t n, in
 
 // ---- fixed-point path ------------------------------------------------------
 // LDS float atomics are the bottleneck of the scatter (about 7x slower than
-// 64-bit integer LDS atomics on gfx950), so the vector path accumulates in
-// fixed point instead: a first pass finds each column's largest hi-plane
-// magnitude, giving an exponent e_j with |A[i,j]| < 2^e_j for every row
+// 64-bit integer LDS atomics on gfx950), so the sums are kept in fixed point
+// instead: a first pass finds each column's largest hi-plane magnitude (over a
+// sample or all rows), giving an exponent e_j with |A[i,j]| < 2^e_j for every row
 // (one bit of margin covers the exact value vs its hi word); each value is
 // then added as the 64-bit integer round(v * 2^(shift - e_j)), with
 // shift = 62 - H and 2^H > rows per split, so a bucket's sum cannot
@@ -247,46 +259,6 @@ __global__ __launch_bounds__(256) void cs_finish_kernel(int64_t s, int64_t n, in
 // deterministic; the resolution is 2^-shift of the column's magnitude
 // (2^-42 at 2e6 rows and 4 splits).  Columns whose max is not finite (Inf
 // or NaN from saturated FP32_16 words) take the float path for the call.
-
-// colmax_bits[j] = max over rows of |value| as float bits (monotone for
-// non-negative floats) of the values the sketch sums, or (BOUND_HI) of the
-// hi words, which bound the exact FP32_BF16 values within a factor 2.
-// grid (n, segments): segment y covers rows [y stride, y stride + len)
-// (stride == len: every row; stride > len: a sample); 16-byte row vectors.
-template <int FMT, bool EXACT, bool NTL>
-__global__ __launch_bounds__(256) void cs_colmax_kernel(int64_t m, const void* __restrict__ a,
-                                                        const uint16_t* __restrict__ wr, int64_t lda,
-                                                        int64_t stride, int64_t len,
-                                                        unsigned* __restrict__ colmax_bits) {
-    constexpr int V = vec_rows<FMT>();
-    constexpr int EB = 16 / V;
-    const int64_t j = blockIdx.x;
-    const int64_t r0 = static_cast<int64_t>(blockIdx.y) * stride;
-    const int64_t r1 = min(m, r0 + len);
-    const char* col = static_cast<const char*>(a) + j * lda * EB;
-    float mx = 0.0f;
-    for (int64_t i0 = r0 + static_cast<int64_t>(threadIdx.x) * V; i0 < r1; i0 += 256 * V) {
-        float v[V];
-        if (i0 + V <= r1) {
-            const uint4 h = load_rows16<NTL>(col + i0 * EB);
-            uint4 l = make_uint4(0, 0, 0, 0);
-            if constexpr (EXACT) l = load_rows16<NTL>(wr + i0 + j * lda);
-            decode_rows<FMT, EXACT>(h, l, v);
-        } else {
-            for (int r = 0; r < V; ++r) v[r] = (i0 + r < r1) ? load_elem<FMT, EXACT>(a, wr, i0 + r + j * lda) : 0.0f;
-        }
-#pragma unroll
-        for (int r = 0; r < V; ++r) {
-            const float av = fabsf(v[r]);
-            mx = (av > mx || av != av) ? av : mx;  // NaN wins
-        }
-    }
-    for (int o = 32; o >= 1; o >>= 1) {
-        const float other = __shfl_xor(mx, o);
-        mx = (other > mx || other != other) ? other : mx;
-    }
-    if ((threadIdx.x & 63) == 0) atomicMax(colmax_bits + j, __float_as_uint(mx));
-}
 
 // e_j from the max bits, plus `margin` bits when the max is a sample's;
 // flag = 1 if the column is not finite
@@ -305,30 +277,23 @@ __device__ __forceinline__ void cs_set_exponent(unsigned bits, int margin, int* 
     *colexp = e + margin;
 }
 
-__global__ __launch_bounds__(256) void cs_colexp_kernel(int64_t n, const unsigned* __restrict__ colmax_bits,
-                                                        int margin, int* __restrict__ colexp,
-                                                        int* __restrict__ flag) {
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (j >= n) return;
-    cs_set_exponent(colmax_bits[j], margin, colexp + j, flag);
-}
-
-// Sampled exponents in one pass, one block per column: the max over `segs`
+// A column's exponent, one block per column: the max of |value| (of the hi
+// words, which bound the exact FP32_BF16 values within a factor 2) over `segs`
 // segments of `len` rows (starts `stride` apart; len a multiple of 8) reduced
 // in the block, then e_j + margin written directly.  The whole sample of a
 // column is one block's work, so no column max crosses blocks (no atomics
 // to one address from many blocks, no cleared buffer).  segs = 1, stride =
-// 0, len = m rounded up to 8 and margin 0 give the exact exponents.
+// 0, len = m rounded up to 8 and margin 0 take every row.
 template <int FMT, bool EXACT>
 __device__ __forceinline__ void cs_sample_exp_body(int64_t j, int64_t m, const void* __restrict__ a,
                                                    const uint16_t* __restrict__ wr, int64_t lda, int64_t stride,
-                                                   int len, int segs, int margin, int* __restrict__ colexp,
+                                                   unsigned len, int segs, int margin, int* __restrict__ colexp,
                                                    int* __restrict__ flag) {
     constexpr int V = vec_rows<FMT>();
     constexpr int EB = 16 / V;
     __shared__ float wmax[4];
     const char* col = static_cast<const char*>(a) + j * lda * EB;
-    const unsigned vps = static_cast<unsigned>(len / V);
+    const unsigned vps = len / V;
     const unsigned total = vps * static_cast<unsigned>(segs);
     float mx = 0.0f;
 #pragma unroll 4
@@ -365,8 +330,10 @@ __device__ __forceinline__ void cs_sample_exp_body(int64_t j, int64_t m, const v
 template <int FMT, bool EXACT>
 __global__ __launch_bounds__(256) void cs_sample_exp_kernel(int64_t m, const void* __restrict__ a,
                                                             const uint16_t* __restrict__ wr, int64_t lda,
-                                                            int64_t stride, int len, int segs, int margin,
-                                                            int* __restrict__ colexp, int* __restrict__ flag) {
+                                                            int64_t stride, unsigned len, int segs, int margin,
+                                                            int* __restrict__ colexp, int* __restrict__ flag,
+                                                            const int* __restrict__ gate) {
+    if (gated_off(gate)) return;
     cs_sample_exp_body<FMT, EXACT>(blockIdx.x, m, a, wr, lda, stride, len, segs, margin, colexp, flag);
 }
 
@@ -382,7 +349,8 @@ struct CsGroupDesc {
     int* flags;  // [0] a column max not finite, [1] a value beyond its bound
     double* y;
     int64_t m, n, lda, s, ldy, rows_per_split, stride;
-    int ncg, splits, shift, len, segs, margin;
+    int ncg, splits, shift, segs, margin;
+    unsigned len;
     int block0;  // first block within its apply launch
     int local;   // index within its apply launch's descriptors
     int owner0;  // block0 plus the launch's first entry in the owner table
@@ -533,40 +501,30 @@ __device__ __forceinline__ void cs_apply_fx_rows(
     for (int64_t t = threadIdx.x; t < s * ncols; t += kVecThreads) out[t] = yfx[t];
 }
 
-template <int FMT, bool EXACT, int CG, bool NTL>
-__device__ __forceinline__ void cs_apply_fx_body(
-    int split, int cg, int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr,
-    int64_t lda, int64_t s, const uint32_t* __restrict__ packed, int64_t rows_per_split,
-    const int* __restrict__ colexp, int shift, unsigned long long* __restrict__ partial, int* __restrict__ over) {
-    if (shift <= kMagicShift)
-        cs_apply_fx_rows<FMT, EXACT, CG, NTL, true>(split, cg, m, n, a, wr, lda, s, packed, rows_per_split, colexp,
-                                                    shift, partial, over);
-    else
-        cs_apply_fx_rows<FMT, EXACT, CG, NTL, false>(split, cg, m, n, a, wr, lda, s, packed, rows_per_split, colexp,
-                                                     shift, partial, over);
-}
-
-template <int FMT, bool EXACT, int CG, bool NTL>
+// One kernel for each kind of term.
+template <int FMT, bool EXACT, int CG, bool NTL, bool MAGIC>
 __global__ __launch_bounds__(kVecThreads) void cs_apply_fx_kernel(
     int64_t m, int64_t n, const void* __restrict__ a, const uint16_t* __restrict__ wr, int64_t lda,
     int64_t s, const uint32_t* __restrict__ packed, int64_t rows_per_split, int ncg,
     const int* __restrict__ colexp, int shift, unsigned long long* __restrict__ partial,
-    int* __restrict__ over) {
+    int* __restrict__ over, const int* __restrict__ gate) {
+    if (gated_off(gate)) return;
     const int split = blockIdx.x / ncg;
-    cs_apply_fx_body<FMT, EXACT, CG, NTL>(split, blockIdx.x - split * ncg, m, n, a, wr, lda, s, packed,
-                                          rows_per_split, colexp, shift, partial, over);
+    cs_apply_fx_rows<FMT, EXACT, CG, NTL, MAGIC>(split, blockIdx.x - split * ncg, m, n, a, wr, lda, s, packed,
+                                                 rows_per_split, colexp, shift, partial, over);
 }
 
 // The blocks of every problem in one launch: block b belongs to problem
-// owner[b] and is its block b - block0 (split-major over its column groups)
-template <int FMT, bool EXACT, int CG, bool NTL>
+// owner[b] and is its block b - block0 (split-major over its column groups).
+// MAGIC: every problem of the launch allows it.
+template <int FMT, bool EXACT, int CG, bool NTL, bool MAGIC>
 __global__ __launch_bounds__(kVecThreads) void cs_group_apply_kernel(const CsGroupDesc* __restrict__ d,
                                                                      const int* __restrict__ owner) {
     const CsGroupDesc& q = d[owner[blockIdx.x]];
     const int lb = static_cast<int>(blockIdx.x) - q.block0;
     const int split = lb / q.ncg;
-    cs_apply_fx_body<FMT, EXACT, CG, NTL>(split, lb - split * q.ncg, q.m, q.n, q.a, q.wr, q.lda, q.s, q.packed,
-                                          q.rows_per_split, q.colexp, q.shift, q.partial, q.flags + 1);
+    cs_apply_fx_rows<FMT, EXACT, CG, NTL, MAGIC>(split, lb - split * q.ncg, q.m, q.n, q.a, q.wr, q.lda, q.s, q.packed,
+                                                 q.rows_per_split, q.colexp, q.shift, q.partial, q.flags + 1);
 }
 
 // y = the splits' integer sums added as integers (exact: |sum| < m 2^shift
@@ -576,7 +534,9 @@ __global__ __launch_bounds__(kVecThreads) void cs_group_apply_kernel(const CsGro
 __global__ __launch_bounds__(256) void cs_finish_fx_kernel(int64_t s, int64_t n, int splits,
                                                            const unsigned long long* __restrict__ partial,
                                                            const int* __restrict__ colexp, int shift,
-                                                           double* __restrict__ y, int64_t ldy) {
+                                                           double* __restrict__ y, int64_t ldy,
+                                                           const int* __restrict__ gate) {
+    if (gated_off(gate)) return;
     const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     if (t >= s * n) return;
     const int64_t c = t / s;
@@ -650,15 +610,14 @@ int fx_shift(int64_t m) {
 size_t a256(size_t v) { return (v + 255) / 256 * 256; }
 
 struct CsLayout {
-    size_t idx, colmax, colexp, flag, partial, total;
+    size_t idx, colexp, flag, partial, total;
 };
 
 CsLayout cs_layout(int64_t m, int64_t n, int64_t s) {
     const CsPlan pf = cs_plan(m, n, s), px = cs_plan_fx(m, n, s);
     CsLayout L;
     L.idx = 0;
-    L.colmax = a256(static_cast<size_t>(std::max<int64_t>(m, 1)) * 4);
-    L.colexp = L.colmax + a256(static_cast<size_t>(std::max<int64_t>(n, 1)) * 4);
+    L.colexp = a256(static_cast<size_t>(std::max<int64_t>(m, 1)) * 4);
     L.flag = L.colexp + a256(static_cast<size_t>(std::max<int64_t>(n, 1)) * 4);
     L.partial = L.flag + 256;
     const size_t pb = std::max(static_cast<size_t>(pf.splits) * s * n * 4, static_cast<size_t>(px.splits) * s * n * 8);
@@ -668,19 +627,18 @@ CsLayout cs_layout(int64_t m, int64_t n, int64_t s) {
 
 size_t cs_scratch(int64_t m, int64_t n, int64_t s) { return cs_layout(m, n, s).total; }
 
-// Whether columns start on 16-byte boundaries.
-template <int FMT>
-bool aligned16(const void* a, const uint16_t* wr, int64_t lda, bool exact) {
-    constexpr int V = vec_rows<FMT>();
-    const bool lo = !(exact && (FMT == FMT_P16 || FMT == FMT_PBF)) ||
-                    (reinterpret_cast<uintptr_t>(wr) % 16 == 0);
-    return reinterpret_cast<uintptr_t>(a) % 16 == 0 && lda % V == 0 && lo;
+// Whether the columns of both planes that are read start on 16-byte boundaries.
+bool aligned16(int a_type, bool exact, const void* a, const uint16_t* wr, int64_t lda) {
+    const bool packed = a_type == TOMOS_FP32_16 || a_type == TOMOS_FP32_BF16;
+    const int64_t v = a_type == TOMOS_F64 ? 2 : a_type == TOMOS_F32 ? 4 : 8;
+    return reinterpret_cast<uintptr_t>(a) % 16 == 0 && lda % v == 0 &&
+           !(exact && packed && reinterpret_cast<uintptr_t>(wr) % 16 != 0);
 }
 
 template <int FMT, bool EXACT, int CG>
 void launch_apply(const CsPlan& p, int64_t m, int64_t n, const void* a, const uint16_t* wr,
                   int64_t lda, int64_t s, const uint32_t* packed, float* partial,
-                  hipStream_t st) {
+                  const int* gate, hipStream_t st) {
     const size_t lds = static_cast<size_t>(s) * CG * 4;
     const int64_t blocks = static_cast<int64_t>(p.splits) * p.ncg;
     require(blocks < (int64_t(1) << 31), "countsketch_apply: grid too large");
@@ -689,28 +647,29 @@ void launch_apply(const CsPlan& p, int64_t m, int64_t n, const void* a, const ui
                                         hipFuncAttributeMaxDynamicSharedMemorySize,
                                         static_cast<int>(lds)));
     k<<<dim3(static_cast<unsigned>(blocks)), kVecThreads, lds, st>>>(
-        m, n, a, wr, lda, s, packed, p.rows_per_split, p.ncg, partial);
+        m, n, a, wr, lda, s, packed, p.rows_per_split, p.ncg, partial, gate);
     TOMOS_LAUNCH_CHECK("cs_apply_vec_kernel");
 }
 
 template <int FMT, bool EXACT>
 void launch_apply_cg(const CsPlan& p, int64_t m, int64_t n, const void* a, const uint16_t* wr,
                      int64_t lda, int64_t s, const uint32_t* packed, float* partial,
-                     hipStream_t st) {
+                     const int* gate, hipStream_t st) {
     switch (p.cg) {
-        case 8: launch_apply<FMT, EXACT, 8>(p, m, n, a, wr, lda, s, packed, partial, st); break;
-        case 4: launch_apply<FMT, EXACT, 4>(p, m, n, a, wr, lda, s, packed, partial, st); break;
-        case 2: launch_apply<FMT, EXACT, 2>(p, m, n, a, wr, lda, s, packed, partial, st); break;
-        default: launch_apply<FMT, EXACT, 1>(p, m, n, a, wr, lda, s, packed, partial, st); break;
+        case 8: launch_apply<FMT, EXACT, 8>(p, m, n, a, wr, lda, s, packed, partial, gate, st); break;
+        case 4: launch_apply<FMT, EXACT, 4>(p, m, n, a, wr, lda, s, packed, partial, gate, st); break;
+        case 2: launch_apply<FMT, EXACT, 2>(p, m, n, a, wr, lda, s, packed, partial, gate, st); break;
+        default: launch_apply<FMT, EXACT, 1>(p, m, n, a, wr, lda, s, packed, partial, gate, st); break;
     }
 }
 
-// Fixed-point apply on the vector path.  The column exponents come from a
-// sample of the rows (kSampleSegs segments spread over A, each 1/256 of
-// the rows long, 64..1024 rows) plus kSampleMargin bits when A has at least
-// kSampleMinRows rows, else from every row.  The apply kernel checks every
-// value against its column's bound; a value beyond it (or not finite)
-// makes the call redo the exponents from every row and apply again.
+// Fixed-point apply.  The column exponents come from a sample of the rows
+// (kSampleSegs segments spread over A, each 1/256 of the rows long, 64..1024
+// rows) plus kSampleMargin bits when A has at least kSampleMinRows rows, else
+// from every row.  The apply kernel checks every value against its column's
+// bound; a value beyond it (or not finite) makes the call redo the exponents
+// from every row and apply again, and a column that is not finite takes the
+// float path for the call.
 constexpr int64_t kSampleSegs = 32;
 constexpr int64_t kSampleMinRows = 16384;  // the sample is at most 1/8 of the rows
 constexpr int kSampleMargin = 12;           // 2^-31 of the sampled max per term at 2e6 rows, 4 splits
@@ -718,16 +677,28 @@ constexpr int kSampleMargin = 12;           // 2^-31 of the sampled max per term
 // own 256 bytes; more take the float path.
 constexpr int64_t kFxMaxBuckets = (160 * 1024 - 256) / 8;
 
-// Enqueue the fixed-point path with the exponents from a sample (sample)
-// or from every row, reading nothing back: flags[0] is set if a column's
-// max is not finite, flags[1] if a value is beyond its column's bound.
-// The caller reads the flags once its work is enqueued.
+// The rows that set the exponents: segments `stride` apart of `len` rows
+// (a multiple of 8; inside A for m >= kSampleMinRows), or all rows.
+struct ExpRows {
+    int64_t stride;
+    unsigned len;
+    int segs, margin;
+};
+ExpRows exp_rows(int64_t m, bool sample) {
+    if (!sample) return {0, static_cast<unsigned>(ceil_div(m, 8) * 8), 1, 0};
+    const int64_t len = std::max<int64_t>(64, std::min<int64_t>(1024, (m / 256) / 8 * 8));
+    return {(m / kSampleSegs) / 8 * 8, static_cast<unsigned>(len), static_cast<int>(kSampleSegs), kSampleMargin};
+}
+
+// Enqueue the fixed-point path, reading nothing back: flags[0] is set if a
+// column's max is not finite, flags[1] if a value is beyond its column's
+// bound.  Gated launches do nothing unless the attempt whose flags `gate` are
+// has failed.
 template <int FMT, bool EXACT>
 void fx_enqueue(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, int64_t s,
-                const uint32_t* packed, char* scratch, const CsLayout& L, double* y, int64_t ldy, bool sample,
-                int* flags, bool clear_flags, hipStream_t st) {
+                const uint32_t* packed, char* scratch, const CsLayout& L, double* y, int64_t ldy, bool aligned,
+                bool sample, int* flags, const int* gate, hipStream_t st) {
     const CsPlan p = cs_plan_fx(m, n, s);
-    unsigned* colmax = reinterpret_cast<unsigned*>(scratch + L.colmax);
     int* colexp = reinterpret_cast<int*>(scratch + L.colexp);
     unsigned long long* partial = reinterpret_cast<unsigned long long*>(scratch + L.partial);
     require(n < (int64_t(1) << 31), "countsketch_apply: n too large");
@@ -736,31 +707,11 @@ void fx_enqueue(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t
     constexpr bool kExactMax = EXACT && FMT == FMT_P16;
     constexpr int64_t kElemBytes = (FMT == FMT_F64 ? 8 : FMT == FMT_F32 ? 4 : 2) * (EXACT && (FMT == FMT_P16 || FMT == FMT_PBF) ? 2 : 1);
     // a vector across two cache lines wants the line kept for its neighbour
-    const bool ntl = aligned16<FMT>(a, wr, lda, EXACT) && stream_loads(m * n * kElemBytes);
-    if (clear_flags) TOMOS_HIP_CHECK(hipMemsetAsync(flags, 0, 8, st));
-    if (sample) {
-        // segments start (m / 32) rounded down to 8 rows apart and are
-        // m / 256 rows (64..1024, a multiple of 8) long: inside A for m >= 16384
-        const int64_t stride = (m / kSampleSegs) / 8 * 8;
-        const int64_t len = std::max<int64_t>(64, std::min<int64_t>(1024, (m / 256) / 8 * 8));
-        require(m >= kSampleMinRows && (kSampleSegs - 1) * stride + len <= m, "countsketch_apply: bad sample");
-        cs_sample_exp_kernel<FMT, kExactMax><<<dim3(static_cast<unsigned>(n)), 256, 0, st>>>(
-            m, a, wr, lda, stride, static_cast<int>(len), static_cast<int>(kSampleSegs), kSampleMargin, colexp,
-            flags);
-        TOMOS_LAUNCH_CHECK("cs_sample_exp_kernel");
-    } else {
-        TOMOS_HIP_CHECK(hipMemsetAsync(colmax, 0, static_cast<size_t>(n) * 4, st));
-        const int64_t csplits = std::max<int64_t>(1, std::min<int64_t>(64, ceil_div(m, 256 * 8 * 64)));
-        const int64_t stride = ceil_div(ceil_div(m, csplits), 8) * 8;
-        const dim3 cgrid(static_cast<unsigned>(n), static_cast<unsigned>(ceil_div(m, stride)));
-        if (ntl)
-            cs_colmax_kernel<FMT, kExactMax, true><<<cgrid, 256, 0, st>>>(m, a, wr, lda, stride, stride, colmax);
-        else
-            cs_colmax_kernel<FMT, kExactMax, false><<<cgrid, 256, 0, st>>>(m, a, wr, lda, stride, stride, colmax);
-        cs_colexp_kernel<<<dim3(static_cast<unsigned>(ceil_div(n, 256))), 256, 0, st>>>(n, colmax, 0, colexp,
-                                                                                        flags);
-        TOMOS_LAUNCH_CHECK("cs_colmax_kernel");
-    }
+    const bool ntl = aligned && stream_loads(m * n * kElemBytes);
+    const ExpRows er = exp_rows(m, sample);
+    cs_sample_exp_kernel<FMT, kExactMax><<<dim3(static_cast<unsigned>(n)), 256, 0, st>>>(
+        m, a, wr, lda, er.stride, er.len, er.segs, er.margin, colexp, flags, gate);
+    TOMOS_LAUNCH_CHECK("cs_sample_exp_kernel");
     const int shift = fx_shift(m);
     const size_t lds = static_cast<size_t>(s) * p.cg * 8;
     const int64_t blocks = static_cast<int64_t>(p.splits) * p.ncg;
@@ -770,57 +721,43 @@ void fx_enqueue(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t
                                             hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
         k<<<dim3(static_cast<unsigned>(blocks)), kVecThreads, lds, st>>>(m, n, a, wr, lda, s, packed,
                                                                         p.rows_per_split, p.ncg, colexp, shift,
-                                                                        partial, flags + 1);
+                                                                        partial, flags + 1, gate);
     };
-    if (ntl) {
-        switch (p.cg) {
-            case 8: launch(cs_apply_fx_kernel<FMT, EXACT, 8, true>); break;
-            case 4: launch(cs_apply_fx_kernel<FMT, EXACT, 4, true>); break;
-            case 2: launch(cs_apply_fx_kernel<FMT, EXACT, 2, true>); break;
-            default: launch(cs_apply_fx_kernel<FMT, EXACT, 1, true>); break;
-        }
-    } else {
-        switch (p.cg) {
-            case 8: launch(cs_apply_fx_kernel<FMT, EXACT, 8, false>); break;
-            case 4: launch(cs_apply_fx_kernel<FMT, EXACT, 4, false>); break;
-            case 2: launch(cs_apply_fx_kernel<FMT, EXACT, 2, false>); break;
-            default: launch(cs_apply_fx_kernel<FMT, EXACT, 1, false>); break;
-        }
+    auto width = [&](auto cg) {
+        constexpr int kCg = decltype(cg)::value;
+        if (shift > kMagicShift) launch(cs_apply_fx_kernel<FMT, EXACT, kCg, false, false>);
+        else if (ntl) launch(cs_apply_fx_kernel<FMT, EXACT, kCg, true, true>);
+        else launch(cs_apply_fx_kernel<FMT, EXACT, kCg, false, true>);
+    };
+    switch (p.cg) {
+        case 8: width(std::integral_constant<int, 8>{}); break;
+        case 4: width(std::integral_constant<int, 4>{}); break;
+        case 2: width(std::integral_constant<int, 2>{}); break;
+        default: width(std::integral_constant<int, 1>{}); break;
     }
     TOMOS_LAUNCH_CHECK("cs_apply_fx_kernel");
     cs_finish_fx_kernel<<<dim3(static_cast<unsigned>(ceil_div(s * n, 256))), 256, 0, st>>>(s, n, p.splits, partial,
-                                                                                          colexp, shift, y, ldy);
+                                                                                          colexp, shift, y, ldy, gate);
     TOMOS_LAUNCH_CHECK("cs_finish_fx_kernel");
 }
 
-// The fixed-point path for one call; returns false (the float path runs)
-// when a column's max over every row is not finite.  Reading the flags waits
-// for the stream, which a stream under capture cannot: a call whose columns
-// are not 16-byte aligned takes the float path there, as it always has.
+// The fixed-point path for one call.  Returns the flags that gate the float
+// path behind it (nullptr: the float path runs whatever they hold).  Nothing
+// is read back: the second attempt and the float path are enqueued as well
+// and exit at once when the first attempt held, about 2 us a launch, where
+// waiting for its flags cost 20 and the stream's overlap with the host
+// (1001 x 10: 72 us, now 26, two of its six launches empty; 60001 x 300 67 and 50).
 template <int FMT, bool EXACT>
-bool try_apply_fx(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, int64_t s,
-                  const uint32_t* packed, char* scratch, const CsLayout& L, double* y, int64_t ldy,
-                  hipStream_t st) {
-    if (s > kFxMaxBuckets) return false;
-    if (!aligned16<FMT>(a, wr, lda, EXACT)) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        TOMOS_HIP_CHECK(hipStreamIsCapturing(st, &cap));
-        if (cap != hipStreamCaptureStatusNone) return false;
-    }
-    int* flags = reinterpret_cast<int*>(scratch + L.flag);
-    int h[2] = {0, 0};
-    auto read_flags = [&]() {
-        TOMOS_HIP_CHECK(hipMemcpyAsync(h, flags, 8, hipMemcpyDeviceToHost, st));
-        TOMOS_HIP_CHECK(hipStreamSynchronize(st));
-    };
-    if (m >= kSampleMinRows) {  // sampled exponents: one pass over A when they hold
-        fx_enqueue<FMT, EXACT>(m, n, a, wr, lda, s, packed, scratch, L, y, ldy, true, flags, true, st);
-        read_flags();
-        if (!h[0] && !h[1]) return true;
-    }
-    fx_enqueue<FMT, EXACT>(m, n, a, wr, lda, s, packed, scratch, L, y, ldy, false, flags, true, st);
-    read_flags();
-    return !h[0] && !h[1];  // the float path redoes a call whose full-row exponents are not finite
+const int* apply_fx(int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda, int64_t s,
+                    const uint32_t* packed, char* scratch, const CsLayout& L, double* y, int64_t ldy, bool aligned,
+                    hipStream_t st) {
+    if (s > kFxMaxBuckets) return nullptr;
+    int* flags = reinterpret_cast<int*>(scratch + L.flag);  // cleared by cs_index_kernel
+    const bool sample = m >= kSampleMinRows;  // one pass over A when the sampled exponents hold
+    fx_enqueue<FMT, EXACT>(m, n, a, wr, lda, s, packed, scratch, L, y, ldy, aligned, sample, flags, nullptr, st);
+    if (!sample) return flags;
+    fx_enqueue<FMT, EXACT>(m, n, a, wr, lda, s, packed, scratch, L, y, ldy, aligned, false, flags + 2, flags, st);
+    return flags + 2;
 }
 
 }  // namespace
@@ -839,56 +776,47 @@ void countsketch_apply(int a_type, int tier, int64_t m, int64_t n, const void* a
     if (n == 0) return;
     require(y != nullptr, "countsketch_apply: null y");
     const size_t need = cs_scratch(m, n, s);
-    if (scratch == nullptr) scratch = fallback_scratch(need);
+    const bool shared = scratch == nullptr;
+    if (shared) scratch = fallback_scratch(need);
     else require(scratch_bytes >= need, "countsketch_apply: scratch too small");
     const CsPlan p = cs_plan(m, n, s);
     const CsLayout L = cs_layout(m, n, s);
     char* sc = static_cast<char*>(scratch);
     uint32_t* packed = reinterpret_cast<uint32_t*>(sc + L.idx);
     float* partial = reinterpret_cast<float*>(sc + L.partial);
+    const int* gate = nullptr;
+    const bool exact = tier == TOMOS_TIER_EXACT, aligned = aligned16(a_type, exact, a, wr, lda);
     if (m > 0) {
         require(a != nullptr, "countsketch_apply: null A");
         cs_index_kernel<<<dim3(static_cast<unsigned>(ceil_div(m, 256))), 256, 0, st>>>(
-            m, s, nullptr, nullptr, packed);
+            m, s, nullptr, nullptr, packed, reinterpret_cast<int*>(sc + L.flag));
         TOMOS_LAUNCH_CHECK("cs_index_kernel");
-        const bool exact = tier == TOMOS_TIER_EXACT;
         if (exact && (a_type == TOMOS_FP32_16 || a_type == TOMOS_FP32_BF16))
             require(wr != nullptr, "countsketch_apply: EXACT needs wr");
-        bool done = false;
+        auto run = [&](auto fmt, auto ex) {
+            constexpr int kFmt = decltype(fmt)::value;
+            constexpr bool kEx = decltype(ex)::value;
+            gate = apply_fx<kFmt, kEx>(m, n, a, wr, lda, s, packed, sc, L, y, ldy, aligned, st);
+            launch_apply_cg<kFmt, kEx>(p, m, n, a, wr, lda, s, packed, partial, gate, st);
+        };
+        auto tier_of = [&](auto fmt) {
+            if (exact) run(fmt, std::true_type{});
+            else run(fmt, std::false_type{});
+        };
         switch (a_type) {
-            case TOMOS_F32: done = try_apply_fx<FMT_F32, false>(m, n, a, wr, lda, s, packed, sc, L, y, ldy, st); break;
-            case TOMOS_F64: done = try_apply_fx<FMT_F64, false>(m, n, a, wr, lda, s, packed, sc, L, y, ldy, st); break;
-            case TOMOS_FP32_16:
-                done = exact ? try_apply_fx<FMT_P16, true>(m, n, a, wr, lda, s, packed, sc, L, y, ldy, st)
-                             : try_apply_fx<FMT_P16, false>(m, n, a, wr, lda, s, packed, sc, L, y, ldy, st);
-                break;
-            case TOMOS_FP32_BF16:
-                done = exact ? try_apply_fx<FMT_PBF, true>(m, n, a, wr, lda, s, packed, sc, L, y, ldy, st)
-                             : try_apply_fx<FMT_PBF, false>(m, n, a, wr, lda, s, packed, sc, L, y, ldy, st);
-                break;
-            default: break;
-        }
-        if (done) return;
-        switch (a_type) {
-            case TOMOS_F32: launch_apply_cg<FMT_F32, false>(p, m, n, a, wr, lda, s, packed, partial, st); break;
-            case TOMOS_F64: launch_apply_cg<FMT_F64, false>(p, m, n, a, wr, lda, s, packed, partial, st); break;
-            case TOMOS_FP32_16:
-                require(!exact || wr, "countsketch_apply: EXACT needs wr");
-                if (exact) launch_apply_cg<FMT_P16, true>(p, m, n, a, wr, lda, s, packed, partial, st);
-                else launch_apply_cg<FMT_P16, false>(p, m, n, a, wr, lda, s, packed, partial, st);
-                break;
-            case TOMOS_FP32_BF16:
-                require(!exact || wr, "countsketch_apply: EXACT needs wr");
-                if (exact) launch_apply_cg<FMT_PBF, true>(p, m, n, a, wr, lda, s, packed, partial, st);
-                else launch_apply_cg<FMT_PBF, false>(p, m, n, a, wr, lda, s, packed, partial, st);
-                break;
+            case TOMOS_F32: run(std::integral_constant<int, FMT_F32>{}, std::false_type{}); break;
+            case TOMOS_F64: run(std::integral_constant<int, FMT_F64>{}, std::false_type{}); break;
+            case TOMOS_FP32_16: tier_of(std::integral_constant<int, FMT_P16>{}); break;
+            case TOMOS_FP32_BF16: tier_of(std::integral_constant<int, FMT_PBF>{}); break;
             default: throw Error(kErrUnsupported, "countsketch_apply: unsupported a_type");
         }
     }
     const int64_t total = s * n;
     cs_finish_kernel<<<dim3(static_cast<unsigned>(ceil_div(total, 256))), 256, 0, st>>>(
-        s, n, m > 0 ? p.splits : 0, partial, y, ldy);
+        s, n, m > 0 ? p.splits : 0, partial, y, ldy, gate);
     TOMOS_LAUNCH_CHECK("cs_finish_kernel");
+    // such calls have always ended with the library's buffer free for other streams
+    if (shared && aligned && m > 0) TOMOS_HIP_CHECK(hipStreamSynchronize(st));
 }
 
 // Many sketches in one call.  Every problem that the fixed-point path takes
@@ -996,15 +924,19 @@ void group_launch(const std::vector<CsGroupDesc>& hd, const int* cg_first,
                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
             k<<<dim3(blocks), kVecThreads, lds, st>>>(d0, o0);
         };
-        switch (widths[w] * 2 + (ntl ? 1 : 0)) {
-            case 17: launch(cs_group_apply_kernel<FMT, EXACT, 8, true>); break;
-            case 16: launch(cs_group_apply_kernel<FMT, EXACT, 8, false>); break;
-            case 9: launch(cs_group_apply_kernel<FMT, EXACT, 4, true>); break;
-            case 8: launch(cs_group_apply_kernel<FMT, EXACT, 4, false>); break;
-            case 5: launch(cs_group_apply_kernel<FMT, EXACT, 2, true>); break;
-            case 4: launch(cs_group_apply_kernel<FMT, EXACT, 2, false>); break;
-            case 3: launch(cs_group_apply_kernel<FMT, EXACT, 1, true>); break;
-            default: launch(cs_group_apply_kernel<FMT, EXACT, 1, false>); break;
+        bool magic = true;
+        for (int k = cg_first[w]; k < cg_first[w] + cg_count[w]; ++k) magic = magic && hd[k].shift <= kMagicShift;
+        auto width = [&](auto cg) {
+            constexpr int kCg = decltype(cg)::value;
+            if (!magic) launch(cs_group_apply_kernel<FMT, EXACT, kCg, false, false>);
+            else if (ntl) launch(cs_group_apply_kernel<FMT, EXACT, kCg, true, true>);
+            else launch(cs_group_apply_kernel<FMT, EXACT, kCg, false, true>);
+        };
+        switch (widths[w]) {
+            case 8: width(std::integral_constant<int, 8>{}); break;
+            case 4: width(std::integral_constant<int, 4>{}); break;
+            case 2: width(std::integral_constant<int, 2>{}); break;
+            default: width(std::integral_constant<int, 1>{}); break;
         }
         TOMOS_LAUNCH_CHECK("cs_group_apply_kernel");
     }
@@ -1079,17 +1011,11 @@ void countsketch_apply_batched(int a_type, int tier, int nprob, const tomos_cs_p
             d.splits = static_cast<int>(ceil_div(q.m, d.rows_per_split));
             d.ncg = static_cast<int>(ceil_div(q.n, widths[w]));
             d.shift = fx_shift(q.m);
-            if (q.m >= kSampleMinRows) {
-                d.stride = (q.m / kSampleSegs) / 8 * 8;
-                d.len = static_cast<int>(std::max<int64_t>(64, std::min<int64_t>(1024, (q.m / 256) / 8 * 8)));
-                d.segs = static_cast<int>(kSampleSegs);
-                d.margin = kSampleMargin;
-            } else {  // every row: one segment
-                d.stride = 0;
-                d.len = static_cast<int>(ceil_div(q.m, 8) * 8);
-                d.segs = 1;
-                d.margin = 0;
-            }
+            const ExpRows er = exp_rows(q.m, q.m >= kSampleMinRows);
+            d.stride = er.stride;
+            d.len = er.len;
+            d.segs = er.segs;
+            d.margin = er.margin;
             d.block0 = static_cast<int>(nblocks - blk_first[w]);
             d.local = static_cast<int>(hd.size()) - cg_first[w];
             d.owner0 = static_cast<int>(nblocks);
@@ -1111,10 +1037,7 @@ void countsketch_apply_batched(int a_type, int tier, int nprob, const tomos_cs_p
         CsGroupDesc* dd = reinterpret_cast<CsGroupDesc*>(sc + L.desc);
         int* downer = reinterpret_cast<int*>(sc + L.owner);
         bool al = true;  // vectors that straddle cache lines are left cacheable
-        const int64_t v = a_type == TOMOS_F64 ? 2 : a_type == TOMOS_F32 ? 4 : 8;
-        for (const CsGroupDesc& d : hd)
-            al = al && d.lda % v == 0 && reinterpret_cast<uintptr_t>(d.a) % 16 == 0 &&
-                 (!exact || reinterpret_cast<uintptr_t>(d.wr) % 16 == 0);
+        for (const CsGroupDesc& d : hd) al = al && aligned16(a_type, exact, d.a, d.wr, d.lda);
         const bool ntl = al && stream_loads(bytes);
         switch (a_type) {
             case TOMOS_F32:
@@ -1179,7 +1102,7 @@ int tomos_countsketch_indices(int64_t m, int64_t s, int32_t* bucket, int8_t* sig
         if (m == 0) return;
         require(bucket || sign, "tomos_countsketch_indices: no output");
         cs_index_kernel<<<dim3(static_cast<unsigned>(ceil_div(m, 256))), 256, 0, st>>>(
-            m, s, bucket, sign, nullptr);
+            m, s, bucket, sign, nullptr, nullptr);
         TOMOS_LAUNCH_CHECK("cs_index_kernel");
     });
 }
