@@ -177,3 +177,21 @@ def test_tile_and_split_edges(capi, orc, a_type, variant, dec_hi, dec_ex, ta, tb
         got = gemm(a_type, tier, ta, tb, 2.0, M, N, K, wh, wr, A.shape[0], B, B.shape[0], -3.0, C0, M + 1)
         assert np.array_equal(got[:M], ref.astype(np.float32)), np.abs(got[:M] - ref).max()
         assert np.array_equal(got[M:], C0[M:])
+
+
+@pytest.mark.parametrize("shape", [(100, 90, 64), (100, 90, 1040)])  # one K split and four
+@pytest.mark.parametrize("exp", [-149, -135, -120, 100])
+def test_split_scale_of_any_operand(capi, shape, exp):
+    """The fp16 split stages FP32 B by a power of two of its largest magnitude
+    and undoes the same one, also where B is subnormal or large.  Integers up
+    to 15 times 2^exp: every product and sum is exact."""
+    M, N, K = shape
+    rng = np.random.default_rng(K)
+    A = np.asfortranarray(rng.integers(-15, 16, (M, K)).astype(np.float32))
+    Bi = np.asfortranarray(rng.integers(-15, 16, (K, N)).astype(np.float32))
+    B = np.ldexp(Bi, exp).astype(np.float32)
+    wh, wr = H.pack(C.PACK_FP32_16, A)
+    print("scale", shape, exp, flush=True)
+    got = gemm(C.FP32_16, C.TIER_MATERIALIZE, 0, 0, 2.0 ** -exp, M, N, K, wh, wr, M, B, K, 0.0,
+               np.zeros((M, N), np.float32, order="F"), M)
+    assert np.array_equal(got, (A.astype(np.float64) @ Bi).astype(np.float32))

@@ -87,6 +87,12 @@ __device__ __forceinline__ int fp16_scale_exp(bool f16, const unsigned* absmax_b
     return 13 - e;
 }
 
+// alpha times 2^-(sA + sB): what the staged scales of both operands leave to
+// undo (absA == nullptr: none).
+__device__ __forceinline__ double unscaled_alpha(double alpha, const unsigned* absA, const unsigned* absB) {
+    return absA ? ldexp(alpha, -(fp16_scale_exp(true, absA) + fp16_scale_exp(true, absB))) : alpha;
+}
+
 __device__ __forceinline__ void split16(bool f16, float v, int sc, uint16_t& h16, uint16_t& l16) {
     if (f16) {
         const float x = ldexpf(v, sc);
@@ -443,13 +449,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mfma_kernel(
     }
     // epilogue: acc[j][i][v] is C(row, col) with row = m tile i, lane % 32 and
     // col = n tile j, 8 (v / 4) + 4 (lane / 32) + v % 4
-    double scale = alpha;
-    if (F16 && absA) {  // fp16 split planes carry the scale 2^(13 - e) per operand
-        int ea = 0, eb = 0;
-        frexpf(fmaxf(__uint_as_float(*absA), 1e-38f), &ea);
-        frexpf(fmaxf(__uint_as_float(*absB), 1e-38f), &eb);
-        scale = ldexp(alpha, -((13 - ea) + (13 - eb)));
-    }
+    const double scale = F16 ? unscaled_alpha(alpha, absA, absB) : alpha;
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const int64_t r = m0 + am + i * 32 + row;
@@ -479,13 +479,7 @@ __global__ __launch_bounds__(256) void gemm_split_sum_kernel(int64_t M, int64_t 
                                                              double beta, float* __restrict__ C, int64_t ldc,
                                                              const unsigned* __restrict__ absA,
                                                              const unsigned* __restrict__ absB) {
-    double scale = alpha;
-    if (absA) {
-        int ea = 0, eb = 0;
-        frexpf(fmaxf(__uint_as_float(*absA), 1e-38f), &ea);
-        frexpf(fmaxf(__uint_as_float(*absB), 1e-38f), &eb);
-        scale = ldexp(alpha, -((13 - ea) + (13 - eb)));
-    }
+    const double scale = unscaled_alpha(alpha, absA, absB);
     const int64_t total = M * N;
     for (int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; t < total;
          t += static_cast<int64_t>(gridDim.x) * 256) {
