@@ -33,7 +33,6 @@
 // not bit for bit.  No reference counterpart: the reference has no adjoint.
 #include <algorithm>
 #include <cmath>
-#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -42,6 +41,7 @@
 #include "codec.hpp"
 #include "common.hpp"
 #include "gemv.hpp"
+#include "graphs.hpp"
 #include "lsqr_fused.hpp"
 #include "partials.hpp"
 #include "tomos_hip.h"
@@ -911,33 +911,11 @@ struct SegKey {
     }
 };
 
-struct SegCache {
-    struct Entry {
-        SegKey key;
-        hipGraphExec_t exec;
-    };
-    std::mutex mu;
-    std::vector<Entry> v;
-    static constexpr int kMax = 8;
-    hipGraphExec_t find(const SegKey& k) {
-        std::lock_guard<std::mutex> lock(mu);
-        for (const Entry& e : v)
-            if (e.key == k) return e.exec;
-        return nullptr;
-    }
-    // Every call synchronizes before it returns, so an evicted graph is idle.
-    void insert(const SegKey& k, hipGraphExec_t exec) {
-        std::lock_guard<std::mutex> lock(mu);
-        if (static_cast<int>(v.size()) >= kMax) {
-            (void)hipGraphExecDestroy(v.front().exec);
-            v.erase(v.begin());
-        }
-        v.push_back(Entry{k, exec});
-    }
-};
-SegCache& seg_cache() {
-    static SegCache c;
-    return c;
+// Kept segment graphs, two a call; never destroyed: at exit the HIP runtime
+// may be gone before them.
+SharedCache<SegKey, GraphExec>& seg_cache() {
+    static auto* c = new SharedCache<SegKey, GraphExec>(8);
+    return *c;
 }
 
 struct Grouped {
@@ -1114,27 +1092,11 @@ struct Grouped {
         }
         return k;
     }
-    hipGraphExec_t graph(int kind) {
-        const SegKey k = key(kind);
-        hipGraphExec_t exec = seg_cache().find(k);
-        if (exec) return exec;
-        hipGraph_t gr = nullptr;
-        TOMOS_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-        try {
+    SharedGraph graph(int kind) {
+        return cached_graph(seg_cache(), key(kind), s, [&] {
             if (kind == 0) restart_seq();
             else iter_seq();
-        } catch (...) {
-            hipGraph_t g2 = nullptr;
-            (void)hipStreamEndCapture(s, &g2);
-            if (g2) (void)hipGraphDestroy(g2);
-            throw;
-        }
-        TOMOS_HIP_CHECK(hipStreamEndCapture(s, &gr));
-        const hipError_t e = hipGraphInstantiate(&exec, gr, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(gr);
-        TOMOS_HIP_CHECK(e);
-        seg_cache().insert(k, exec);
-        return exec;
+        });
     }
 
     void states_to_host(std::vector<GState>& h) {
@@ -1147,8 +1109,7 @@ struct Grouped {
         k_gadj_init<<<static_cast<unsigned>(ceil_div(nprob, 64)), 64, 0, s>>>(dprobs(), nprob);
         k_gadj_zero_w<<<static_cast<unsigned>(nprob), kTail, 0, s>>>(dprobs());
         TOMOS_LAUNCH_CHECK("adjoint (grouped) set-up");
-        hipGraphExec_t rexec = graph(0);
-        hipGraphExec_t iexec = graph(1);
+        const SharedGraph rexec = graph(0), iexec = graph(1);  // held until the rounds have synchronized
         std::vector<GState> h(static_cast<size_t>(nprob));
         // a restart cycle takes one restart launch and at most
         // ceil(max_iters / kSegIters) + 1 rounds: a bound on the rounds
@@ -1157,8 +1118,8 @@ struct Grouped {
         bool restart_pending = true;  // every problem starts with its first restart
         bool all_done = false;
         for (int64_t round = 0; round < max_rounds && !all_done; ++round) {
-            if (restart_pending) TOMOS_HIP_CHECK(hipGraphLaunch(rexec, s));
-            TOMOS_HIP_CHECK(hipGraphLaunch(iexec, s));
+            if (restart_pending) TOMOS_HIP_CHECK(hipGraphLaunch(rexec.get(), s));
+            TOMOS_HIP_CHECK(hipGraphLaunch(iexec.get(), s));
             states_to_host(h);
             all_done = true;
             restart_pending = false;

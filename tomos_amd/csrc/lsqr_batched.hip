@@ -28,14 +28,11 @@
 // tunable.
 #include <algorithm>
 #include <cmath>
-#include <memory>
-#include <mutex>
-#include <type_traits>
-#include <utility>
 #include <vector>
 
 #include "codec.hpp"
 #include "common.hpp"
+#include "graphs.hpp"
 #include "lsqr_fused.hpp"
 #include "partials.hpp"
 #include "tomos_hip.h"
@@ -664,29 +661,9 @@ struct Batched {
     }
 
     // The segment as a graph, instantiated once per key and kept
-    // (library-wide cache of the last few keys).
-    using SharedGraph = std::shared_ptr<std::remove_pointer_t<hipGraphExec_t>>;
+    // (library-wide cache of the last few keys, two a solve).
     SharedGraph segment_graph(bool first) {
-        const GraphKey k = key(first);
-        if (SharedGraph kept = graph_cache_find(k)) return kept;
-        hipGraphExec_t exec = nullptr;
-        hipGraph_t graph = nullptr;
-        TOMOS_HIP_CHECK(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-        try {
-            segment(first);
-        } catch (...) {
-            hipGraph_t g2 = nullptr;
-            (void)hipStreamEndCapture(s, &g2);
-            if (g2) (void)hipGraphDestroy(g2);
-            throw;
-        }
-        TOMOS_HIP_CHECK(hipStreamEndCapture(s, &graph));
-        const hipError_t e = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        TOMOS_HIP_CHECK(e);
-        SharedGraph made(exec, [](hipGraphExec_t x) { (void)hipGraphExecDestroy(x); });
-        graph_cache_insert(k, made);
-        return made;
+        return cached_graph(graph_cache(), key(first), s, [&] { segment(first); });
     }
 
     // Restart by restart until every problem has stopped.  A solve whose
@@ -722,33 +699,10 @@ struct Batched {
         }
     }
 
-    // Library-wide cache of instantiated segment graphs (a few keys, oldest
-    // evicted; a solve that still runs an evicted graph holds its own share).
-    static constexpr int kGraphCache = 16;  // two a solve
-    struct CacheEntry {
-        GraphKey key;
-        SharedGraph exec;
-    };
-    static std::vector<CacheEntry>& cache() {
+    static SharedCache<GraphKey, GraphExec>& graph_cache() {
         // never destroyed: at exit the HIP runtime may be gone before it
-        static auto* c = new std::vector<CacheEntry>;
+        static auto* c = new SharedCache<GraphKey, GraphExec>(16);
         return *c;
-    }
-    static std::mutex& cache_mutex() {
-        static std::mutex m;
-        return m;
-    }
-    static SharedGraph graph_cache_find(const GraphKey& k) {
-        std::lock_guard<std::mutex> lock(cache_mutex());
-        for (const CacheEntry& e : cache())
-            if (e.key == k) return e.exec;
-        return nullptr;
-    }
-    static void graph_cache_insert(const GraphKey& k, SharedGraph exec) {
-        std::lock_guard<std::mutex> lock(cache_mutex());
-        auto& c = cache();
-        if (static_cast<int>(c.size()) >= kGraphCache) c.erase(c.begin());
-        c.push_back(CacheEntry{k, std::move(exec)});
     }
 };
 
