@@ -174,3 +174,23 @@ def test_default_shape_edges(capi, a_type, m, n, threads):
     finally:
         C.call("tomos_fused_config_clear")
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]) and got[2] == want[2]
+
+
+@pytest.mark.parametrize("a_type", [C.F32, C.FP32_BF16, C.FP32_16])
+def test_error_of_the_transposed_product(capi, orc, a_type):
+    """A^T u of the default shape: a tile's 64 rows are added in FP32, a block's
+    tiles in FP64, and the block's sum is rounded once.  A rounding is 2^-24 /
+    sqrt(3) rms of its sum at most.  Sums over k rows of a column have a mean
+    square of k |a|^2 u^2, so a row's share of the squared error is (in
+    2^-48 / 3): 4.5 from a lane's chain of 8 products, 1 from each of the 3
+    stages that add the row groups, 1 from the block's rounding, and the
+    error of the whole is 2^-24 sqrt(8.5 / 3) |a| |u|.  A sum over a block's
+    tiles in FP32 as well comes to 1.4 times that (FP32_BF16)."""
+    m, n = 200000, 300
+    rng = np.random.default_rng(2)
+    A = np.asfortranarray(rng.standard_normal((m, n), dtype=np.float32))
+    p, u0 = rng.standard_normal(n), rng.standard_normal(m).astype(np.float32)
+    u, t, _ = run_pair(a_type, A, m, p, u0, 0.5)
+    M = used_matrix(orc, a_type, A)
+    err = t - M.T @ u.astype(np.float64)
+    assert np.linalg.norm(err) <= 2.0 ** -24 * np.sqrt(8.5 / 3) * np.linalg.norm(M) / np.sqrt(m) * np.linalg.norm(u)

@@ -219,9 +219,13 @@ __device__ __forceinline__ void fused_body(int64_t m, int64_t n, const void* __r
                       : 0.0f;
     }
     constexpr int TOUT = ROUNDS / G;  // column partials owned by this lane
-    float tacc[TOUT];
+    // a tile's A^T u is FP32, the block's sum over its tiles FP64: with fewer,
+    // longer blocks (512 threads) the FP32 sum over a block's tiles lost to the
+    // 256-thread shape (200000 x 300 FP32_BF16, error of A^T u 5.4e-9 and
+    // 3.9e-9, now 3.3e-9)
+    double tacc[TOUT];
 #pragma unroll
-    for (int i = 0; i < TOUT; ++i) tacc[i] = 0.0f;
+    for (int i = 0; i < TOUT; ++i) tacc[i] = 0.0;
 
     // row partials and u rows in two copies, by tile parity: a wave may
     // write the next tile's partials while slower waves still read this
@@ -365,7 +369,7 @@ __device__ __forceinline__ void fused_body(int64_t m, int64_t n, const void* __r
         // reduce over the G row groups (lane bits 0..LOG_G-1); lane keeps TOUT columns
         LaneTRf<ROUNDS, G / 2, 1, true>::run(cs, lane);
 #pragma unroll
-        for (int i = 0; i < TOUT; ++i) tacc[i] += cs[i];
+        for (int i = 0; i < TOUT; ++i) tacc[i] += static_cast<double>(cs[i]);
         // no barrier here: the next tile writes the other copy, and this
         // copy is rewritten only after every wave has passed the next
         // tile's first barrier, that is, finished reading it
@@ -378,7 +382,7 @@ __device__ __forceinline__ void fused_body(int64_t m, int64_t n, const void* __r
 #pragma unroll
     for (int i = 0; i < TOUT; ++i) {
         const int64_t j = static_cast<int64_t>(base + i) * CS + c;
-        if (j < n) tpart_out[j] = tacc[i];
+        if (j < n) tpart_out[j] = static_cast<float>(tacc[i]);
     }
     // sum of squares of this block's u_raw rows
     for (int o = 32; o >= 1; o >>= 1) sq += __shfl_xor(sq, o);
@@ -942,11 +946,13 @@ FusedPlan lsqr_fused_plan(int a_type, int64_t m, int64_t n, int g, int blocks_pe
         threads = d.threads;
         // Between 256 and 512 columns twice the threads halve each wave's
         // rounds: faster except where the pass is bound by streaming bf16
-        // rows from HBM (more than the 256 MiB last-level cache holds).  us per pass, 256 / 512 threads: FP32_BF16
-        // 20000 x 400 22.5 / 18.2, 60000 x 300 30.6 / 24.7, 200000 x 512
-        // 53.3 / 50.3, but 700000 x 300 106 / 110.5 and 700000 x 512 130 /
-        // 137; FP32_16 60000 x 300 39.6 / 34.5, 700000 x 300 250 / 212.
-        // Up to 256 columns 256 threads (700000 x 130 60.6 / 96.4).
+        // rows from HBM (more than the 256 MiB last-level cache holds).  us per
+        // pass, 256 / 512 threads: FP32_BF16 20000 x 400 22.5 / 18.2, 60000 x
+        // 300 30.6 / 24.7, 200000 x 512 53.3 / 50.3, but 700000 x 300 106 /
+        // 110.5 and 700000 x 512 130 / 137; FP32_16 60000 x 300 39.6 / 34.5,
+        // 700000 x 300 250 / 212; F32 20000 x 300 23.3 / 21.9, 700000 x 300
+        // 154 / 151, 700000 x 512 245 / 243, 2000000 x 300 415 / 406.  Up to
+        // 256 columns 256 threads (700000 x 130 60.6 / 96.4).
         const bool bf16 = a_type == TOMOS_FP32_BF16 || a_type == TOMOS_BF16;
         if (n > 256 && n <= 512 && !(bf16 && bytes > (int64_t{256} << 20))) threads = 512;
     }
