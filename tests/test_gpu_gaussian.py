@@ -3,8 +3,8 @@ seeded counter layout, plus the reference's contract itself: i.i.d. N(0,1)
 entries (create_gaussian_sketch(Dense&), sketch.hpp:11-13,
 gaussian_sketch_registries.cpp:16-30) in FP64, FP32, FP16 and BF16.
 
-Tolerance: the kernel runs Box-Muller in FP32 (logf, sqrtf, sincospif),
-the oracle in FP64 with libm: |gpu - oracle| <= 1e-6 (1 + |x|) for
+Tolerance: the kernel runs Box-Muller in FP32 (hardware logarithm and
+reciprocal square root, polynomials for sine and cosine), the oracle in FP64 with libm: |gpu - oracle| <= 1e-6 (1 + |x|) for
 FP32/FP64 output, a few FP32 rounding errors; the 16-bit types are within
 one unit in the last place of the rounded oracle value (RNE of a value that
 differs by ~1e-7 can land on the neighbouring 16-bit number)."""

@@ -539,7 +539,7 @@ struct Solver {
         if (use_fused_restart) {
             float* tpart = reinterpret_cast<float*>(sc + L.tpart);
             lsqr_restart_launch(o.a_type, m, n, a, wr, lda, static_cast<const double*>(x), x_zero, U(), v64,
-                                red(), tpart, nullptr, rplan, &S->done, s);
+                                red(), tpart, rplan, &S->done, s);
             beta_temp(rplan.nblocks);
             tail(true, true);
             return;

@@ -974,8 +974,6 @@ FusedPlan lsqr_fused_plan(int a_type, int64_t m, int64_t n, int g, int blocks_pe
     p.tiles_per_block = std::max<int64_t>(1, ceil_div(ntiles, want));
     p.nblocks = static_cast<int>(ceil_div(ntiles, p.tiles_per_block));
     p.splits = std::min(kMaxSplits, std::max(1, p.nblocks / 16));
-    p.tpart_bytes = static_cast<size_t>(p.nblocks) * n * 4;
-    p.tsum_bytes = static_cast<size_t>(p.splits) * n * 8;
     return p;
 }
 
@@ -1083,15 +1081,12 @@ FusedPlan lsqr_restart_plan(int a_type, int64_t m, int64_t n) {
                                            lsqr_fused_max_blocks(m));
     p.tiles_per_block = std::max<int64_t>(1, ceil_div(ntiles, want));
     p.nblocks = static_cast<int>(ceil_div(ntiles, p.tiles_per_block));
-    p.splits = std::min(kMaxSplits, std::max(1, p.nblocks / 16));
-    p.tpart_bytes = static_cast<size_t>(p.nblocks) * n * 4;
-    p.tsum_bytes = static_cast<size_t>(p.splits) * n * 8;
     return p;
 }
 
 void lsqr_restart_launch(int a_type, int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda,
                          const double* x, bool xzero, void* u, bool u64, double* sumsq, float* tpart,
-                         double* tsum, const FusedPlan& plan, const int* skip, hipStream_t s) {
+                         const FusedPlan& plan, const int* skip, hipStream_t s) {
     require(n <= kRestartMaxN && plan.nblocks <= lsqr_fused_max_blocks(m), "lsqr_restart: plan does not fit");
     const void* k = restart_kernel_for(a_type, plan.stream, xzero);
     int64_t tpb = plan.tiles_per_block;
@@ -1099,10 +1094,6 @@ void lsqr_restart_launch(int a_type, int64_t m, int64_t n, const void* a, const 
                     &u, &u64, &tpb, &sumsq, &tpart, const_cast<int**>(&skip)};
     TOMOS_HIP_CHECK(hipLaunchKernel(k, dim3(static_cast<unsigned>(plan.nblocks)), dim3(kRsNT), args, 0, s));
     TOMOS_LAUNCH_CHECK("lsqr_restart_kernel");
-    if (!tsum) return;  // the caller adds the block partials itself
-    fused_tsum_kernel<<<dim3(static_cast<unsigned>(ceil_div(n, kThreads)), static_cast<unsigned>(plan.splits)),
-                        kThreads, 0, s>>>(n, plan.nblocks, plan.splits, tpart, tsum, skip);
-    TOMOS_LAUNCH_CHECK("fused_tsum_kernel");
 }
 
 }  // namespace tomos_hip

@@ -18,9 +18,7 @@ struct FusedPlan {
     int rounds = 0;  // column rounds per lane
     int nblocks = 0;
     int64_t tiles_per_block = 0;
-    int splits = 1;
-    size_t tpart_bytes = 0;  // [nblocks][n] float block partials of A^T u_raw
-    size_t tsum_bytes = 0;   // [splits][n] double level-1 sums
+    int splits = 1;          // of the blocks, in the sums of their partials (lsqr_fused_launch)
     bool stream = false;     // non-temporal loads of A (stream_loads of its bytes)
 };
 
@@ -34,7 +32,8 @@ bool lsqr_fused_supported(int a_type, int tier, int64_t m, int64_t n, int64_t ld
 FusedPlan lsqr_fused_plan(int a_type, int64_t m, int64_t n, int g = 0, int blocks_per_cu = 0,
                           int threads = 0);
 FusedShape lsqr_fused_default_shape(int64_t n);
-// upper bounds over every plan for (m, n): blocks and FusedPlan::tpart_bytes
+// upper bounds over every plan for (m, n): blocks, and the bytes of tpart
+// ([blocks][n] floats) and tsum ([splits][n] doubles)
 int64_t lsqr_fused_max_blocks(int64_t m);
 size_t lsqr_fused_max_tpart_bytes(int64_t m, int64_t n);
 size_t lsqr_fused_max_tsum_bytes(int64_t n);
@@ -55,7 +54,7 @@ void lsqr_fused_launch(int a_type, int64_t m, int64_t n, const void* a, int64_t 
 
 // ---- restart in one pass ------------------------------------------------
 // u_raw = u - A x at the exact tier (u holds b on entry, x FP64, FP64 row
-// sums), sumsq[b] per block and tsum = level-1 sums of A_hi^T u_raw, from
+// sums), sumsq[b] and tpart[b][j] per block as above (A_hi^T u_raw), from
 // one read of both planes.  xzero: x is known to be zero (the first restart
 // of a solve), so u_raw = u and only the hi plane is read.  Supported for
 // F32 and FP32_BF16 at the EXACT tier, n <= 1024, aligned as the
@@ -65,7 +64,7 @@ bool lsqr_restart_supported(int a_type, int tier, int64_t m, int64_t n, int64_t 
 FusedPlan lsqr_restart_plan(int a_type, int64_t m, int64_t n);
 void lsqr_restart_launch(int a_type, int64_t m, int64_t n, const void* a, const uint16_t* wr, int64_t lda,
                          const double* x, bool xzero, void* u, bool u64, double* sumsq, float* tpart,
-                         double* tsum, const FusedPlan& plan, const int* skip, hipStream_t s);
+                         const FusedPlan& plan, const int* skip, hipStream_t s);
 
 // ---- many problems in one launch ----------------------------------------
 // Device table entry of one problem: A (hi plane / F32), p (FP64, n),
