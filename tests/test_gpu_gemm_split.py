@@ -55,3 +55,26 @@ def test_split_gemm_alpha_beta(capi):
                     M, K, alpha=-0.5, beta=2.0, C0=C0)
     ref = -0.5 * (A.astype(np.float64) @ B.astype(np.float64)) + 2.0 * C0
     assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 3e-5
+
+
+@pytest.mark.parametrize("a_type,variant", [(C.FP32_BF16, C.PACK_FP32_BF16), (C.FP32_16, C.PACK_FP32_16)])
+@pytest.mark.parametrize("offset", [0, 1, 4, 8, 15])
+@pytest.mark.parametrize("shape", [(130, 100, 70), (130, 100, 600)])  # without and with K splits
+def test_split_gemm_scratch_alignment(capi, a_type, variant, offset, shape):
+    """Scratch of exactly the advertised size at any address: the staged planes
+    are moved to 16 bytes inside it, and nothing is written outside.  Integers
+    up to 15: every product and sum is exact."""
+    M, N, K = shape
+    rng = np.random.default_rng(K)
+    A = np.asfortranarray(rng.integers(-15, 16, (M, K)).astype(np.float32))
+    B = np.asfortranarray(rng.integers(-15, 16, (K, N)).astype(np.float32))
+    (aw, ar), (bw, br) = H.pack(variant, A), H.pack(variant, B)
+    size, guard = C.lib().tomos_gemm_split_scratch_size(M, N, K), 1024
+    sc = H.dev(np.full(guard + size + guard, 0xA5, np.uint8))
+    Cd = H.dev(np.zeros((M, N), np.float32))
+    print("scratch", a_type, offset, shape, flush=True)
+    C.call("tomos_gemm_split", a_type, M, N, K, 1.0, aw.ptr, ar.ptr, M, bw.ptr, br.ptr, K, 0.0, Cd.ptr, M,
+           sc.ptr + guard + offset, size, None)
+    assert np.array_equal(Cd.to_numpy(np.float32, (M, N)), (A.astype(np.float64) @ B).astype(np.float32))
+    raw = sc.to_numpy(np.uint8, (guard + size + guard,))
+    assert np.all(raw[:guard + offset] == 0xA5) and np.all(raw[guard + offset + size:] == 0xA5)

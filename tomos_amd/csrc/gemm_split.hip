@@ -508,9 +508,11 @@ Planes planes_of(int terms, int64_t M, int64_t N, int64_t K, void* base_ptr) {
     p.Np = ceil_div(N, kPadRows) * kPadRows;
     p.nk = std::max<int64_t>(ceil_div(K, slice_k(terms)), 1);
     p.Kp = p.nk * slice_k(terms);
-    char* base = static_cast<char*>(base_ptr);
-    p.absmax = reinterpret_cast<unsigned*>(base);
-    p.A = reinterpret_cast<uint16_t*>(base + 256);
+    // the planes start on 16 bytes, which their stores and the DMA take, at any
+    // alignment of the scratch: up to 15 of the 256 bytes ahead of them go
+    const uintptr_t base = reinterpret_cast<uintptr_t>(base_ptr);
+    p.absmax = reinterpret_cast<unsigned*>((base + 15) & ~uintptr_t(15));
+    p.A = reinterpret_cast<uint16_t*>((base + 256) & ~uintptr_t(15));
     p.B = p.A + p.Mp * p.nk * 2 * kBlockK;
     p.partial = reinterpret_cast<float*>(p.B + p.Np * p.nk * 2 * kBlockK);
     return p;
