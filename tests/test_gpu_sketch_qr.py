@@ -480,3 +480,24 @@ def test_sketch_is_asynchronous(capi, m, pad):
         with np.errstate(invalid="ignore"):
             np.add.at(ref, bucket, sign[:, None] * values[:, :m].t().double().cpu().numpy())
         assert np.array_equal(y.t().cpu().numpy(), ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("value", [3.0e7, float("inf")])
+def test_batched_sketch_leaves_library_scratch_free(capi, value):
+    """With NULL scratch a batch whose problems are redone one by one (an
+    outlier between the sampled rows, a column that is not finite) ends with
+    the library's buffer free: the stream has nothing left."""
+    torch = pytest.importorskip("torch")
+    m, n, s = 400000, 64, 512
+    a = torch.ones((n, m), device="cuda")
+    a[3, 5000] = value
+    y = torch.zeros((n, s), dtype=torch.float64, device="cuda")
+    table = (C.CsProblem * 1)(C.CsProblem(m, n, m, s, s, a.data_ptr(), None, y.data_ptr()))
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    for _ in range(2):  # the first call allocates the buffer
+        C.call("tomos_countsketch_apply_batched", C.F32, C.TIER_DEFAULT, 1, table, None, 0, side.cuda_stream)
+        idle = side.query()
+    torch.cuda.synchronize()
+    assert idle
+    assert float(y[3].abs().max()) > 2.0e7 and bool(torch.isfinite(y[4]).all())

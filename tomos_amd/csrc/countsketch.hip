@@ -969,7 +969,8 @@ void countsketch_apply_batched(int a_type, int tier, int nprob, const tomos_cs_p
     }
     if (nprob == 0) return;
     const size_t need = countsketch_batched_scratch_bytes(nprob, pr);
-    if (scratch == nullptr) scratch = fallback_scratch(need);
+    const bool shared = scratch == nullptr;
+    if (shared) scratch = fallback_scratch(need);
     else require(scratch_bytes >= need, "countsketch_apply_batched: scratch too small");
     char* sc = static_cast<char*>(scratch);
     const GroupLayout L = group_layout(nprob, pr);
@@ -1070,12 +1071,16 @@ void countsketch_apply_batched(int a_type, int tier, int nprob, const tomos_cs_p
     std::vector<int> h(2 * static_cast<size_t>(nprob), 0);
     TOMOS_HIP_CHECK(hipMemcpyAsync(h.data(), flags, h.size() * sizeof(int), hipMemcpyDeviceToHost, st));
     TOMOS_HIP_CHECK(hipStreamSynchronize(st));
+    bool alone = false;
     for (int i = 0; i < nprob; ++i) {
         const tomos_cs_problem& q = pr[i];
         if (q.n == 0) continue;
         if (grouped[static_cast<size_t>(i)] && !h[2 * i] && !h[2 * i + 1]) continue;
+        alone = true;
         countsketch_apply(a_type, tier, q.m, q.n, q.a, q.wr, q.lda, q.s, q.y, q.ldy, sc, need, st);
     }
+    // the library's buffer is free for other streams, as after the grouped problems
+    if (shared && alone) TOMOS_HIP_CHECK(hipStreamSynchronize(st));
 }
 
 }  // namespace tomos_hip
